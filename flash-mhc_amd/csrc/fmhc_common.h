@@ -25,6 +25,17 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
 
+// 16 (8) bytes at any address that is a multiple of 2: gfx950 moves unaligned
+// vectors in one instruction, so odd widths and operands off 16-byte
+// alignment take the same kernels as aligned ones (the code for an aligned
+// and an unaligned vector is the same global_load_dwordx4).
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned int u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ u32x4 ld16(const void* p) { return *static_cast<const u32x4_any*>(p); }
+__device__ __forceinline__ f32x4 ld16f(const void* p) { return *static_cast<const f32x4_any*>(p); }
+
 // Streaming loads/stores.  Data that is read or written exactly once per
 // launch carries the nontemporal hint so it does not evict the small,
 // reused operands (W, coefficients) from the caches.
@@ -50,6 +61,30 @@ __device__ __forceinline__ void st_stream(V* p, V v) {
   __builtin_nontemporal_store(v, p);
 #else
   *p = v;
+#endif
+}
+
+__device__ __forceinline__ u32x4 ld16_stream(const void* p) {
+#if FMHC_NT_LOADS
+  return __builtin_nontemporal_load(static_cast<const u32x4_any*>(p));
+#else
+  return ld16(p);
+#endif
+}
+
+__device__ __forceinline__ void st16_stream(void* p, u32x4 v) {
+#if FMHC_NT_STORES
+  __builtin_nontemporal_store(v, static_cast<u32x4_any*>(p));
+#else
+  *static_cast<u32x4_any*>(p) = v;
+#endif
+}
+
+__device__ __forceinline__ void st8_stream(void* p, u32x2 v) {
+#if FMHC_NT_STORES
+  __builtin_nontemporal_store(v, static_cast<u32x2_any*>(p));
+#else
+  *static_cast<u32x2_any*>(p) = v;
 #endif
 }
 

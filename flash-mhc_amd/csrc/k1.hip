@@ -5,8 +5,9 @@
 // few tokens, a column split whose partial sums k1_fwd_finish adds),
 // k1_bwd_mfma (dx; with DW also grad_W's per-run partials, which
 // k1_dw_reduce adds; with EPI / GI the pre-map backward's extra terms of
-// grad_x in the same store), and element-wise kernels for shapes off the
-// matrix-core path (nC % 8 != 0, unaligned pointers).
+// grad_x in the same store), and element-wise kernels for what these do not
+// take (forward: nC % 8 != 0, unaligned pointers; backward: fewer than 8
+// columns; rows beyond their 32-bit offsets).
 //
 //   forward   inv_rms[t] = rsqrt(sum_k x[t,k]^2 / nC + 1e-6)
 //             out[t,d]   = bf16(inv_rms[t] * sum_k x[t,k] * W[d,k])
@@ -539,8 +540,7 @@ __global__ __launch_bounds__(256) void k1_fwd_finish(const float* __restrict__ p
 }
 
 // ---------------------------------------------------------------------------
-// K1 backward dx, matrix-core path (nC % 8 == 0, 16-byte aligned x / W / go /
-// proj_out / inv_rms / grad_x).
+// K1 backward dx, matrix-core path (any nC from 8 on, any alignment).
 //
 // Each wave owns a 128-wide slice of the nC axis and walks one run of blocks
 // of 16 tokens (strided by the number of runs, see below; the host picks the
@@ -554,6 +554,25 @@ __global__ __launch_bounds__(256) void k1_fwd_finish(const float* __restrict__ p
 // instruction covers 4 token rows x 256 contiguous bytes (whole cache lines).
 // The B tiles depend only on the slice, so each wave builds them once: eight
 // 16-byte loads of W rows and an 8 x 8 bf16 transpose in registers.
+//
+// The slices cut either the whole row (one part of nC columns) or, for the
+// pre-map backward with C % 8 != 0, each stream's row (four parts of C
+// columns), so that a lane's eight columns never straddle two streams.
+// Bound by HBM like the aligned shapes, with 16-byte accesses that cross
+// lines.  Against the element-wise kernels these shapes took before (a wave
+// per token; grad_W one thread per element over all tokens): pre-map backward
+// at T = 20011, C = 300 5444 -> 81 us, T = 30011, C = 1001 13430 -> 271 us;
+// x 2 bytes off 16-byte alignment at T = 8192, C = 1024 2802 -> 83 us.
+// Loading the columns past the row's end without a mask (the compiler then
+// counts its waits exactly) is worth 6-14% where nC % 128 != 0: pre-map
+// backward at C = 520 (T = 20000) 118 -> 104 us, 1032 185 -> 161 us, 1000
+// (T = 65536) 528 -> 495 us.
+struct BwdSlices {
+  int len;  // columns of a part
+  int spp;  // 128-wide slices of a part
+  int n;    // slices of all parts
+};
+
 template <bool EPI, bool GI>
 struct BwdFrag {
   u32x4 gv, pv;   // go / proj_out row of token tbase + col, d = 8 * grp .. + 8
@@ -597,7 +616,7 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
                                                    const uint16_t* __restrict__ go3,
                                                    const float* __restrict__ h_pre,
                                                    const uint16_t* __restrict__ gi,
-                                                   int64_t T, int nC, int nslices, int64_t nruns, int C) {
+                                                   int64_t T, int nC, const BwdSlices sl, int64_t nruns, int C) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int col = lane & 15;  // A row (token) for the loads of go, B/D column
@@ -615,15 +634,22 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
   const unsigned full = gridDim.x & ~63u;
   const unsigned lid = bid < full ? (bid & ~63u) + 8u * (bid % 8u) + (bid % 64u) / 8u : bid;
   const int64_t wid = static_cast<int64_t>(lid) * 4 + wave;
-  const int slice = static_cast<int>(wid % nslices);
-  const int64_t run = wid / nslices;
+  const int slice = static_cast<int>(wid % sl.n);
+  const int64_t run = wid / sl.n;
   // Token blocks run, run + nruns, run + 2 * nruns, ...: the waves resident at
   // one time work on neighbouring blocks, so the concurrent reads and writes
   // cover contiguous memory instead of addresses a power-of-two apart.
   const int64_t nblocks = (T + 15) / 16;  // nruns <= nblocks
   if (run >= nruns) return;
-  const int kl = slice * 128 + 8 * col;  // this lane's 8 consecutive k
-  const bool kok = FULLK || kl < nC;     // nC % 8 == 0: all 8 valid or none
+  // This lane's 8 consecutive k.  Lanes that would pass the end of their part
+  // take its last 8 columns instead: every load stays in bounds without a
+  // mask, a lane that is only partly past the end (kok) stores its neighbour's
+  // last columns once more with the same values, and a lane wholly past it
+  // stores nothing.
+  const int part = FULLK ? 0 : slice / sl.spp;
+  const int c0 = (slice - part * sl.spp) * 128 + 8 * col;
+  const bool kok = FULLK || c0 < sl.len;
+  const int kl = FULLK ? slice * 128 + 8 * col : part * sl.len + (c0 < sl.len - 8 ? c0 : sl.len - 8);
   // Addresses are a wave-uniform block base plus a 32-bit per-lane byte offset
   // (16 rows of x span 32 * nC bytes < 2^32, checked by the caller).
   const uint32_t row_bytes = 2u * static_cast<uint32_t>(nC);
@@ -634,7 +660,8 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
   // VALU build: W[d][kl .. kl + 8) for d = 0..31 and the lane columns, and the token block's go rows.
   __shared__ u32x4 wvl[kValu ? 4 : 1][kValu ? 32 * 16 : 1];
   __shared__ u32x4 gvl[kValu ? 4 : 1][kValu ? 16 * 4 : 1];
-  // EPI: the lane's stream j and position c (C % 8 == 0: k .. k + 7 stay in one stream).
+  // EPI: the lane's stream j and position c (k .. k + 7 stay in one stream:
+  // C % 8 == 0, or the parts are the streams).
   const int sj = EPI ? kl / C : 0;
   const uint32_t c3bytes = EPI ? 2u * static_cast<uint32_t>(kl - sj * C) : 0u;
   f32x4 dacc[DW ? 8 : 1][2];
@@ -647,8 +674,7 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
     u32x4 rows[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      rows[e] = u32x4{0u, 0u, 0u, 0u};
-      if (kok) rows[e] = *reinterpret_cast<const u32x4*>(W + static_cast<int64_t>(8 * grp + e) * nC + kl);
+      rows[e] = ld16(W + static_cast<int64_t>(8 * grp + e) * nC + kl);
     }
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
@@ -688,14 +714,14 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
     const int last = block_rows(tbase) - 1;  // rows past the end re-read the last one
     const int rg = col < last ? col : last;
     const uint32_t goff = static_cast<uint32_t>(rg) * (2u * kDout) + 16u * static_cast<uint32_t>(grp);
-    f.gv = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(go + tbase * kDout) + goff);
-    f.pv = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(proj + tbase * kDout) + goff);
+    f.gv = ld16(reinterpret_cast<const char*>(go + tbase * kDout) + goff);
+    f.pv = ld16(reinterpret_cast<const char*>(proj + tbase * kDout) + goff);
     const char* ib = reinterpret_cast<const char*>(inv_rms + tbase);
     const char* xb = reinterpret_cast<const char*>(x + tbase * nC);
     // The lane's four tokens are consecutive: a full block reads their
     // inv_rms with one 16-byte load (the block-uniform branch below).
     if (last == 15) {
-      const f32x4 iv = *reinterpret_cast<const f32x4*>(ib + 16u * static_cast<uint32_t>(grp));
+      const f32x4 iv = ld16f(ib + 16u * static_cast<uint32_t>(grp));
 #pragma unroll
       for (int q = 0; q < 4; ++q) f.inv[q] = iv[q];
     }
@@ -704,26 +730,17 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
       const int r0 = 4 * grp + q;
       const uint32_t r = static_cast<uint32_t>(r0 < last ? r0 : last);
       if (last != 15) f.inv[q] = *reinterpret_cast<const float*>(ib + 4u * r);
-      f.xv[q] = u32x4{0u, 0u, 0u, 0u};
-      if (kok) f.xv[q] = ld_stream(reinterpret_cast<const u32x4*>(xb + (r * row_bytes + kbytes)));
+      f.xv[q] = ld16_stream(xb + (r * row_bytes + kbytes));
       if constexpr (EPI) {
-        f.hp[q] = 0.f;
-        f.g3[q] = u32x4{0u, 0u, 0u, 0u};
-        if (kok) {  // lanes past nC have no stream
-          const char* g3b = reinterpret_cast<const char*>(go3 + tbase * C);
-          f.hp[q] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(h_pre + tbase * 4) +
-                                                    16u * r + 4u * static_cast<uint32_t>(sj));
-          // Ordinary load: the four streams' slices read the same go3 row, and
-          // the nontemporal hint kept it out of L2 between them (1.14x FETCH).
-          f.g3[q] = *reinterpret_cast<const u32x4*>(g3b + (r * 2u * static_cast<uint32_t>(C) + c3bytes));
-        }
+        const char* g3b = reinterpret_cast<const char*>(go3 + tbase * C);
+        f.hp[q] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(h_pre + tbase * 4) + 16u * r +
+                                                  4u * static_cast<uint32_t>(sj));
+        // Ordinary load: the four streams' slices read the same go3 row, and
+        // the nontemporal hint kept it out of L2 between them (1.14x FETCH).
+        f.g3[q] = ld16(g3b + (r * 2u * static_cast<uint32_t>(C) + c3bytes));
       }
-      if constexpr (GI) {
-        f.gi[q] = u32x4{0u, 0u, 0u, 0u};
-        if (kok)
-          f.gi[q] = ld_stream(reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(gi + tbase * nC) +
-                                                             (r * row_bytes + kbytes)));
-      }
+      if constexpr (GI)
+        f.gi[q] = ld16_stream(reinterpret_cast<const char*>(gi + tbase * nC) + (r * row_bytes + kbytes));
     }
   };
   auto compute = [&](const BwdFrag<EPI, GI>& f, int tb) {
@@ -793,7 +810,7 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
               for (int m = 0; m < 8; ++m) o[m] = gif[m] + bf16_to_f32(f32_to_bf16(o[m]));
             }
           }
-          st_stream(reinterpret_cast<u32x4*>(gxb + (static_cast<uint32_t>(r) * row_bytes + kbytes)), pack8(o));
+          st16_stream(gxb + (static_cast<uint32_t>(r) * row_bytes + kbytes), pack8(o));
         }
       }
     }
@@ -879,7 +896,7 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
 
   if constexpr (DW) {
     // Partial layout [run][slice][m][h][r][lane]: one 256-byte row per store.
-    float* dst = dw_partial + (run * nslices + slice) * (8 * 2 * 4 * kWave);
+    float* dst = dw_partial + (run * sl.n + slice) * (8 * 2 * 4 * kWave);
 #pragma unroll
     for (int m = 0; m < 8; ++m)
 #pragma unroll
@@ -892,20 +909,20 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
 // Sums the per-run partials of k1_bwd_mfma<true, ...> in run order and
 // writes grad_W (32, nC) bf16.  Partial element
 // i = (((slice * 8 + m) * 2 + h) * 4 + r) * 64 + lane stands for
-// d = 16 h + (lane & 15), k = 128 slice + 8 (4 (lane >> 4) + r) + m; each
-// thread sums four consecutive elements (16-byte loads, four parts per trip).
+// d = 16 h + (lane & 15) and column m of the kernel's lane column
+// 4 (lane >> 4) + r of the slice; each thread sums four consecutive elements (16-byte loads, four parts per trip).
 // Workgroups from dw_blocks on sum K2's parameter gradients instead, one
 // workgroup per parameter (the pre-map backward; one launch fewer than K2's
 // own reduce).
 __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ partial,
                                                     uint16_t* __restrict__ dW, int64_t nparts,
-                                                    int nslices, int nC, unsigned dw_blocks,
+                                                    const BwdSlices sl, int nC, unsigned dw_blocks,
                                                     const K2ParamSums k2) {
   if (blockIdx.x >= dw_blocks) {  // one workgroup per K2 parameter
     k2_param_sum(k2, static_cast<int>(blockIdx.x - dw_blocks));
     return;
   }
-  const int64_t per_part = static_cast<int64_t>(nslices) * (8 * 2 * 4 * kWave);
+  const int64_t per_part = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave);
   const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (i0 >= per_part) return;
   const f32x4* src = reinterpret_cast<const f32x4*>(partial + i0);
@@ -926,8 +943,12 @@ __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ pa
   const int h = static_cast<int>((i0 / (4 * kWave)) % 2);
   const int m = static_cast<int>((i0 / (8 * kWave)) % 8);
   const int slice = static_cast<int>(i0 / (64 * kWave));
-  const int k = 128 * slice + 8 * (4 * (lane0 >> 4) + rr) + m;
-  if (k >= nC) return;
+  const int part = slice / sl.spp;
+  const int c0 = 128 * (slice - part * sl.spp) + 8 * (4 * (lane0 >> 4) + rr);
+  const int c = (c0 < sl.len - 8 ? c0 : sl.len - 8) + m;
+  // Past the part's end, or a column that the lane before holds as well.
+  if (c0 >= sl.len || c < c0) return;
+  const int k = part * sl.len + c;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int d = 16 * h + ((lane0 + e) & 15);
@@ -961,9 +982,9 @@ __global__ __launch_bounds__(256) void k1_dw_scalar(const uint16_t* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Element-wise paths for shapes or alignments the matrix-core paths do not
-// take (nC % 8 != 0, or a base pointer not 16-byte aligned).  One wave per
-// token; results agree with the matrix-core paths to fp32 summation order.
+// Element-wise paths for what the matrix-core paths do not take (forward:
+// nC % 8 != 0 or a base pointer not 16-byte aligned; backward: fewer than 8
+// columns; rows beyond 2^24 / 2^26 columns).  One wave per token; results agree with the matrix-core paths to fp32 summation order.
 __global__ __launch_bounds__(256) void k1_fwd_scalar(const uint16_t* __restrict__ x,
                                                      const uint16_t* __restrict__ W,
                                                      uint16_t* __restrict__ out,
@@ -1098,13 +1119,19 @@ bool bad_sizes(int64_t T, int64_t nC, int64_t D_out) {
   return T < 0 || nC <= 0 || nC > (int64_t{1} << 30) || D_out != kDout;
 }
 
-// The backward MFMA kernel addresses 16 rows of x with 32-bit byte offsets
-// and reads inv_rms four tokens at a time.
-bool k1_bwd_mfma_path(const void* x, const void* W, const void* go, const void* proj, const void* inv_rms,
-                      const void* gx, int64_t nC) {
-  return nC % 8 == 0 && nC <= (int64_t{1} << 26) && aligned16(x) && aligned16(W) && aligned16(go) &&
-         aligned16(proj) && aligned16(inv_rms) && aligned16(gx);
+// The backward MFMA kernel addresses 16 rows of x with 32-bit byte offsets,
+// and a lane holds 8 columns of one part (of `len` columns).
+bool k1_bwd_mfma_path(int64_t nC, int64_t len) { return len >= 8 && nC <= (int64_t{1} << 26); }
+
+// The row of nC columns cut in parts of `len` columns.
+BwdSlices bwd_slices(int64_t nC, int64_t len) {
+  const int spp = static_cast<int>((len + 127) / 128);
+  return BwdSlices{static_cast<int>(len), spp, static_cast<int>(nC / len) * spp};
 }
+
+// The pre-map backward's parts: the streams where a lane's 8 columns of the
+// whole row could belong to two of them.
+BwdSlices bwd_premap_slices(int64_t C) { return bwd_slices(4 * C, C % 8 == 0 ? 4 * C : C); }
 
 // Column split of the forward for T tokens (S = 1: the one-pass kernel).
 struct K1FwdSplit {
@@ -1197,17 +1224,16 @@ int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* 
 }
 
 // Number of runs of k1_bwd_mfma for T tokens (nblocks blocks of 16) and
-// nC / 128 slices: ceil(nblocks / max_blocks) runs, or, when those leave SIMDs
+// nslices slices: ceil(nblocks / max_blocks) runs, or, when those leave SIMDs
 // without a wave, more and shorter runs (down to min_blocks blocks) until
 // there is one wave per SIMD (kBwdFillWaves).  Measured with grad_W: T = 1024,
 // C = 1024 63 -> 14 us, T = 8192 70 -> 40 us; dx alone at T = 1024 16 -> 6 us.
 // Filling two waves per SIMD instead, or rounding large run counts to whole
 // rounds of resident waves, was slower at C = 4096; two waves per SIMD also
 // at C = 1024 (block step at T = 4096 / 6000: 170 -> 178 / 230 -> 236 us).
-int64_t k1_bwd_nruns(int64_t T, int64_t nC, int64_t max_blocks, int64_t min_blocks) {
+int64_t k1_bwd_nruns(int64_t T, int64_t nslices, int64_t max_blocks, int64_t min_blocks) {
   const int64_t nblocks = (T + 15) / 16;
   if (nblocks <= 0) return 1;
-  const int64_t nslices = (nC + 127) / 128;
   const int64_t fill = kBwdFillWaves / nslices > 1 ? kBwdFillWaves / nslices : 1;
   const int64_t nmin = (nblocks + max_blocks - 1) / max_blocks;
   int64_t n = nblocks / min_blocks;
@@ -1218,9 +1244,9 @@ int64_t k1_bwd_nruns(int64_t T, int64_t nC, int64_t max_blocks, int64_t min_bloc
 template <bool DW, bool EPI = false, bool GI = false>
 void launch_k1_bwd_mfma(hipStream_t s, const uint16_t* x, const uint16_t* W, const uint16_t* go,
                         const uint16_t* proj, const float* inv_rms, uint16_t* gx, float* partial, int64_t T, int nC,
-                        int nslices, int64_t nruns, const uint16_t* go3 = nullptr, const float* h_pre = nullptr,
-                        int C = 1, const uint16_t* gi = nullptr) {
-  const dim3 grid(blocks_for(nruns * nslices, 4));
+                        const BwdSlices& sl, int64_t nruns, const uint16_t* go3 = nullptr,
+                        const float* h_pre = nullptr, int C = 1, const uint16_t* gi = nullptr) {
+  const dim3 grid(blocks_for(nruns * sl.n, 4));
   constexpr int nbuf = EPI ? kBwdEpiBufs : kBwdBufs;
   // dx alone: one workgroup per CU (LDS reserved that the kernel does not
   // use; its registers allow two) up to C = 2560 per stream.  Measured in
@@ -1231,17 +1257,16 @@ void launch_k1_bwd_mfma(hipStream_t s, const uint16_t* x, const uint16_t* W, con
   // slower (T = 65536 and 262144).  With grad_W it changed nothing
   // (202.7-203.1 against 201.8-203.3 us at T = 65536, C = 1024).
   const bool cap = !DW && !EPI && FMHC_LDS_CAP && nC <= 4 * 2560;
-  if (nC % 128 == 0) {
+  if (sl.len % 128 == 0) {
     static const unsigned lds =
         lds_reserve(reinterpret_cast<const void*>(&k1_bwd_mfma<DW, true, EPI, GI, nbuf>), kLdsCapOne);
     k1_bwd_mfma<DW, true, EPI, GI, nbuf><<<grid, 256, cap ? lds : 0u, s>>>(x, W, go, proj, inv_rms, gx, partial,
-                                                                          go3, h_pre, gi, T, nC, nslices, nruns, C);
+                                                                          go3, h_pre, gi, T, nC, sl, nruns, C);
   } else {
     static const unsigned lds =
         lds_reserve(reinterpret_cast<const void*>(&k1_bwd_mfma<DW, false, EPI, GI, nbuf>), kLdsCapOne);
     k1_bwd_mfma<DW, false, EPI, GI, nbuf><<<grid, 256, cap ? lds : 0u, s>>>(x, W, go, proj, inv_rms, gx, partial,
-                                                                           go3, h_pre, gi, T, nC, nslices, nruns,
-                                                                           C);
+                                                                           go3, h_pre, gi, T, nC, sl, nruns, C);
   }
 }
 
@@ -1282,10 +1307,10 @@ extern "C" int fmhc_k1_bwd_dx(const uint16_t* x_flat, const uint16_t* W, const u
     return FMHC_ERR_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int nc = static_cast<int>(nC);
-  if (k1_bwd_mfma_path(x_flat, W, grad_out, proj_out, inv_rms, grad_x, nC)) {
-    const int nslices = static_cast<int>((nC + 127) / 128);
-    const int64_t nruns = k1_bwd_nruns(T, nC, kBwdNTB, 1);
-    launch_k1_bwd_mfma<false>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, nullptr, T, nc, nslices, nruns);
+  if (k1_bwd_mfma_path(nC, nC)) {
+    const BwdSlices sl = bwd_slices(nC, nC);
+    const int64_t nruns = k1_bwd_nruns(T, sl.n, kBwdNTB, 1);
+    launch_k1_bwd_mfma<false>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, nullptr, T, nc, sl, nruns);
   } else {
     const dim3 grid(blocks_for(T, 4));
     k1_bwd_scalar<false><<<grid, 256, 0, s>>>(x_flat, W, grad_out, proj_out, inv_rms, grad_x, nullptr, T, nc);
@@ -1301,23 +1326,26 @@ namespace {
 // pre-map backward's split kernel walks side by side (premap_split.hip), so
 // that each group takes the same number of runs; it shares these runs, and so
 // grad_W's partial sums, with this kernel.
-int64_t k1_bwd_runs(int64_t T, int64_t nC) {
-  const int64_t n = k1_bwd_nruns(T, nC, kBwdDwNTB, kBwdDwMinNTB);
-  const int64_t nslices = (nC + 127) / 128;
+int64_t k1_bwd_runs(int64_t T, int64_t nslices) {
+  const int64_t n = k1_bwd_nruns(T, nslices, kBwdDwNTB, kBwdDwMinNTB);
   const int64_t fill = kBwdFillWaves / nslices > 1 ? kBwdFillWaves / nslices : 1;
   const int64_t nblocks = (T + 15) / 16;
   if (n <= fill) return n;
   const int64_t r = (n + fill - 1) / fill * fill;
   return r < nblocks ? r : nblocks;
 }
+
+// Bytes of grad_W's partial sums.
+int64_t k1_bwd_dw_bytes(int64_t T, const BwdSlices& sl) {
+  return k1_bwd_runs(T, sl.n) * sl.n * (8 * 2 * 4 * kWave) * static_cast<int64_t>(sizeof(float));
+}
 }  // namespace
 }  // namespace fmhc
 
 extern "C" int64_t fmhc_k1_bwd_workspace_bytes(int64_t T, int64_t nC) {
   using namespace fmhc;
-  if (T <= 0 || nC <= 0 || nC % 8 != 0 || nC > (int64_t{1} << 26)) return 0;  // no MFMA path: no workspace
-  const int64_t nslices = (nC + 127) / 128;
-  return k1_bwd_runs(T, nC) * nslices * (8 * 2 * 4 * kWave) * static_cast<int64_t>(sizeof(float));
+  if (T <= 0 || !k1_bwd_mfma_path(nC, nC)) return 0;  // no MFMA path: no workspace
+  return k1_bwd_dw_bytes(T, bwd_slices(nC, nC));
 }
 
 extern "C" int fmhc_k1_bwd(const uint16_t* x_flat, const uint16_t* W, const uint16_t* grad_out,
@@ -1334,18 +1362,18 @@ extern "C" int fmhc_k1_bwd(const uint16_t* x_flat, const uint16_t* W, const uint
     return launch_status();
   }
   if (!x_flat || !W || !grad_out || !proj_out || !inv_rms || !grad_x) return FMHC_ERR_INVALID_ARGUMENT;
-  if (k1_bwd_mfma_path(x_flat, W, grad_out, proj_out, inv_rms, grad_x, nC)) {
+  if (k1_bwd_mfma_path(nC, nC)) {
     const int64_t need = fmhc_k1_bwd_workspace_bytes(T, nC);
     if (!workspace || workspace_bytes < need || !aligned16(workspace)) return FMHC_ERR_INVALID_ARGUMENT;
-    const int nslices = static_cast<int>((nC + 127) / 128);
-    const int64_t nruns = k1_bwd_runs(T, nC);
+    const BwdSlices sl = bwd_slices(nC, nC);
+    const int64_t nruns = k1_bwd_runs(T, sl.n);
     float* partial = static_cast<float*>(workspace);
-    launch_k1_bwd_mfma<true>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, partial, T, nc, nslices, nruns);
+    launch_k1_bwd_mfma<true>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, partial, T, nc, sl, nruns);
     const int st = launch_status();
     if (st != FMHC_OK) return st;
-    const int64_t per_part = static_cast<int64_t>(nslices) * (8 * 2 * 4 * kWave);
+    const int64_t per_part = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave);
     const unsigned nb = blocks_for(per_part / 4, 256);
-    k1_dw_reduce<<<dim3(nb), 256, 0, s>>>(partial, grad_W, nruns, nslices, nc, nb, K2ParamSums{});
+    k1_dw_reduce<<<dim3(nb), 256, 0, s>>>(partial, grad_W, nruns, sl, nc, nb, K2ParamSums{});
     return launch_status();
   }
   const int st = fmhc_k1_bwd_dx(x_flat, W, grad_out, proj_out, inv_rms, grad_x, T, nC, D_out, stream);
@@ -1383,24 +1411,32 @@ int k1_fwd_partials(const uint16_t* x_flat, const uint16_t* W, void* ws, int64_t
   return st == FMHC_OK ? p.S : -st;
 }
 
-int64_t k1_bwd_dw_runs(int64_t T, int64_t nC) { return k1_bwd_runs(T, nC); }
+int64_t k1_bwd_dw_runs(int64_t T, int64_t nC) { return k1_bwd_runs(T, (nC + 127) / 128); }
 
-int k1_dw_finish(const float* partial, uint16_t* grad_W, int64_t nruns, int nslices, int nC,
-                 const K2ParamSums& sums, hipStream_t s) {
-  const int64_t per_part = static_cast<int64_t>(nslices) * (8 * 2 * 4 * kWave);
+namespace {
+int dw_finish(const float* partial, uint16_t* grad_W, int64_t nruns, const BwdSlices& sl, int nC,
+              const K2ParamSums& sums, hipStream_t s) {
+  const int64_t per_part = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave);
   const unsigned nb = blocks_for(per_part / 4, 256);
   static_assert(kK2SumThreads == 256, "K2's parameter sums share the reduce's workgroups");
-  k1_dw_reduce<<<dim3(nb + kNPar), 256, 0, s>>>(partial, grad_W, nruns, nslices, nC, nb, sums);
+  k1_dw_reduce<<<dim3(nb + kNPar), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
   return launch_status();
+}
+}  // namespace
+
+int k1_dw_finish(const float* partial, uint16_t* grad_W, int64_t nruns, int nC, const K2ParamSums& sums,
+                 hipStream_t s) {
+  return dw_finish(partial, grad_W, nruns, bwd_slices(nC, nC), nC, sums, s);
 }
 
 // K1 backward of the pre-map region (premap.hip): grad_W as fmhc_k1_bwd and
 // grad_x = bf16(bf16(h_pre[t, j] go3[t, c]) + bf16(dx)).  On the MFMA path the
 // K3 term is computed in the store; otherwise grad_x must already hold it
 // (fmhc_k3_bwd's grad_x) and the element-wise kernel adds dx to it.
-bool k1_bwd_premap_fused(const void* x, const void* W, const void* go, const void* proj, const void* inv_rms,
-                         const void* gx, const void* go3, const void* gi, int64_t C) {
-  return C % 8 == 0 && k1_bwd_mfma_path(x, W, go, proj, inv_rms, gx, 4 * C) && aligned16(go3) && aligned16(gi);
+bool k1_bwd_premap_fused(int64_t C) { return k1_bwd_mfma_path(4 * C, bwd_premap_slices(C).len); }
+
+int64_t k1_bwd_premap_ws_bytes(int64_t T, int64_t C) {
+  return T > 0 && k1_bwd_premap_fused(C) ? k1_bwd_dw_bytes(T, bwd_premap_slices(C)) : 0;
 }
 
 int k1_bwd_premap(const uint16_t* x_flat, const uint16_t* W, const uint16_t* grad_proj,
@@ -1414,21 +1450,21 @@ int k1_bwd_premap(const uint16_t* x_flat, const uint16_t* W, const uint16_t* gra
     launch_k2_param_reduce(k2_sums, s);
     return launch_status();
   }
-  if (k1_bwd_premap_fused(x_flat, W, grad_proj, proj, inv_rms, grad_x, go3, grad_x_in, C)) {
-    if (!workspace || workspace_bytes < fmhc_k1_bwd_workspace_bytes(T, nC) || !aligned16(workspace))
+  if (k1_bwd_premap_fused(C)) {
+    if (!workspace || workspace_bytes < k1_bwd_premap_ws_bytes(T, C) || !aligned16(workspace))
       return FMHC_ERR_INVALID_ARGUMENT;
-    const int nslices = static_cast<int>((nC + 127) / 128);
-    const int64_t nruns = k1_bwd_runs(T, nC);
+    const BwdSlices sl = bwd_premap_slices(C);
+    const int64_t nruns = k1_bwd_runs(T, sl.n);
     float* partial = static_cast<float*>(workspace);
     if (grad_x_in)
-      launch_k1_bwd_mfma<true, true, true>(s, x_flat, W, grad_proj, proj, inv_rms, grad_x, partial, T, nc, nslices,
-                                           nruns, go3, h_pre, static_cast<int>(C), grad_x_in);
+      launch_k1_bwd_mfma<true, true, true>(s, x_flat, W, grad_proj, proj, inv_rms, grad_x, partial, T, nc, sl, nruns,
+                                           go3, h_pre, static_cast<int>(C), grad_x_in);
     else
-      launch_k1_bwd_mfma<true, true>(s, x_flat, W, grad_proj, proj, inv_rms, grad_x, partial, T, nc, nslices,
-                                     nruns, go3, h_pre, static_cast<int>(C));
+      launch_k1_bwd_mfma<true, true>(s, x_flat, W, grad_proj, proj, inv_rms, grad_x, partial, T, nc, sl, nruns,
+                                     go3, h_pre, static_cast<int>(C));
     const int st = launch_status();
     if (st != FMHC_OK) return st;
-    return k1_dw_finish(partial, grad_W, nruns, nslices, nc, k2_sums, s);
+    return dw_finish(partial, grad_W, nruns, sl, nc, k2_sums, s);
   }
   k1_bwd_scalar<true><<<dim3(blocks_for(T, 4)), 256, 0, s>>>(x_flat, W, grad_proj, proj, inv_rms, grad_x,
                                                              grad_x_in, T, nc);

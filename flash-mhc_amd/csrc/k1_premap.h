@@ -55,14 +55,15 @@ int k1_fwd_partials(const uint16_t* x_flat, const uint16_t* W, void* ws, int64_t
                     int64_t nC, hipStream_t s);
 
 // True when k1_bwd_premap computes the K3 term of grad_x itself (MFMA path);
-// otherwise grad_x must hold it on entry.  gi: the incoming gradient or null.
-bool k1_bwd_premap_fused(const void* x, const void* W, const void* go, const void* proj, const void* inv_rms,
-                         const void* gx, const void* go3, const void* gi, int64_t C);
+// otherwise grad_x must hold it on entry.
+bool k1_bwd_premap_fused(int64_t C);
+// Workspace bytes k1_bwd_premap needs (0 off the MFMA path).
+int64_t k1_bwd_premap_ws_bytes(int64_t T, int64_t C);
 
 // grad_W (32, 4C) and grad_x = bf16(bf16(h_pre[t, j] go3[t, c]) + bf16(dx)) of
 // K1 for x (T, 4, C); with grad_x_in (may be null, must not overlap grad_x)
-// grad_x = bf16(grad_x_in + that).  `workspace` as fmhc_k1_bwd
-// (fmhc_k1_bwd_workspace_bytes(T, 4C)).  K2's parameter gradients
+// grad_x = bf16(grad_x_in + that).  `workspace`: k1_bwd_premap_ws_bytes(T, C),
+// 16-byte aligned.  K2's parameter gradients
 // (k2_bwd_partials) are summed by the same launch as grad_W's partials.
 int k1_bwd_premap(const uint16_t* x_flat, const uint16_t* W, const uint16_t* grad_proj,
                   const uint16_t* proj, const float* inv_rms, const uint16_t* go3, const float* h_pre,
@@ -86,8 +87,8 @@ int k3_bwd_lanes8(int C);
 // plus, in extra workgroups, K2's parameter gradients from `sums`
 // (k1_dw_reduce, k1.hip).
 int64_t k1_bwd_dw_runs(int64_t T, int64_t nC);
-int k1_dw_finish(const float* partial, uint16_t* grad_W, int64_t nruns, int nslices, int nC,
-                 const K2ParamSums& sums, hipStream_t s);
+int k1_dw_finish(const float* partial, uint16_t* grad_W, int64_t nruns, int nC, const K2ParamSums& sums,
+                 hipStream_t s);
 
 // The pre-map backward with one read of x (premap_split.hip), for many tokens
 // (T >= kSplitMinT) and C a multiple of 128 with the MFMA path's alignments.

@@ -301,7 +301,7 @@ PremapWs premap_ws(int64_t T, int64_t C) {
   w.gp = round_up(T * 4 * 4);                   // grad_proj (T, 32) bf16
   w.k2 = w.gp + round_up(T * 32 * 2);           // K2 parameter partials
   w.k1 = w.k2 + round_up(fmhc_k2_bwd_workspace_bytes(T));  // K1 grad_W partials
-  w.ring = w.k1 + round_up(fmhc_k1_bwd_workspace_bytes(T, 4 * C));  // the split backward's exchange ring
+  w.ring = w.k1 + round_up(k1_bwd_premap_ws_bytes(T, C));  // the split backward's exchange ring
   w.total = w.ring + (T > 0 && C % kSliceCols == 0 ? round_up(premap_split_ring_bytes(T, C)) : 0);
   return w;
 }
@@ -486,7 +486,7 @@ extern "C" int fmhc_premap_bwd(const uint16_t* x, const uint16_t* W, const void*
   float* gh = T > 0 ? reinterpret_cast<float*>(ws + w.gh) : nullptr;
   uint16_t* gp = T > 0 ? reinterpret_cast<uint16_t*>(ws + w.gp) : nullptr;
   int st = FMHC_OK;
-  const bool fused = T > 0 && k1_bwd_premap_fused(x, W, gp, proj, inv_rms, grad_x, grad_layer_input, grad_x_in, C);
+  const bool fused = T > 0 && k1_bwd_premap_fused(C);
   K2Params P;
   if (!k2_params(alpha_pre, alpha_post, alpha_res, bias, perm, param_dtype, P)) return FMHC_ERR_INVALID_ARGUMENT;
   // K2's backward, whose parameter partials K1's grad_W reduce also sums.

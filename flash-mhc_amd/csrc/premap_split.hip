@@ -541,8 +541,10 @@ int split_spin() {
 bool premap_split_ok(const void* x, const void* W, const void* proj, const void* inv_rms, const void* gx,
                      const void* go3, const void* gi, int64_t T, int64_t C) {
   if (T < kSplitMinT || C % kSliceCols != 0 || C / kSliceCols > kMaxSlices) return false;
-  // The alignments and sizes of k1_bwd_mfma's pre-map path (its grad_proj operand is proj's alignment here).
-  if (!k1_bwd_premap_fused(x, W, proj, proj, inv_rms, gx, go3, gi, C)) return false;
+  // k1_bwd_mfma's pre-map path, with 16-byte aligned operands.
+  if (!k1_bwd_premap_fused(C)) return false;
+  for (const void* p : {x, W, proj, inv_rms, gx, go3, gi})
+    if (!aligned16(p)) return false;
   // The slice order is K3's backward's for this shape.
   return k3_canon(C, k3_bwd_lanes8(static_cast<int>(C)));
 }
@@ -596,7 +598,7 @@ int premap_bwd_split(const uint16_t* x, const uint16_t* W, const uint16_t* proj,
   st = launch_status();
   if (st != FMHC_OK) return st;
   const K2ParamSums sums{k2_partial, sh.nblocks, grad_alpha_pre, grad_alpha_post, grad_alpha_res, grad_bias, P.bf16};
-  return k1_dw_finish(dw_partial, grad_W, sh.nruns, sh.nslices, static_cast<int>(4 * C), sums, s);
+  return k1_dw_finish(dw_partial, grad_W, sh.nruns, static_cast<int>(4 * C), sums, s);
 }
 
 }  // namespace fmhc

@@ -1,0 +1,85 @@
+"""Widths that are not a multiple of eight, and operands off 16-byte alignment,
+on the matrix-core and 16-byte kernels: the last columns of a row (fewer than
+eight), rows shorter than a wave's slice, the first and last rows of a 16-token
+block, and base addresses 2 and 6 bytes off a 16-byte boundary.  Against the
+oracle (tests/parity.py's bounds), and bit for bit against the separate
+kernels where both do the same arithmetic."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from flash_mhc import build_permutation_matrices
+from flash_mhc import kernels as K
+from oracle import mhc_oracle as O
+from parity import check_bf16
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+BF16 = torch.bfloat16
+
+# C = 8 ... 17: rows of one or two groups; 127 / 129 / 131: either side of a
+# 128-column slice; 257, 1001: several slices, odd.  T around the 16-token
+# block and beyond the few-token forms (1037, 6150).
+SHAPES = [(1, 9), (15, 15), (16, 8), (17, 17), (33, 127), (300, 129), (1037, 131), (6150, 257), (2100, 1001)]
+
+
+def _at(t: torch.Tensor, off: int) -> torch.Tensor:
+    """t on the GPU, its base `off` elements past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 8, device=DEV, dtype=t.dtype)
+    view = buf[off:off + t.numel()].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+def _inputs(T, C, off, seed):
+    g = torch.Generator().manual_seed(seed)
+    rn = lambda *s, scale=1.0: (torch.randn(s, generator=g) * scale).to(BF16)
+    x = rn(T, 4, C)
+    x[::5] *= 50
+    return rn, _at(x, off), _at(rn(32, 4 * C, scale=0.02), off)
+
+
+def _params(C):
+    g = torch.Generator().manual_seed(C)
+    return [t.to(DEV) for t in (torch.tensor([0.8]), torch.tensor([1.2]), torch.tensor([1.7]),
+                                torch.randn(32, generator=g) * 0.5, build_permutation_matrices(4)[0])]
+
+
+@pytest.mark.parametrize("off", [0, 1, 3])
+@pytest.mark.parametrize("T,C", SHAPES)
+def test_k1_bwd(T, C, off):
+    nC = 4 * C
+    rn, x, W = _inputs(T, C, off, 11 * T + C + off)
+    x = x.view(T, nC)
+    proj, inv = K.k1_fwd(x, W)
+    go = _at(rn(T, 32), off)
+    inv = _at(inv.cpu(), off)  # 4-byte alignment only
+    gx, gW = K.k1_bwd(go, x, W, proj, inv)
+    R, S = O.k1_bwd_dx(go.cpu(), x.cpu(), W.cpu(), proj.cpu(), inv.cpu())
+    check_bf16("grad_x", gx, R, S, 64)
+    assert torch.equal(K.k1_bwd_dx(go, x, W, proj, inv), gx)
+    R, S = O.k1_grad_W(go.cpu(), x.cpu(), inv.cpu())
+    check_bf16("grad_W", gW, R, S, T)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("T,C", SHAPES)
+def test_premap_bwd(T, C, off):
+    nC = 4 * C
+    rn, x, W = _inputs(T, C, off, 13 * T + C + off)
+    p = _params(C)
+    li, H, hq, hp, proj, inv = K.premap_fwd(x, W, *p)
+    g_li, g_in = _at(rn(T, C), off), _at(rn(T, 4, C), off)
+    gx, gW, *pg = K.premap_bwd(x, W, *p, hp, proj, inv, g_li, hq, H, g_in)
+    gx3, gh = K.k3_bwd(g_li, x, hp)
+    gp, *rpg = K.k2_bwd(proj, *p, gh, hq, H)
+    dx, _ = K.k1_bwd(gp, x.view(T, nC), W, proj, inv)
+    # Three gradients of x, each rounded to bf16, added in autograd's order.
+    assert torch.equal(gx, g_in + (gx3 + dx.view(T, 4, C)))
+    for u, v in zip(pg, rpg):
+        assert torch.equal(u, v)
+    R, S = O.k1_grad_W(gp.cpu(), x.view(T, nC).cpu(), inv.cpu())
+    check_bf16("grad_W", gW, R, S, T)
