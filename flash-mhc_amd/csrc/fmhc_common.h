@@ -4,14 +4,15 @@
 //   * bf16 tensors arrive as uint16_t bit patterns, row-major and contiguous.
 //   * fp32 accumulation everywhere; every bf16 output is rounded exactly once,
 //     round-to-nearest-even, by the hardware v_cvt_pk_bf16_f32 conversion.
-//   * The "vector" code paths move 16 bytes (8 bf16) per lane per memory
-//     instruction; they need C % 8 == 0 and 16-byte aligned base pointers.
-//     The "scalar" code paths move one element per lane and accept any C and
-//     any 2-byte alignment.
+//   * A lane moves 16 bytes (8 bf16) per memory instruction, at any 2-byte
+//     alignment; the up to 7 last elements of a row with C % 8 != 0 are moved
+//     one per lane.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "../../include/flash_mhc_hip.h"
 
@@ -34,6 +35,7 @@ typedef unsigned int u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *static_cast<const u32x4_any*>(p); }
+__device__ __forceinline__ void st16(void* p, u32x4 v) { *static_cast<u32x4_any*>(p) = v; }
 __device__ __forceinline__ f32x4 ld16f(const void* p) { return *static_cast<const f32x4_any*>(p); }
 
 // Streaming loads/stores.  Data that is read or written exactly once per
@@ -76,7 +78,7 @@ __device__ __forceinline__ void st16_stream(void* p, u32x4 v) {
 #if FMHC_NT_STORES
   __builtin_nontemporal_store(v, static_cast<u32x4_any*>(p));
 #else
-  *static_cast<u32x4_any*>(p) = v;
+  st16(p, v);
 #endif
 }
 
@@ -120,94 +122,111 @@ __device__ __forceinline__ u32x4 pack8(const float f[8]) {
   return v;
 }
 
-// Element group moved by one lane per step: VEC = 8 (one 16-byte vector) or
-// VEC = 1 (one bf16 scalar).  `idx` counts groups, so the element offset is
+// Element group moved by one lane per step: VEC = 8 (one 16-byte vector) or,
+// for the elements past a row's last whole group, VEC = 1 (one bf16 scalar).  `idx` counts groups, so the element offset is
 // idx * VEC.  raw() issues the load and keeps the packed bf16 bits; unpack()
-// widens them to fp32; load() does both.
-template <int VEC>
+// widens them to fp32; load() does both.  NT: with the nontemporal hint.
+template <int VEC, bool NT>
 struct Lanes;
+template <int VEC>
+using Vec = std::integral_constant<int, VEC>;
 
-template <>
-struct Lanes<8> {
+template <bool NT>
+struct Lanes<8, NT> {
   using Raw = u32x4;
   __device__ static __forceinline__ Raw raw(const uint16_t* __restrict__ row, int idx) {
-    return ld_stream(reinterpret_cast<const u32x4*>(row) + idx);
+    return NT ? ld16_stream(row + 8 * idx) : ld16(row + 8 * idx);
   }
   __device__ static __forceinline__ void unpack(const Raw v, float f[8]) { unpack8(v, f); }
   __device__ static __forceinline__ void load(const uint16_t* __restrict__ row, int idx, float f[8]) {
     unpack8(raw(row, idx), f);
   }
   __device__ static __forceinline__ void store(uint16_t* __restrict__ row, int idx, const float f[8]) {
-    st_stream(reinterpret_cast<u32x4*>(row) + idx, pack8(f));
+    if constexpr (NT)
+      st16_stream(row + 8 * idx, pack8(f));
+    else
+      st16(row + 8 * idx, pack8(f));
   }
 };
 
-template <>
-struct Lanes<1> {
-  using Raw = uint32_t;
-  __device__ static __forceinline__ Raw raw(const uint16_t* __restrict__ row, int idx) { return row[idx]; }
-  __device__ static __forceinline__ void unpack(const Raw v, float f[1]) { f[0] = __uint_as_float(v << 16); }
+template <bool NT>
+struct Lanes<1, NT> {
   __device__ static __forceinline__ void load(const uint16_t* __restrict__ row, int idx, float f[1]) {
-    unpack(raw(row, idx), f);
+    f[0] = bf16_to_f32(row[idx]);
   }
   __device__ static __forceinline__ void store(uint16_t* __restrict__ row, int idx, const float f[1]) {
     row[idx] = f32_to_bf16(f[0]);
   }
 };
 
-// K3 forward of one token: out[c] = bf16(h0 x0[c] + h1 x1[c] + h2 x2[c] +
-// h3 x3[c]), the products added in stream order with fused multiply-adds;
-// element groups g = first, first + step, ... below C / VEC.  Shared by the
-// K3 kernel and the pre-map's few-token kernel, which must agree bit for bit.
-template <int VEC>
-__device__ __forceinline__ void k3_token(const uint16_t* __restrict__ x0, const float h[4],
-                                         uint16_t* __restrict__ orow, int first, int step, int C) {
-  const uint16_t* x1 = x0 + C;
-  const uint16_t* x2 = x1 + C;
-  const uint16_t* x3 = x2 + C;
-  const int ng = C / VEC;
-#pragma unroll 2
-  for (int g = first; g < ng; g += step) {
-    float a[VEC], b[VEC], c[VEC], d[VEC], o[VEC];
-    Lanes<VEC>::load(x0, g, a);
-    Lanes<VEC>::load(x1, g, b);
-    Lanes<VEC>::load(x2, g, c);
-    Lanes<VEC>::load(x3, g, d);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      float acc = h[0] * a[e];
-      acc = __builtin_fmaf(h[1], b[e], acc);
-      acc = __builtin_fmaf(h[2], c[e], acc);
-      o[e] = __builtin_fmaf(h[3], d[e], acc);
-    }
-    Lanes<VEC>::store(orow, g, o);
+// The elements past a row's last whole group of 8 (at most 7), one per lane:
+// f(idx) in lane `first` of the row's lanes (8 or more).  WHOLE: there are
+// none (C % 8 == 0), and the kernel carries no code for them.
+template <bool WHOLE, typename F>
+__device__ __forceinline__ void row_tail(int C, int first, F&& f) {
+  if constexpr (!WHOLE) {
+    const int c = (C & ~7) + first;
+    if (c < C) f(c);
   }
 }
 
-// Residency caps.  The K3 / K4 kernels use a few dozen VGPRs, so eight
-// 4-wave workgroups could share a CU; several run faster with fewer (the
-// host's launch reserves LDS the kernel does not use: the CU's 160 KiB hold
-// six workgroups of kLdsCapSix, five of kLdsCapFive).  K1's backward dx
-// likewise runs faster with one workgroup per CU than with two (k1.hip).
-// Measured at T = 65536 (GB/s in the six-kernel step, eight workgroups per CU
-// against the cap): K3 forward 6047-6092 against 6344-6405 with six (C =
-// 1024; also 5.60-5.67 against 5.88-5.93 TB/s at T = 262144, C = 4096);
-// K3 backward 6015-6070 against 6123-6175 with five at C = 1024 and
-// 6195-6252 against 6436-6605 at C = 2048; K4 forward 6325-6368 against
-// 6440-6478 with five at C = 1024, 6135-6175 against 6364-6420 at C = 2048.
-// Where a cap lost it is not applied: K3 backward at C = 4096 (5.57 against
-// 5.35-5.41 TB/s at T = 262144) and in the pre-map backward's reduce-only
-// pass (C = 2048: 846 against 862-872 us; at C = 1024 five per CU changed
-// nothing, 424-427 against 426-437 us at T = 65536), and K4 forward with few
-// workgroups per CU (T = 4096, C = 1024: a second round of workgroups).
-// Caps of five for K3 forward or six for K3 backward measured slower than
-// none, so the effect is not simply fewer memory requests in flight.
+// K3 forward of one element group of a token: out[c] = bf16(h0 x0[c] +
+// h1 x1[c] + h2 x2[c] + h3 x3[c]), the products added in stream order with
+// fused multiply-adds.  Shared by the K3 kernel and the pre-map's kernels,
+// which must agree bit for bit.
+template <int VEC, bool NT>
+__device__ __forceinline__ void k3_mix(const uint16_t* __restrict__ x0, const float h[4], uint16_t* __restrict__ orow,
+                                       int g, int C) {
+  const uint16_t* x1 = x0 + C;
+  const uint16_t* x2 = x1 + C;
+  const uint16_t* x3 = x2 + C;
+  float a[VEC], b[VEC], c[VEC], d[VEC], o[VEC];
+  Lanes<VEC, NT>::load(x0, g, a);
+  Lanes<VEC, NT>::load(x1, g, b);
+  Lanes<VEC, NT>::load(x2, g, c);
+  Lanes<VEC, NT>::load(x3, g, d);
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    float acc = h[0] * a[e];
+    acc = __builtin_fmaf(h[1], b[e], acc);
+    acc = __builtin_fmaf(h[2], c[e], acc);
+    o[e] = __builtin_fmaf(h[3], d[e], acc);
+  }
+  Lanes<VEC, NT>::store(orow, g, o);
+}
+
+// A whole token: groups first, first + step, ... below C / 8, then the tail.
+template <bool NT>
+__device__ __forceinline__ void k3_token(const uint16_t* __restrict__ x0, const float h[4],
+                                         uint16_t* __restrict__ orow, int first, int step, int C) {
+  const int ng = C / 8;
+#pragma unroll 2
+  for (int g = first; g < ng; g += step) k3_mix<8, NT>(x0, h, orow, g, C);
+  row_tail<NT>(C, first, [&](int c) { k3_mix<1, NT>(x0, h, orow, c, C); });
+}
+
+// Residency caps.  K3's and K4's kernels use a few dozen VGPRs, so eight
+// 4-wave workgroups could share a CU; they run faster with fewer, from 16
+// workgroups per CU on (below, a cap adds a round of workgroups).  The host's
+// launch reserves LDS the kernel does not use (cap_lds).  With one 16-byte
+// group per lane the best residency found is about kCapLanes lanes with work
+// per CU, 10 to 12 waves.  Swept over 0, 16, 20, ... 64 KiB per workgroup (us,
+// no cap against this one): T = 65536, C = 1000 K3 forward 110 against 104,
+// K3 backward 222 / 195, K4 forward 221 / 197, K4 backward 342 / 314; C = 1024
+// 112 / 106, 190 / 189, 194 / 187, 303 / 298; C = 2048 222 / 210, 398 / 382,
+// 398 / 378, 629 / 601; T = 32768, C = 2560 142 / 132, 247 / 236, 246 / 238,
+// 374 / 374; T = 60000, C = 520 (65 of 128 lanes) K3 backward 105 / 97, K4
+// backward 165 / 160.  K3 forward with a quarter of the lanes idle or more
+// loses with any cap (C = 520 52 -> 54, 712 35 -> 37) and takes none.
+// With several groups per lane (kLoopLpt): K3 forward six workgroups per CU
+// (T = 262144, C = 4096 5.60-5.67 -> 5.88-5.93 TB/s), K4 forward five, the
+// backwards none (K3 backward there 5.57 -> 5.35-5.41 with five).
+// K1's backward dx likewise runs faster with one workgroup per CU (k1.hip).
 #ifndef FMHC_LDS_CAP
 #define FMHC_LDS_CAP 1
 #endif
 constexpr unsigned kLdsCapSix = 24 * 1024;
 constexpr unsigned kLdsCapFive = 32 * 1024;
-constexpr unsigned kLdsCapFour = 40 * 1024;  // K4 backward, one group per lane (k4.hip)
 // One workgroup per CU (K1 backward dx, k1.hip).
 constexpr unsigned kLdsCapOne = 96 * 1024;
 constexpr unsigned kLdsPerCu = 160 * 1024;
@@ -220,6 +239,34 @@ inline unsigned lds_reserve(const void* kernel, unsigned dyn) {
   hipFuncAttributes a;
   if (dyn == 0 || hipFuncGetAttributes(&a, kernel) != hipSuccess) return 0u;
   return a.sharedSizeBytes + dyn <= kLdsPerCu ? dyn : 0u;
+}
+
+constexpr int kCapLanes = 680;
+// Unaligned groups keep more waves in flight (T = 30011, C = 1001, no cap / 1150
+// / 680 lanes: K3 backward 105 / 96 / 97, K4 forward 103 / 96 / 95, K4 backward
+// 157 / 154 / 153; T = 50000, C = 700 off 16 bytes 122 / 127 / 137, 120 / 126 /
+// 134, 197 / 206 / 223); K3 forward 52 / 55 / 58 there and takes none.
+constexpr int kCapLanesUnaligned = 1150;
+constexpr unsigned kCapMinBlocks = 16u * 256u;
+
+// A kernel's own LDS; callers keep it in a static of the launch site's
+// instantiation.
+inline unsigned own_lds(const void* kernel) {
+  hipFuncAttributes a;
+  return hipFuncGetAttributes(&a, kernel) == hipSuccess ? static_cast<unsigned>(a.sharedSizeBytes) : kLdsPerCu;
+}
+
+// The LDS reserve that leaves about kCapLanes (kCapLanesUnaligned) lanes with
+// work resident on a CU, for `blocks` workgroups of a kernel with `own` bytes
+// of LDS and `block` threads, lpt lanes per token and `groups` groups per row.
+// 1280 bytes stay free per workgroup, the granularity of an allocation.
+inline unsigned cap_lds(unsigned own, unsigned blocks, int block, int lpt, int groups, bool aligned) {
+  if (blocks < kCapMinBlocks || lpt < kWave) return 0u;
+  const int busy = block * groups / lpt;  // lanes with work in a workgroup
+  const int n = busy > 0 ? ((aligned ? kCapLanes : kCapLanesUnaligned) + busy / 2) / busy : 0;
+  if (n < 1 || n >= 8) return 0u;
+  const unsigned each = kLdsPerCu / static_cast<unsigned>(n);
+  return each > own + 1280u ? each - own - 1280u : 0u;
 }
 
 // Sum over the wave's 64 lanes, every lane receiving the total, with the
@@ -326,6 +373,102 @@ __device__ __forceinline__ float group_sum(float v) {
     for (int m = LPT / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
     return v;
   }
+}
+
+// Lanes per token of K3 and K4 for rows of C columns: one 16-byte group per
+// lane, rounded up to 8, 16, 32 or whole waves up to kMaxLpt lanes; longer
+// rows are walked by kLoopLpt lanes.  With one wave for all widths below 1024,
+// and 256 lanes above, the last trip of a lane's loop was nearly empty for many
+// widths, and every trip waited for its own loads.  K3 forward / backward, K4
+// forward / backward with that rule against this one (and its residency caps),
+// us: T = 65536, C = 1000 131 / 258 / 262 / 423 against 103 / 196 / 198 / 307;
+// T = 60000, C = 520 79 / 139 / 146 / 249 against 52 / 100 / 100 / 162;
+// T = 30000, C = 712 48 / 91 / 93 / 147 against 35 / 64 / 64 / 104, C = 1536
+// 80 / 147 / 142 / 237 against 73 / 131 / 131 / 204, C = 3000 168 / 338 / 324 /
+// 521 against 141 / 278 / 275 / 440; T = 16384, C = 2056 77 / 118 / 139 / 245
+// against 59 / 105 / 107 / 170.  512 lanes lost at C = 4096 (T = 16384 108 /
+// 203 / 193 / 315 against 124 / 227 / 206 / 351), which keeps 256 lanes with
+// two groups each.
+constexpr int kMaxLpt = 448;
+constexpr int kLoopLpt = 256;
+inline int lanes_per_token(int C) {
+  const int groups = C / 8;
+  if (groups > kMaxLpt) return kLoopLpt;
+  if (groups > 32) return (groups + kWave - 1) / kWave * kWave;
+  return groups > 16 ? 32 : groups > 8 ? 16 : 8;
+}
+
+constexpr int kBlock = 256;  // threads per workgroup, or one token's lanes where they do not divide it
+
+// Threads per workgroup for LPT lanes per token.
+template <int LPT>
+constexpr int block_of() {
+  return kBlock % LPT == 0 ? kBlock : LPT;
+}
+
+// Tokens per workgroup with lpt lanes per token.
+inline int64_t tokens_per_block(int lpt) { return kBlock % lpt == 0 ? kBlock / lpt : 1; }
+
+// How K3 and K4 walk a row, as compile-time constants: LPT lanes per token,
+// LOOP: several groups per lane, NT: whole, aligned groups, accessed with the
+// nontemporal hint.
+template <int kLpt, bool kLoop, bool kNt>
+struct RowWalk {
+  static constexpr int LPT = kLpt;
+  static constexpr bool LOOP = kLoop;
+  static constexpr bool NT = kNt;
+};
+
+// f(RowWalk) for rows of C columns whose 16-byte groups are aligned or not.
+// Unaligned groups (C % 8 != 0, or a base address off 16 bytes) leave out the
+// nontemporal hint: neighbouring lanes' groups share lines, and the hint
+// makes each access fetch or write its part on its own (K3 forward / backward,
+// K4 forward / backward with the hint against without, us: T = 65536, C = 100
+// 17.5 / 32.0 / 32.5 / 53.4 against 11.8 / 24.0 / 24.7 / 45.1; T = 20011,
+// C = 300 14.3 / 24.0 / 23.8 / 42.5 against 12.1 / 19.3 / 19.9 / 38.3).
+template <typename F>
+void with_row_walk(int C, bool aligned, F&& f) {
+  auto pick = [&](auto nt) {
+    constexpr bool NT = decltype(nt)::value;
+    const int lpt = lanes_per_token(C);
+    if (C / 8 > lpt) return f(RowWalk<kLoopLpt, true, NT>{});
+    switch (lpt) {
+      case 448: return f(RowWalk<448, false, NT>{});
+      case 384: return f(RowWalk<384, false, NT>{});
+      case 320: return f(RowWalk<320, false, NT>{});
+      case 256: return f(RowWalk<256, false, NT>{});
+      case 192: return f(RowWalk<192, false, NT>{});
+      case 128: return f(RowWalk<128, false, NT>{});
+      case 64: return f(RowWalk<64, false, NT>{});
+      case 32: return f(RowWalk<32, false, NT>{});
+      case 16: return f(RowWalk<16, false, NT>{});
+      default: return f(RowWalk<8, false, NT>{});
+    }
+  };
+  if (aligned && C % 8 == 0)
+    pick(std::true_type{});
+  else
+    pick(std::false_type{});
+}
+
+// Token of a lane.  LPT <= 64: 64 / LPT tokens per wave; wider: LPT / 64 waves
+// per token.
+template <int LPT>
+__device__ __forceinline__ int64_t token_of_lane(int lane) {
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  if constexpr (LPT > kWave) {
+    return static_cast<int64_t>(blockIdx.x) * (block_of<LPT>() / LPT) + wave / (LPT / kWave);
+  } else {
+    constexpr int TPW = kWave / LPT;
+    const int64_t first = (static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + wave) * TPW;
+    return LPT == kWave ? first : first + lane / LPT;
+  }
+}
+
+// Position of this lane among its token's LPT lanes.
+template <int LPT>
+__device__ __forceinline__ int sub_of_lane() {
+  return static_cast<int>(threadIdx.x) % LPT;
 }
 
 // Status helpers shared by the C entry points.

@@ -120,7 +120,7 @@ __device__ __forceinline__ void k3_block_pipelined(const uint16_t* __restrict__ 
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[4 * s + j] = Lanes<8>::raw(row + j * C, lane + 128 * p + 64 * s);
+      for (int j = 0; j < 4; ++j) v[4 * s + j] = Lanes<8, true>::raw(row + j * C, lane + 128 * p + 64 * s);
   };
   auto mix_store = [&](const u32x4 (&v)[8], int u) __attribute__((always_inline)) {
     const int tt = u / np, p = u - tt * np;
@@ -131,10 +131,10 @@ __device__ __forceinline__ void k3_block_pipelined(const uint16_t* __restrict__ 
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       float a[8], b[8], c[8], d[8], o[8];
-      Lanes<8>::unpack(v[4 * s], a);
-      Lanes<8>::unpack(v[4 * s + 1], b);
-      Lanes<8>::unpack(v[4 * s + 2], c);
-      Lanes<8>::unpack(v[4 * s + 3], d);
+      Lanes<8, true>::unpack(v[4 * s], a);
+      Lanes<8, true>::unpack(v[4 * s + 1], b);
+      Lanes<8, true>::unpack(v[4 * s + 2], c);
+      Lanes<8, true>::unpack(v[4 * s + 3], d);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         float acc = h[0] * a[e];
@@ -142,7 +142,7 @@ __device__ __forceinline__ void k3_block_pipelined(const uint16_t* __restrict__ 
         acc = __builtin_fmaf(h[2], c[e], acc);
         o[e] = __builtin_fmaf(h[3], d[e], acc);
       }
-      Lanes<8>::store(out + t * C, lane + 128 * p + 64 * s, o);
+      Lanes<8, true>::store(out + t * C, lane + 128 * p + 64 * s, o);
     }
   };
   u32x4 va[8], vb[8];
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
           if (t >= T) break;
           const f32x4 hv = tile_sm.hpre[16 * r + tt];
           const float h[4] = {hv[0], hv[1], hv[2], hv[3]};
-          k3_token<8>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
+          k3_token<true>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
         }
       }
     }
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
         if (t >= T) break;
         const f32x4 hv = tile_sm.hpre[tt];
         const float h[4] = {hv[0], hv[1], hv[2], hv[3]};
-        k3_token<8>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
+        k3_token<true>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
       }
     }
   }

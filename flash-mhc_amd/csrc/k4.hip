@@ -22,46 +22,20 @@ namespace fmhc {
 
 namespace {
 
-constexpr int kBlock = 256;  // 4 waves per workgroup, or one token's LPT lanes when more
-
-// Threads per workgroup for LPT lanes per token.
-template <int LPT>
-constexpr int block_of() {
-  return LPT > kBlock ? LPT : kBlock;
-}
-
-// LPT <= 64: 64 / LPT tokens per wave.  LPT = 128 or 256: LPT / 64 waves per
-// token; LPT a multiple of 64 above 256: one token per workgroup.
-template <int LPT>
-__device__ __forceinline__ int64_t token_of_lane(int lane) {
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  if constexpr (LPT > kWave) {
-    return static_cast<int64_t>(blockIdx.x) * (block_of<LPT>() / LPT) + wave / (LPT / kWave);
-  } else {
-    constexpr int TPW = kWave / LPT;
-    const int64_t first = (static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + wave) * TPW;
-    return LPT == kWave ? first : first + lane / LPT;
-  }
-}
-
-// Position of this lane among its token's LPT lanes.
-template <int LPT>
-__device__ __forceinline__ int sub_of_lane() {
-  return static_cast<int>(threadIdx.x) % LPT;
-}
-
-template <int VEC, int LPT>
-__global__ __launch_bounds__(block_of<LPT>()) void k4_fwd_kernel(const uint16_t* __restrict__ x,
+template <typename WALK>
+__global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_fwd_kernel(const uint16_t* __restrict__ x,
                                                         const uint16_t* __restrict__ lo,
                                                         const float* __restrict__ H,
                                                         const float* __restrict__ h_post,
                                                         uint16_t* __restrict__ out,
                                                         int64_t T, int C) {
+  constexpr int LPT = WALK::LPT;
+  constexpr bool LOOP = WALK::LOOP, NT = WALK::NT;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
   if (tok >= T) return;
   const int sub = sub_of_lane<LPT>();
-  const int ng = C / VEC;
+  const int ng = C / 8;
 
   float h[4][4], p[4];
   {
@@ -85,12 +59,12 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_fwd_kernel(const uint16_t*
   }
   const uint16_t* lrow = lo + tok * C;
 
-#pragma unroll 2
-  for (int g = sub; g < ng; g += LPT) {
+  auto mix = [&](auto vec, int g) __attribute__((always_inline)) {
+    constexpr int VEC = decltype(vec)::value;
     float l[VEC], xv[4][VEC];
-    Lanes<VEC>::load(lrow, g, l);
+    Lanes<VEC, NT>::load(lrow, g, l);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) Lanes<VEC>::load(xr[j], g, xv[j]);
+    for (int j = 0; j < 4; ++j) Lanes<VEC, NT>::load(xr[j], g, xv[j]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float o[VEC];
@@ -101,13 +75,20 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_fwd_kernel(const uint16_t*
         for (int j = 0; j < 4; ++j) acc = __builtin_fmaf(h[i][j], xv[j][e], acc);
         o[e] = acc;
       }
-      Lanes<VEC>::store(orow[i], g, o);
+      Lanes<VEC, NT>::store(orow[i], g, o);
     }
+  };
+  if constexpr (!LOOP) {
+    if (sub < ng) mix(Vec<8>{}, sub);
+  } else {
+#pragma unroll 2
+    for (int g = sub; g < ng; g += LPT) mix(Vec<8>{}, g);
   }
+  row_tail<NT>(C, sub, [&](int c) { mix(Vec<1>{}, c); });
 }
 
-template <int VEC, int LPT, bool EARLY>
-__global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t* __restrict__ x,
+template <typename WALK, bool EARLY>
+__global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uint16_t* __restrict__ x,
                                                         const uint16_t* __restrict__ lo,
                                                         const float* __restrict__ H,
                                                         const float* __restrict__ h_post,
@@ -117,6 +98,8 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t*
                                                         float* __restrict__ grad_H,
                                                         float* __restrict__ grad_hp,
                                                         int64_t T, int C) {
+  constexpr int LPT = WALK::LPT;
+  constexpr bool LOOP = WALK::LOOP, NT = WALK::NT;
   constexpr int WPT = LPT > kWave ? LPT / kWave : 1;  // waves per token
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
@@ -126,7 +109,7 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t*
   }
   const bool live = tok < T;
   const int sub = sub_of_lane<LPT>();
-  const int ng = C / VEC;
+  const int ng = C / 8;
 
   float shp[4] = {0.f, 0.f, 0.f, 0.f};
   float sH[4][4];
@@ -162,19 +145,19 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t*
   const uint16_t* lrow = lo + tok * C;
   uint16_t* glrow = grad_lo + tok * C;
 
-#pragma unroll 2
-  for (int g = sub; g < ng; g += LPT) {
+  auto round = [&](auto vec, int g) __attribute__((always_inline)) {
+    constexpr int VEC = decltype(vec)::value;
     float q[4][VEC], l[VEC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) Lanes<VEC>::load(gr[i], g, q[i]);
-    Lanes<VEC>::load(lrow, g, l);
+    for (int i = 0; i < 4; ++i) Lanes<VEC, NT>::load(gr[i], g, q[i]);
+    Lanes<VEC, NT>::load(lrow, g, l);
 
     // EARLY: the iteration's x rows load with grad_out and lo, before its
     // first store (the compiler keeps a load behind an earlier store).
     float xs[EARLY ? 4 : 1][VEC];
     if constexpr (EARLY) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) Lanes<VEC>::load(xr[j], g, xs[j]);
+      for (int j = 0; j < 4; ++j) Lanes<VEC, NT>::load(xr[j], g, xs[j]);
     }
     // grad_lo and the grad_h_post partial sums.
     {
@@ -186,7 +169,7 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t*
         acc = __builtin_fmaf(p[2], q[2][e], acc);
         o[e] = __builtin_fmaf(p[3], q[3][e], acc);
       }
-      Lanes<VEC>::store(glrow, g, o);
+      Lanes<VEC, NT>::store(glrow, g, o);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -201,7 +184,7 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t*
       if constexpr (EARLY)
         xv = xs[j];
       else
-        Lanes<VEC>::load(xr[j], g, xl);
+        Lanes<VEC, NT>::load(xr[j], g, xl);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -213,9 +196,16 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t*
         acc = __builtin_fmaf(h[2][j], q[2][e], acc);
         o[e] = __builtin_fmaf(h[3][j], q[3][e], acc);
       }
-      Lanes<VEC>::store(gxr[j], g, o);
+      Lanes<VEC, NT>::store(gxr[j], g, o);
     }
+  };
+  if constexpr (!LOOP) {
+    if (sub < ng) round(Vec<8>{}, sub);
+  } else {
+#pragma unroll 2
+    for (int g = sub; g < ng; g += LPT) round(Vec<8>{}, g);
   }
+  row_tail<NT>(C, sub, [&](int c) { round(Vec<1>{}, c); });
   }
 
   constexpr int GS = LPT < kWave ? LPT : kWave;
@@ -265,149 +255,62 @@ __global__ __launch_bounds__(block_of<LPT>()) void k4_bwd_kernel(const uint16_t*
   }
 }
 
-// Lanes per token: a full wave from one 8-element group per lane on (at
-// C = 512, 64 lanes make the backward 20% and the forward 4% faster than 32),
-// fewer lanes (more tokens per wave) for narrower rows.
-template <int VEC>
-int pick_lpt(int C) {
-  const int groups = C / VEC;
-  if (groups >= 64) return 64;
-  if (groups >= 32) return 32;
-  if (groups >= 16) return 16;
-  return 8;
-}
-
-// Widest layout (16-byte path): a workgroup of exactly one 8-element group
-// per lane and stream when a row's groups (a multiple of 64, from 320 to
-// kMaxLpt) do not split evenly over 256 lanes: C = 2560, 3072, 3584.  With
-// 256 lanes at C = 2560 (320 groups) a quarter of the lanes took a second
-// group while the rest waited; 320 lanes took the six-kernel step at
-// T = 65536 from 5677 to 6054 GB/s (K4 backward 5378 -> 6307).  C = 4096
-// (512 groups, two per lane at 256) measured the same at 512 and 256 lanes
-// (T = 65536 and 262144, within 2%) and keeps 256.
-#ifndef FMHC_K34_MAX_LPT
-#define FMHC_K34_MAX_LPT 512
-#endif
-constexpr int kMaxLpt = FMHC_K34_MAX_LPT;
-
-template <int VEC>
-int wide_lpt(int groups) {
-  if constexpr (VEC == 8) {
-    if (groups % kWave == 0 && groups % 256 != 0 && groups > 256 && groups <= kMaxLpt) return groups;
-  }
-  return 256;
-}
-
-// f(std::integral_constant<int, L>{}) for the lanes per token L the kernels
-// are built for; threads per workgroup block_of<L>().
-template <typename F>
-void with_lpt(int lpt, F&& f) {
-  switch (lpt) {
-    case 512: f(std::integral_constant<int, 512>{}); break;
-    case 448: f(std::integral_constant<int, 448>{}); break;
-    case 384: f(std::integral_constant<int, 384>{}); break;
-    case 320: f(std::integral_constant<int, 320>{}); break;
-    case 256: f(std::integral_constant<int, 256>{}); break;
-    case 128: f(std::integral_constant<int, 128>{}); break;
-    case 64: f(std::integral_constant<int, 64>{}); break;
-    case 32: f(std::integral_constant<int, 32>{}); break;
-    case 16: f(std::integral_constant<int, 16>{}); break;
-    default: f(std::integral_constant<int, 8>{}); break;
-  }
-}
-
-// Tokens per workgroup with lpt lanes per token.
-int64_t tokens_per_block(int lpt) {
-  return lpt > kWave ? (lpt > kBlock ? 1 : kBlock / lpt) : (kBlock / kWave) * (kWave / lpt);
-}
-
-// The forward kernel spreads a token over more lanes (up to a workgroup),
-// so that each lane has one or two 8-element groups per stream instead of a
-// loop over them.  Measured at T x C = 64 Mi elements: with 256 lanes per
-// token from C = 2048 on the kernel is 13-17% faster than with one wave, and
-// at C = 1024 2% faster with 128 lanes; few tokens gain most (latency bounds
-// that regime).
-template <int VEC>
-int pick_lpt_fwd(int C) {
-  const int groups = C / VEC;
-  if (groups >= 256) return wide_lpt<VEC>(groups);
-  if (groups >= 128) return 128;
-  return pick_lpt<VEC>(C);
-}
-
-// Backward: a workgroup per token from C = 2048 on (the 20 per-token sums
-// then finish across the waves in LDS): 13% faster there than one wave per
-// token at T x C = 64 Mi elements.  At C = 1024 two waves per token (one
-// 16-byte group per lane) with the residency cap of launch_k4_bwd: at
-// T = 65536 6389-6454 against 6270-6291 GB/s in the six-kernel step, 32768
-// 6298-6330 against 6149-6150, 20000 6071-6121 against 5999-6008, 262144
-// 6298-6369 against 6145-6233; below the cap's threshold two waves were
-// already 1-4 us faster (T = 4096 22.1 -> 21.0 us).  Other widths below
-// 2048 keep one wave (a second wave would leave lanes without a group).
-template <int VEC>
-int pick_lpt_bwd(int C) {
-  if (VEC == 8 && C / VEC == 128) return 128;
-  return C / VEC >= 256 ? wide_lpt<VEC>(C / VEC) : pick_lpt<VEC>(C);
-}
-
-template <int VEC>
 int launch_k4_fwd(const uint16_t* x, const uint16_t* lo, const float* H, const float* hp,
                   uint16_t* out, int64_t T, int C, hipStream_t s) {
-  const int lpt = pick_lpt_fwd<VEC>(C);
-  const dim3 grid(blocks_for(T, tokens_per_block(lpt)));
-  // Residency cap (fmhc_common.h) from 16 workgroups per CU on.
-  const bool cap = VEC == 8 && FMHC_LDS_CAP && grid.x >= 16u * 256u;
-  with_lpt(lpt, [&](auto l) {
-    constexpr int L = decltype(l)::value;
-    static const unsigned lds = lds_reserve(reinterpret_cast<const void*>(&k4_fwd_kernel<VEC, L>), kLdsCapFive);
-    k4_fwd_kernel<VEC, L><<<grid, block_of<L>(), cap ? lds : 0u, s>>>(x, lo, H, hp, out, T, C);
+  with_row_walk(C, aligned16(x) && aligned16(lo) && aligned16(out), [&](auto w) {
+    constexpr int L = decltype(w)::LPT;
+    // Tokens narrower than a wave are faster in the loop's schedule (T = 65536,
+    // C = 176 42.7 -> 36.5 us, 256 50.5 -> 48.6); wider ones equal or slower.
+    using Walk = RowWalk<L, decltype(w)::LOOP || L < kWave, decltype(w)::NT>;
+    const dim3 grid(blocks_for(T, tokens_per_block(L)));
+    // Residency cap (fmhc_common.h).
+    static const unsigned own = own_lds(reinterpret_cast<const void*>(&k4_fwd_kernel<Walk>));
+    unsigned lds = 0;
+    if (decltype(w)::LOOP)
+      lds = grid.x >= kCapMinBlocks ? kLdsCapFive : 0u;
+    else
+      lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::NT);
+    k4_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(x, lo, H, hp, out, T, C);
   });
   return launch_status();
 }
 
 constexpr int64_t kK4EarlyLanes = int64_t{16384} * 64;
 
-template <int VEC>
 int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const float* hp,
                   const uint16_t* go, uint16_t* gx, uint16_t* glo, float* gH, float* ghp,
                   int64_t T, int C, hipStream_t s) {
-  const int lpt = pick_lpt_bwd<VEC>(C);
-  const dim3 grid(blocks_for(T, tokens_per_block(lpt)));
-  // Residency cap (fmhc_common.h): four workgroups per CU where each lane
-  // has one 16-byte group (C = 512, 1024, 2048), from 16 workgroups per CU
-  // on.  Six-kernel step, GB/s for K4 backward, no cap against four:
-  // T = 65536, C = 512 6401-6416 against 6448-6455, C = 2048 6139-6169
-  // against 6387-6395 (cold 6127-6155 against 6426-6467); T = 262144,
-  // C = 512 6278-6295 against 6452-6485.  With two groups per lane a cap
-  // lost (C = 1024 on one wave per token: 5949-5969 against 6242-6249;
-  // C = 4096: 4742 against 5624); at C = 2560 and 3072 it changed nothing.
-  const bool cap = VEC == 8 && FMHC_LDS_CAP && C / VEC == lpt && lpt <= 256 && grid.x >= 16u * 256u;
-  // Few waves (up to 64 per CU): each iteration's loads go out before its
-  // stores, so a wave waits for one round trip per iteration instead of five
-  // (block step at C = 1024, HIP graph: T = 1024 96.5 -> 94.6 us, 6000 232.2
-  // -> 228.5 us; K4 backward alone at T = 16384 81.1 -> 79.0 us).  With more
-  // waves the extra registers (124 against 90: four waves per SIMD instead of
-  // five) cost more than the latency they hide (T = 32768 150.8 -> 153.5 us,
-  // 65536 302.2 -> 304.3 us).
-  auto launch = [&](auto early) {
-    constexpr bool E = decltype(early)::value;
-    with_lpt(lpt, [&](auto l) {
-      constexpr int L = decltype(l)::value;
-      static const unsigned lds =
-          lds_reserve(reinterpret_cast<const void*>(&k4_bwd_kernel<VEC, L, E && L >= kWave>), kLdsCapFour);
-      k4_bwd_kernel<VEC, L, E && L >= kWave><<<grid, block_of<L>(), cap ? lds : 0u, s>>>(x, lo, H, hp, go, gx, glo,
-                                                                                         gH, ghp, T, C);
-    });
-  };
-  // Measured on the 16-byte path with a wave or more per token; narrower
-  // tokens (C < 512) keep the loop as it is.
-  if constexpr (VEC == 8) {
-    if (lpt >= kWave && T * lpt <= kK4EarlyLanes) {
-      launch(std::true_type{});
-      return launch_status();
-    }
-  }
-  launch(std::false_type{});
+  const bool aligned = aligned16(x) && aligned16(lo) && aligned16(go) && aligned16(gx) && aligned16(glo);
+  with_row_walk(C, aligned, [&](auto w) {
+    using Walk = decltype(w);
+    constexpr int L = Walk::LPT;
+    const dim3 grid(blocks_for(T, tokens_per_block(L)));
+    auto launch = [&](auto walk, auto early) {
+      using W = decltype(walk);
+      constexpr bool E = decltype(early)::value;
+      // Residency cap (fmhc_common.h) with one group per lane, up to 256 lanes
+      // (T = 30000, C = 3000 440 us with and without).
+      static const unsigned own = own_lds(reinterpret_cast<const void*>(&k4_bwd_kernel<W, E>));
+      unsigned lds = 0;
+      if (FMHC_LDS_CAP && C / 8 <= L && L <= 256) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::NT);
+      k4_bwd_kernel<W, E><<<grid, block_of<L>(), lds, s>>>(x, lo, H, hp, go, gx, glo, gH, ghp, T, C);
+    };
+    // EARLY: all of a lane's loads go out before its first store, so a wave
+    // waits for one round trip instead of five, but holds more registers and
+    // leaves its stores to the end.  Few waves (up to 64 per CU) and unaligned
+    // rows take it (T = 1000, C = 2560 15.6 us, in the plain order 16.4; T = 1024,
+    // C = 1024 8.1 / 8.3; T = 30011, C = 1001 151 / 157); many waves are faster
+    // in the plain order, as the loop over groups schedules it even for one
+    // group per lane (T = 65536, C = 1000 322 -> 307 us, 1024 304 -> 299, 2048
+    // 618 -> 599; T = 65537, C = 2560 765 -> 756).  Tokens narrower than a wave
+    // keep the coefficients in vector registers and the plain order.
+    if constexpr (L < kWave)
+      launch(w, std::false_type{});
+    else if (!Walk::NT || T * L <= kK4EarlyLanes)
+      launch(w, std::true_type{});
+    else
+      launch(RowWalk<L, true, Walk::NT>{}, std::false_type{});
+  });
   return launch_status();
 }
 
@@ -426,10 +329,7 @@ extern "C" int fmhc_k4_fwd(const uint16_t* x, const uint16_t* lo, const float* H
   if (T == 0) return FMHC_OK;
   if (!x || !lo || !H || !h_post || !out) return FMHC_ERR_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int c = static_cast<int>(C);
-  if (C % 8 == 0 && aligned16(x) && aligned16(lo) && aligned16(out))
-    return launch_k4_fwd<8>(x, lo, H, h_post, out, T, c, s);
-  return launch_k4_fwd<1>(x, lo, H, h_post, out, T, c, s);
+  return launch_k4_fwd(x, lo, H, h_post, out, T, static_cast<int>(C), s);
 }
 
 extern "C" int fmhc_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H,
@@ -442,11 +342,6 @@ extern "C" int fmhc_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H
   if (!x || !lo || !H || !h_post || !grad_out || !grad_x || !grad_lo || !grad_H || !grad_h_post)
     return FMHC_ERR_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int c = static_cast<int>(C);
-  if (C % 8 == 0 && aligned16(x) && aligned16(lo) && aligned16(grad_out) && aligned16(grad_x) &&
-      aligned16(grad_lo))
-    return launch_k4_bwd<8>(x, lo, H, h_post, grad_out, grad_x, grad_lo, grad_H, grad_h_post, T,
-                            c, s);
-  return launch_k4_bwd<1>(x, lo, H, h_post, grad_out, grad_x, grad_lo, grad_H, grad_h_post, T, c,
-                          s);
+  return launch_k4_bwd(x, lo, H, h_post, grad_out, grad_x, grad_lo, grad_H, grad_h_post, T, static_cast<int>(C),
+                       s);
 }

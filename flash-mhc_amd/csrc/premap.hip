@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
   __syncthreads();
   const float h[4] = {hsh[0], hsh[1], hsh[2], hsh[3]};
   if (!pre) {
-    k3_token<VEC>(x0, h, layer_input + t * C, lane, kFinishThreads, C);
+    k3_token<VEC == 8>(x0, h, layer_input + t * C, lane, kFinishThreads, C);
     return;
   }
 #pragma unroll
@@ -188,16 +188,15 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
         acc = __builtin_fmaf(h[2], c[e], acc);
         o[e] = __builtin_fmaf(h[3], d[e], acc);
       }
-      Lanes<8>::store(layer_input + t * C, g, o);
+      Lanes<8, true>::store(layer_input + t * C, g, o);
     }
   }
 }
 
-// Backward, few tokens (T <= kK2BwdSmallT) where K3's backward runs 32 or 64
-// lanes per token: K3's reduce-only pass and K2's backward in one kernel,
+// Backward, few tokens (T <= kK2BwdSmallT) for rows of 17 to 255 groups of 8
+// columns: K3's reduce-only pass and K2's backward in one kernel,
 // kK2BwdTok tokens per workgroup.  A token's four grad_h_pre sums are
-// k3_bwd_kernel's (the same lanes, loop order and group sums) and stay in
-// registers; the token's first 32 lanes then run k2_bwd_token32 as
+// k3_bwd_kernel's (the same sums in the same order) and stay in registers; the token's first 32 lanes then run k2_bwd_token32 as
 // k2_bwd_small does, and the workgroup adds its tokens' parameter terms in
 // token order.  grad_proj and the parameter partials are those of K3's
 // backward followed by k2_bwd_small, bit for bit, with one launch and one
@@ -233,45 +232,44 @@ __global__ __launch_bounds__(kK2BwdTok * LPT) void k3_reduce_k2_bwd(
   const uint16_t* x2 = x1 + C;
   const uint16_t* x3 = x2 + C;
   const uint16_t* grow = go3 + t * C;
-  auto round = [&](int g, float (&acc)[4]) {
-    float gq[8], a[8], b[8], c[8], d[8];
-    Lanes<8>::load(grow, g, gq);
-    Lanes<8>::load(x0, g, a);
-    Lanes<8>::load(x1, g, b);
-    Lanes<8>::load(x2, g, c);
-    Lanes<8>::load(x3, g, d);
+  auto round = [&](auto vec, int g, float (&acc)[4]) __attribute__((always_inline)) {
+    constexpr int VEC = decltype(vec)::value;
+    float gq[VEC], a[VEC], b[VEC], c[VEC], d[VEC];
+    Lanes<VEC, true>::load(grow, g, gq);
+    Lanes<VEC, true>::load(x0, g, a);
+    Lanes<VEC, true>::load(x1, g, b);
+    Lanes<VEC, true>::load(x2, g, c);
+    Lanes<VEC, true>::load(x3, g, d);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < VEC; ++e) {
       acc[0] = __builtin_fmaf(a[e], gq[e], acc[0]);
       acc[1] = __builtin_fmaf(b[e], gq[e], acc[1]);
       acc[2] = __builtin_fmaf(c[e], gq[e], acc[2]);
       acc[3] = __builtin_fmaf(d[e], gq[e], acc[3]);
     }
   };
-  if constexpr (CANON) {
-    // Every slot computes (idle ones on the last token), so the slot's lanes
-    // are all active for the row sums.
-    constexpr int kRounds = LPT == 64 ? 4 : 2;  // fewer than 256 (64) groups for 64 (32) lanes
-    float e[kRounds][4];
+  // Every slot computes (idle ones on the last token), so the slot's lanes are
+  // all active for the sums below.
+  constexpr int kRounds = LPT == 64 ? 4 : 1;  // fewer than 256 groups for 64 lanes, up to 32 for 32
+  const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+  float e[kRounds][4];
 #pragma unroll
-    for (int k = 0; k < kRounds; ++k) {
+  for (int k = 0; k < kRounds; ++k) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) e[k][j] = 0.f;
-      if (sub + k * LPT < ng) round(sub + k * LPT, e[k]);
-    }
-    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    for (int j = 0; j < 4; ++j) e[k][j] = 0.f;
+    if (sub + k * LPT < ng) round(Vec<8>{}, sub + k * LPT, e[k]);
+    if (k == 0) row_tail<false>(C, sub, [&](int c) { round(Vec<1>{}, c, e[0]); });
+  }
 #pragma unroll
-    for (int k = 0; k < kRounds; ++k) {
-      if (k * LPT >= ng) break;  // uniform
+  for (int k = 0; k < kRounds; ++k) {
+    if (k * LPT >= ng) break;  // uniform
+    if constexpr (CANON) {
       slice_sums_add<LPT>(e[k], s, k, ng / 16, lane);
-    }
-  } else {
-    if (valid) {
-#pragma unroll 2
-      for (int g = sub; g < ng; g += LPT) round(g, s);
-    }
+    } else {
+      // k3_bwd_kernel's waves hold 64 groups each and add their sums in order.
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s[j] = group_sum<LPT>(s[j]);
+      for (int j = 0; j < 4; ++j) s[j] += group_sum<LPT>(e[k][j]);
+    }
   }
   const float s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3];
 
@@ -491,8 +489,10 @@ extern "C" int fmhc_premap_bwd(const uint16_t* x, const uint16_t* W, const void*
   if (!k2_params(alpha_pre, alpha_post, alpha_res, bias, perm, param_dtype, P)) return FMHC_ERR_INVALID_ARGUMENT;
   // K2's backward, whose parameter partials K1's grad_W reduce also sums.
   K2ParamSums sums;
-  const int lanes = C % 8 == 0 ? k3_bwd_lanes8(static_cast<int>(C)) : 0;
-  if (fused && T <= kK2BwdSmallT && (lanes == 32 || lanes == 64) && aligned16(x) && aligned16(grad_layer_input)) {
+  // Half a wave per token for rows of 17 to 32 groups of 8, a wave up to 255.
+  const int64_t groups = C / 8;
+  const int lanes = groups > 32 ? 64 : 32;
+  if (fused && T <= kK2BwdSmallT && groups > 16 && groups < 256) {
     // Few tokens: K3's reduce-only pass and K2's backward as one kernel.
     float* partial = reinterpret_cast<float*>(ws + w.k2);
     const dim3 grid(static_cast<unsigned>((T + kK2BwdTok - 1) / kK2BwdTok));

@@ -546,7 +546,7 @@ bool premap_split_ok(const void* x, const void* W, const void* proj, const void*
   for (const void* p : {x, W, proj, inv_rms, gx, go3, gi})
     if (!aligned16(p)) return false;
   // The slice order is K3's backward's for this shape.
-  return k3_canon(C, k3_bwd_lanes8(static_cast<int>(C)));
+  return k3_canon(C, lanes_per_token(static_cast<int>(C)));
 }
 
 int64_t premap_split_ring_bytes(int64_t T, int64_t C) {

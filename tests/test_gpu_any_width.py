@@ -13,7 +13,7 @@ import torch
 from flash_mhc import build_permutation_matrices
 from flash_mhc import kernels as K
 from oracle import mhc_oracle as O
-from parity import check_bf16
+from parity import check_bf16, check_fp32
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +83,34 @@ def test_premap_bwd(T, C, off):
         assert torch.equal(u, v)
     R, S = O.k1_grad_W(gp.cpu(), x.view(T, nC).cpu(), inv.cpu())
     check_bf16("grad_W", gW, R, S, T)
+
+
+# K3 / K4: one 16-byte group per lane over 8, 16, 32, 64, 128, 192, ... 448
+# lanes per token and several groups per lane beyond; rows that end inside a
+# group, at a wave's edge, or one group into the next wave; enough tokens for
+# the residency caps in two of them.
+K34 = [(1, 1), (33, 7), (9, 8), (130, 65), (65, 136), (31, 264), (77, 512), (45, 519), (5, 520), (19, 1032),
+       (7, 1535), (3, 1536), (6, 2056), (4, 3079), (2, 3592), (3, 4100), (20001, 200), (9001, 1000)]
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("T,C", K34)
+def test_k3_k4(T, C, off):
+    rn, x, _W = _inputs(T, C, off, 17 * T + C + off)
+    g = torch.Generator().manual_seed(T + C)
+    h = torch.rand(T, 4, generator=g).to(DEV)
+    H = torch.randn(T, 4, 4, generator=g).to(DEV)
+    lo, go3, go4 = _at(rn(T, C), off), _at(rn(T, C), off), _at(rn(T, 4, C), off)
+    c = lambda t: t.cpu()
+    check_bf16("k3 out", K.k3_fwd(x, h), *O.k3_fwd(c(x), c(h)), 4)
+    gx, gh = K.k3_bwd(go3, x, h)
+    gxR, gxS, ghR, ghS = O.k3_bwd(c(go3), c(x), c(h))
+    check_bf16("k3 grad_x", gx, gxR, gxS, 1)
+    check_fp32("k3 grad_h_pre", gh, ghR, ghS, C)
+    check_bf16("k4 out", K.k4_fwd(x, lo, H, h), *O.k4_fwd(c(x), c(lo), c(H), c(h)), 5)
+    gx, glo, gH, ghp = K.k4_bwd(go4, x, lo, H, h)
+    ref = O.k4_bwd(c(go4), c(x), c(lo), c(H), c(h))
+    check_bf16("k4 grad_x", gx, *ref["grad_x"], 4)
+    check_bf16("k4 grad_lo", glo, *ref["grad_lo"], 4)
+    check_fp32("k4 grad_H", gH, *ref["grad_H"], C)
+    check_fp32("k4 grad_hp", ghp, *ref["grad_hp"], C)
