@@ -6,8 +6,7 @@
 // k1_bwd_mfma (dx; with DW also grad_W's per-run partials, which
 // k1_dw_reduce adds; with EPI / GI the pre-map backward's extra terms of
 // grad_x in the same store), and element-wise kernels for what these do not
-// take (forward: nC % 8 != 0, unaligned pointers; backward: fewer than 8
-// columns; rows beyond their 32-bit offsets).
+// take: fewer than 8 columns, and rows beyond their 32-bit offsets.
 //
 //   forward   inv_rms[t] = rsqrt(sum_k x[t,k]^2 / nC + 1e-6)
 //             out[t,d]   = bf16(inv_rms[t] * sum_k x[t,k] * W[d,k])
@@ -62,7 +61,7 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 
 // ---------------------------------------------------------------------------
-// K1 forward, matrix-core path (nC % 8 == 0, 16-byte aligned x / W / out).
+// K1 forward, matrix-core path (any nC from 8 on, any alignment).
 //
 // A workgroup owns 16*R consecutive tokens and SPLIT waves.  The nC axis is
 // cut into 64-wide chunks; wave w accumulates chunks w, w + SPLIT, ... for all
@@ -80,6 +79,17 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 // directly from HBM is 3% slower than loading whole lines (8 tokens x 128
 // bytes per instruction) and moving them into the MFMA layout through a
 // wave-private LDS tile (16R tokens x 128 bytes).
+// The first n (0 to 7) of a group's 8 elements cleared (SKIP: n is 0).
+template <bool SKIP>
+__device__ __forceinline__ u32x4 drop_front(u32x4 v, int n) {
+  if constexpr (!SKIP) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      v[w] &= (2 * w < n ? 0u : 0xffffu) | (2 * w + 1 < n ? 0u : 0xffff0000u);
+  }
+  return v;
+}
+
 // The pre-map tile epilogue's shared memory (TILE below).
 template <int R>
 struct TileSmem {
@@ -157,6 +167,29 @@ __device__ __forceinline__ void k3_block_pipelined(const uint16_t* __restrict__ 
   }
 }
 
+// K3 over n tokens from tb on by wave `wave` of `waves`, for rows of up to
+// kNarrowC columns: 8, 16 or 32 lanes per token, as many tokens at a time as
+// fill the wave.  A wave per token left half to seven eighths of its lanes
+// idle (pre-map forward at T = 65536, C = 24 28.4 -> 16.8 us, 64 30.4 -> 19.0,
+// 128 39.3 -> 27.7, 256 50.9 -> 46.5).
+constexpr int kNarrowC = 8 * 32 + 7;
+__device__ __forceinline__ void k3_narrow_tokens(const uint16_t* __restrict__ x, const f32x4* hpre,
+                                                 uint16_t* __restrict__ out, int64_t tb, int64_t T, int C,
+                                                 bool groups16, int lane, int wave, int waves, int n) {
+  const int sh = C >= 8 * 17 ? 5 : C >= 8 * 9 ? 4 : 3;  // lanes per token: 1 << sh
+  const int per = kWave >> sh;
+  for (int tt = wave * per + (lane >> sh); tt < n; tt += waves * per) {
+    const int64_t t = tb + tt;
+    if (t >= T) break;
+    const f32x4 hv = hpre[tt];
+    const float h[4] = {hv[0], hv[1], hv[2], hv[3]};
+    if (groups16)
+      k3_token<true>(x + t * 4 * C, h, out + t * C, lane & ((1 << sh) - 1), 1 << sh, C);
+    else
+      k3_token<false>(x + t * 4 * C, h, out + t * C, lane & ((1 << sh) - 1), 1 << sh, C);
+  }
+}
+
 // SPLITK (few tokens): blockIdx.y selects a range of cps chunks, and the
 // workgroup writes its fp32 partial sums (32 projections + sum of squares per
 // token) to part[t][33][S4] (S4 = gridDim.y rounded up to 4) instead of the
@@ -168,7 +201,18 @@ __device__ __forceinline__ void k3_block_pipelined(const uint16_t* __restrict__ 
 // streams into the layer input while L2 and the memory-side cache may still
 // hold the rows it just read (its x loads are ordinary loads, which allocate
 // there).  Same values as K1 -> K2 -> K3 launched separately.
-template <int R, int SPLIT, bool SPLITK, bool TILE = false>
+// WHOLE: rows of whole 128-byte lines (the plain kernel), of whole aligned
+// 16-byte groups and more than kNarrowC columns (TILE), or of whole groups
+// (SPLITK); otherwise x is loaded without the nontemporal hint, the last group
+// of a row may be partial, and K3 runs its unaligned or narrow form.  Lines
+// that two tokens' loads share are fetched twice under the hint (C = 1000
+// FETCH_SIZE 1.26 x x; T = 65536 119 -> 113 us without it, T = 60000, C = 520
+// 59.7 -> 56.6, T = 65536, C = 100 17.8 -> 13.1); against the element-wise
+// kernel odd widths took before, T = 30011, C = 1001 2197 -> 64 us, T = 3000,
+// C = 77 18.2 -> 3.8, and with K2 and K3 on each tile (pre-map forward)
+// 2246 -> 125 and 24.6 -> 6.5 us, T = 20011, C = 300 42 -> 32, T = 65536,
+// C = 100 43 -> 28; x off 16 bytes at T = 8192, C = 1024 781 -> 52.
+template <int R, int SPLIT, bool SPLITK, bool TILE, bool WHOLE>
 __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __restrict__ x,
                                                              const uint16_t* __restrict__ W,
                                                              uint16_t* __restrict__ out,
@@ -248,15 +292,15 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
     const int k = chunk_at(p) * 64;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      f.wa[s] = *reinterpret_cast<const u32x4*>(w0 + k + 32 * s);
-      f.wb[s] = *reinterpret_cast<const u32x4*>(w1 + k + 32 * s);
+      f.wa[s] = ld16(w0 + k + 32 * s);
+      f.wb[s] = ld16(w1 + k + 32 * s);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const u32x4* px = reinterpret_cast<const u32x4*>(xw + xoff[s * R + r] + k);
-        if constexpr (!SPLITK && (!TILE || kTileNt))
-          f.xv[s][r] = __builtin_nontemporal_load(px);
+        const uint16_t* px = xw + xoff[s * R + r] + k;
+        if constexpr (WHOLE && !SPLITK && (!TILE || kTileNt))
+          f.xv[s][r] = ld16_stream(px);
         else
-          f.xv[s][r] = *px;
+          f.xv[s][r] = ld16(px);
       }
     }
   };
@@ -373,23 +417,27 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
       compute(f0);
     }
   }
-  // Ragged last chunk (nC % 64 != 0): 16-byte pieces past nC contribute zero.
+  // Ragged last chunk (nC % 64 != 0): columns past nC contribute zero.  A
+  // group that would pass the row's end is loaded as the row's last 8 columns
+  // with those of earlier groups cleared (in W and in x, which then agree on
+  // the columns' places).
   if ((nC & 63) != 0 && last_split && wave == nfull % SPLIT) {
     const int k = nall * 64;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const bool ok = k + 32 * s + 8 * grp < nC;
+      const int kp = k + 32 * s + 8 * grp;
+      const int kb = WHOLE || kp < nC - 8 ? kp : nC - 8;
       f0.wa[s] = f0.wb[s] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
       for (int r = 0; r < R; ++r) f0.xv[s][r] = u32x4{0u, 0u, 0u, 0u};
-      if (ok) {
-        f0.wa[s] = *reinterpret_cast<const u32x4*>(w0 + k + 32 * s);
-        f0.wb[s] = *reinterpret_cast<const u32x4*>(w1 + k + 32 * s);
+      if (kp < nC) {
+        f0.wa[s] = drop_front<WHOLE>(ld16(w0 + (kb - 8 * grp)), kp - kb);
+        f0.wb[s] = drop_front<WHOLE>(ld16(w1 + (kb - 8 * grp)), kp - kb);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           int64_t t = t0 + 16 * r + row;
           t = t < T ? t : T - 1;
-          f0.xv[s][r] = *reinterpret_cast<const u32x4*>(x + t * nC + 8 * grp + k + 32 * s);
+          f0.xv[s][r] = drop_front<WHOLE>(ld16(x + t * nC + kb), kp - kb);
         }
       }
     }
@@ -448,8 +496,8 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
         uint16_t* orow = out + t * kDout + 4 * grp;
         u32x2 lo2 = {pack_bf16x2(a[0] * inv, a[1] * inv), pack_bf16x2(a[2] * inv, a[3] * inv)};
         u32x2 hi2 = {pack_bf16x2(a[4] * inv, a[5] * inv), pack_bf16x2(a[6] * inv, a[7] * inv)};
-        st_stream(reinterpret_cast<u32x2*>(orow), lo2);
-        st_stream(reinterpret_cast<u32x2*>(orow + 16), hi2);
+        st8_stream(orow, lo2);
+        st8_stream(orow + 16, hi2);
         if (grp == 0) inv_rms[t] = inv;
       }
       if constexpr (TILE) {
@@ -485,7 +533,9 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
       if (qd == 0) tile_sm.hpre[16 * r + i] = f32x4{hp_all[0], hp_all[1], hp_all[2], hp_all[3]};
     }
     if (R >= SPLIT && pt.layer_input) {
-      if (pt.C % 4096 == 0) {
+      if (!WHOLE && pt.C <= kNarrowC) {
+        k3_narrow_tokens(x, tile_sm.hpre + 16 * r, pt.layer_input, t0 + 16 * r, T, pt.C, pt.groups16, lane, 0, 1, 16);
+      } else if (WHOLE && pt.C % 4096 == 0) {
         k3_block_pipelined(x, tile_sm.hpre + 16 * r, pt.layer_input, t0 + 16 * r, T, pt.C, lane);
       } else {
         for (int tt = 0; tt < 16; ++tt) {
@@ -493,19 +543,23 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
           if (t >= T) break;
           const f32x4 hv = tile_sm.hpre[16 * r + tt];
           const float h[4] = {hv[0], hv[1], hv[2], hv[3]};
-          k3_token<true>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
+          k3_token<WHOLE>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
         }
       }
     }
     }
     if (R < SPLIT && pt.layer_input) {  // the same branch in every thread
       __syncthreads();
+      if (!WHOLE && pt.C <= kNarrowC) {
+        k3_narrow_tokens(x, tile_sm.hpre, pt.layer_input, t0, T, pt.C, pt.groups16, lane, wave, SPLIT, 16 * R);
+        return;
+      }
       for (int tt = wave; tt < 16 * R; tt += SPLIT) {
         const int64_t t = t0 + tt;
         if (t >= T) break;
         const f32x4 hv = tile_sm.hpre[tt];
         const float h[4] = {hv[0], hv[1], hv[2], hv[3]};
-        k3_token<true>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
+        k3_token<WHOLE>(x + t * 4 * pt.C, h, pt.layer_input + t * pt.C, lane, kWave, pt.C);
       }
     }
   }
@@ -982,9 +1036,8 @@ __global__ __launch_bounds__(256) void k1_dw_scalar(const uint16_t* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Element-wise paths for what the matrix-core paths do not take (forward:
-// nC % 8 != 0 or a base pointer not 16-byte aligned; backward: fewer than 8
-// columns; rows beyond 2^24 / 2^26 columns).  One wave per token; results agree with the matrix-core paths to fp32 summation order.
+// Element-wise paths for what the matrix-core paths do not take: fewer than 8
+// columns, and rows beyond 2^24 / 2^26 columns.  One wave per token; results agree with the matrix-core paths to fp32 summation order.
 __global__ __launch_bounds__(256) void k1_fwd_scalar(const uint16_t* __restrict__ x,
                                                      const uint16_t* __restrict__ W,
                                                      uint16_t* __restrict__ out,
@@ -1133,6 +1186,10 @@ BwdSlices bwd_slices(int64_t nC, int64_t len) {
 // whole row could belong to two of them.
 BwdSlices bwd_premap_slices(int64_t C) { return bwd_slices(4 * C, C % 8 == 0 ? 4 * C : C); }
 
+// The forward MFMA kernel addresses a workgroup's 16 R rows of x with 32-bit
+// element offsets.
+bool k1_fwd_mfma_path(int64_t nC) { return nC >= 8 && nC <= (int64_t{1} << 24); }
+
 // Column split of the forward for T tokens (S = 1: the one-pass kernel).
 struct K1FwdSplit {
   int S = 1, cps = 0;
@@ -1142,7 +1199,7 @@ struct K1FwdSplit {
 K1FwdSplit k1_fwd_split(int64_t T, int64_t nC) {
   K1FwdSplit p;
   const int64_t nall = nC >> 6;
-  if (T <= 0 || nC % 8 != 0 || nC > (int64_t{1} << 24) || nall < 2) return p;
+  if (T <= 0 || !k1_fwd_mfma_path(nC) || nall < 2) return p;
   const int64_t nblk = (T + 16 * kSplitR - 1) / (16 * kSplitR);
   int64_t S = (kSplitTarget + nblk - 1) / nblk;
   if (S < (nall <= 64 ? 2 * kSplitMinS : kSplitMinS)) return p;
@@ -1178,14 +1235,14 @@ constexpr int fwd_waves() {
 
 // The one-pass forward with R blocks per workgroup (k1_fwd_blocks); TILE: the
 // pre-map forward on the same tiles.
-template <bool TILE>
+template <bool TILE, bool WHOLE>
 void launch_k1_fwd_onepass(int R, const uint16_t* x, const uint16_t* W, uint16_t* out, float* inv_rms,
                            int64_t T, int nc, const PremapTile& pt, hipStream_t s) {
   const dim3 grid(blocks_for(T, 16 * R));
   auto launch = [&](auto r) {
     constexpr int kR = decltype(r)::value;
     constexpr int kS = fwd_waves<kR>();
-    k1_fwd_mfma<kR, kS, false, TILE><<<grid, kWave * kS, 0, s>>>(x, W, out, inv_rms, nullptr, T, nc, 0, pt);
+    k1_fwd_mfma<kR, kS, false, TILE, WHOLE><<<grid, kWave * kS, 0, s>>>(x, W, out, inv_rms, nullptr, T, nc, 0, pt);
   };
   switch (R) {
     case 1: launch(std::integral_constant<int, 1>{}); break;
@@ -1195,26 +1252,36 @@ void launch_k1_fwd_onepass(int R, const uint16_t* x, const uint16_t* W, uint16_t
   }
 }
 
+// The column-split forward's first kernel.
+int launch_k1_fwd_split(const K1FwdSplit& p, const uint16_t* x, const uint16_t* W, float* part, int64_t T, int nc,
+                        hipStream_t s) {
+  const dim3 grid(blocks_for(T, 16 * kSplitR), p.S);
+  if (nc % 8 == 0)
+    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, true><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr, part,
+                                                                                       T, nc, p.cps);
+  else
+    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, false><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr,
+                                                                                        part, T, nc, p.cps);
+  return launch_status();
+}
+
 // K1 forward; with a workspace of k1_fwd_split(T, nC).bytes (allow_split) few
 // tokens take the column-split kernel.
 int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* inv_rms, void* ws,
                int64_t ws_bytes, bool allow_split, int64_t T, int64_t nC, hipStream_t s) {
   const int nc = static_cast<int>(nC);
-  // The MFMA kernel addresses a workgroup's 16 R rows of x with 32-bit
-  // element offsets.
-  if (nC % 8 == 0 && nC <= (int64_t{1} << 24) && aligned16(x_flat) && aligned16(W) && aligned16(out)) {
+  if (k1_fwd_mfma_path(nC)) {
     const K1FwdSplit p = allow_split ? k1_fwd_split(T, nC) : K1FwdSplit{};
     if (p.S > 1) {
       if (!ws || ws_bytes < p.bytes || !aligned16(ws)) return FMHC_ERR_INVALID_ARGUMENT;
       float* part = static_cast<float*>(ws);
-      const dim3 grid(blocks_for(T, 16 * kSplitR), p.S);
-      k1_fwd_mfma<kSplitR, kFwdSplit, true><<<grid, kWave * kFwdSplit, 0, s>>>(x_flat, W, out, inv_rms, part,
-                                                                              T, nc, p.cps);
-      const int st = launch_status();
+      const int st = launch_k1_fwd_split(p, x_flat, W, part, T, nc, s);
       if (st != FMHC_OK) return st;
       k1_fwd_finish<<<dim3(blocks_for(T, 4)), 256, 0, s>>>(part, out, inv_rms, T, nc, p.S);
+    } else if (nC % 64 == 0 && aligned16(x_flat)) {
+      launch_k1_fwd_onepass<false, true>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     } else {
-      launch_k1_fwd_onepass<false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
+      launch_k1_fwd_onepass<false, false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     }
   } else {
     const dim3 grid(blocks_for(T, 4));
@@ -1390,24 +1457,23 @@ bool k1_premap_tile(const uint16_t* x, const uint16_t* W, uint16_t* proj, float*
   const int64_t nC = 4 * C;
   // Where K1's column split is planned (few tokens) the pre-map forward takes
   // it and its second stage fused with K2 and K3 (premap.hip) instead.
-  if (T <= 0 || k1_fwd_split(T, nC).S > 1 || C % 8 != 0 || nC > (int64_t{1} << 24) || !aligned16(x) || !aligned16(W) ||
-      !aligned16(proj) || (pt.layer_input && !aligned16(pt.layer_input)))
-    return false;
-  launch_k1_fwd_onepass<true>(k1_fwd_blocks(T), x, W, proj, inv_rms, T, static_cast<int>(nC), pt, s);
+  if (T <= 0 || !k1_fwd_mfma_path(nC) || k1_fwd_split(T, nC).S > 1) return false;
+  PremapTile p = pt;
+  p.groups16 = C % 8 == 0 && aligned16(x) && (!pt.layer_input || aligned16(pt.layer_input));
+  if (p.groups16 && C > kNarrowC)
+    launch_k1_fwd_onepass<true, true>(k1_fwd_blocks(T), x, W, proj, inv_rms, T, static_cast<int>(nC), p, s);
+  else
+    launch_k1_fwd_onepass<true, false>(k1_fwd_blocks(T), x, W, proj, inv_rms, T, static_cast<int>(nC), p, s);
   *status = launch_status();
   return true;
 }
 
 int k1_fwd_partials(const uint16_t* x_flat, const uint16_t* W, void* ws, int64_t ws_bytes, int64_t T,
                     int64_t nC, hipStream_t s) {
-  if (!(nC % 8 == 0 && nC <= (int64_t{1} << 24) && aligned16(x_flat) && aligned16(W))) return 0;
   const K1FwdSplit p = k1_fwd_split(T, nC);
   if (p.S < 2) return 0;
   if (!ws || ws_bytes < p.bytes || !aligned16(ws)) return -FMHC_ERR_INVALID_ARGUMENT;
-  const dim3 grid(blocks_for(T, 16 * kSplitR), p.S);
-  k1_fwd_mfma<kSplitR, kFwdSplit, true><<<grid, kWave * kFwdSplit, 0, s>>>(
-      x_flat, W, nullptr, nullptr, static_cast<float*>(ws), T, static_cast<int>(nC), p.cps);
-  const int st = launch_status();
+  const int st = launch_k1_fwd_split(p, x_flat, W, static_cast<float*>(ws), T, static_cast<int>(nC), s);
   return st == FMHC_OK ? p.S : -st;
 }
 

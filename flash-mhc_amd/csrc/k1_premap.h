@@ -26,12 +26,12 @@ struct PremapTile {
   float* H = nullptr;
   uint16_t* layer_input = nullptr;
   int C = 0;
+  bool groups16 = false;  // K3's rows are whole, aligned 16-byte groups
   ZeroWords z{};
 };
 
-// The pre-map forward as one kernel, when T takes K1's one-pass forward (no
-// column split planned) and the shapes allow (C % 8 == 0, 16-byte aligned x /
-// W / proj / layer_input): K1 on tiles of 16 to 64 tokens, then K2 and K3 on
+// The pre-map forward as one kernel, when T takes K1's one-pass forward on the
+// matrix cores (no column split planned): K1 on tiles of 16 to 64 tokens, then K2 and K3 on
 // each tile by the same workgroup.  Returns false (nothing launched) when
 // they do not; otherwise launches and returns true with *status set.
 bool k1_premap_tile(const uint16_t* x, const uint16_t* W, uint16_t* proj, float* inv_rms, const PremapTile& pt,

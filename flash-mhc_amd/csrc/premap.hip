@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2(
 // reading the stored h_pre).  Saves K3's launch for few tokens.  Up to
 // C = 4096 (two 16-byte groups per lane) every lane loads its x vectors
 // before K1's partial sums and K2's chain run, so their latency overlaps.
-template <int VEC>
+template <bool WHOLE>
 __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
     const float* __restrict__ part, int S, int nC, const K2Params P, uint16_t* __restrict__ proj,
     float* __restrict__ inv_rms, float* __restrict__ h_pre, float* __restrict__ h_post, float* __restrict__ H,
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
   const int lane = static_cast<int>(threadIdx.x);
   const uint16_t* x0 = x + t * 4 * C;
   const int ng = C / 8;
-  const bool pre = VEC == 8 && ng <= kPre * kFinishThreads;
+  const bool pre = ng <= kPre * kFinishThreads;
   u32x4 xv[kPre][4];
   if (pre) {
 #pragma unroll
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         xv[it][j] = u32x4{0u, 0u, 0u, 0u};
-        if (g < ng) xv[it][j] = ld_stream(reinterpret_cast<const u32x4*>(x0 + j * C) + g);
+        if (g < ng) xv[it][j] = Lanes<8, WHOLE>::raw(x0 + j * C, g);
       }
     }
   }
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
   __syncthreads();
   const float h[4] = {hsh[0], hsh[1], hsh[2], hsh[3]};
   if (!pre) {
-    k3_token<VEC == 8>(x0, h, layer_input + t * C, lane, kFinishThreads, C);
+    k3_token<WHOLE>(x0, h, layer_input + t * C, lane, kFinishThreads, C);
     return;
   }
 #pragma unroll
@@ -188,9 +188,10 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
         acc = __builtin_fmaf(h[2], c[e], acc);
         o[e] = __builtin_fmaf(h[3], d[e], acc);
       }
-      Lanes<8, true>::store(layer_input + t * C, g, o);
+      Lanes<8, WHOLE>::store(layer_input + t * C, g, o);
     }
   }
+  row_tail<WHOLE>(C, lane, [&](int c) { k3_mix<1, WHOLE>(x0, h, layer_input + t * C, c, C); });
 }
 
 // Backward, few tokens (T <= kK2BwdSmallT) for rows of 17 to 255 groups of 8
@@ -353,11 +354,11 @@ int premap_fwd_run(const uint16_t* x, const uint16_t* W, const void* alpha_pre, 
     const dim3 grid(static_cast<unsigned>(T));
     const int c = static_cast<int>(C);
     if (C % 8 == 0 && aligned16(x) && aligned16(layer_input))
-      k1_finish_k2_k3<8><<<grid, kFinishThreads, 0, s>>>(part, S, nc, P, proj, inv_rms, h_pre, h_post, H_merged,
-                                                          z, x, layer_input, c);
+      k1_finish_k2_k3<true><<<grid, kFinishThreads, 0, s>>>(part, S, nc, P, proj, inv_rms, h_pre, h_post, H_merged,
+                                                            z, x, layer_input, c);
     else
-      k1_finish_k2_k3<1><<<grid, kFinishThreads, 0, s>>>(part, S, nc, P, proj, inv_rms, h_pre, h_post, H_merged,
-                                                          z, x, layer_input, c);
+      k1_finish_k2_k3<false><<<grid, kFinishThreads, 0, s>>>(part, S, nc, P, proj, inv_rms, h_pre, h_post, H_merged,
+                                                             z, x, layer_input, c);
     return fmhc::launch_status();
   }
   if (S >= 2) {

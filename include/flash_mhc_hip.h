@@ -19,10 +19,9 @@
  *     32, matching the reference's n = 4 specialisation.
  *   - bf16 pointers need 2-byte alignment, fp32 pointers 4-byte, unless an
  *     entry point asks for more.  Any C is taken; lanes move 16 bytes each,
- *     and the last columns of rows with C % 8 != 0 one element each.  K1's
- *     forward for nC % 8 != 0 or operands off 16-byte alignment, and its
- *     backward for fewer than 8 columns, run element-wise, with the same
- *     values up to the order of fp32 sums.
+ *     and the last columns of rows with C % 8 != 0 one element each.  K1 for
+ *     fewer than 8 columns runs element-wise, with the same values up to the
+ *     order of fp32 sums.
  *   - Return value: FMHC_OK (0), or an FMHC_ERR_* code; for HIP runtime
  *     failures FMHC_ERR_HIP_BASE + hipError_t.  fmhc_error_string() names it.
  */

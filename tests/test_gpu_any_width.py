@@ -13,7 +13,7 @@ import torch
 from flash_mhc import build_permutation_matrices
 from flash_mhc import kernels as K
 from oracle import mhc_oracle as O
-from parity import check_bf16, check_fp32
+from parity import check_bf16, check_fp32, check_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -46,6 +46,41 @@ def _params(C):
     g = torch.Generator().manual_seed(C)
     return [t.to(DEV) for t in (torch.tensor([0.8]), torch.tensor([1.2]), torch.tensor([1.7]),
                                 torch.randn(32, generator=g) * 0.5, build_permutation_matrices(4)[0])]
+
+
+# The forward's tiles of 16, 32, 48 and 64 tokens (from T = 4097, 8193, 12289),
+# its column split (up to 2720 tokens, nC of two chunks and more) and its last
+# chunk of 1 to 63 columns: C = 2 and 3 (one group, rows of 8 and 12 columns),
+# 15 ... 17 around one 64-column chunk.
+FWD = [*SHAPES, (5, 2), (40, 3), (4096, 16), (2721, 129), (5000, 131), (9000, 33), (12300, 25), (20011, 300),
+       (2720, 4099), (3, 4103)]
+
+
+@pytest.mark.parametrize("off", [0, 1, 3])
+@pytest.mark.parametrize("T,C", FWD)
+def test_k1_fwd(T, C, off):
+    nC = 4 * C
+    rn, x, W = _inputs(T, C, off, 7 * T + C + off)
+    proj, inv = K.k1_fwd(x.view(T, nC), W, out=_at(torch.zeros(T, 32, dtype=BF16), off))
+    i = torch.cat([torch.arange(min(T, 80)), torch.arange(max(0, T - 80), T)]).unique()
+    xs = x.view(T, nC)[i.to(DEV)].cpu()
+    R, S, invR = O.k1_fwd(xs, W.cpu())
+    check_bf16("proj", proj[i.to(DEV)], R, S, nC)
+    check_rel("inv_rms", inv[i.to(DEV)], invR, rtol=4 * nC ** 0.5 * 2.0**-24 + 4 * 2.0**-24)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("T,C", FWD)
+def test_premap_fwd(T, C, off):
+    nC = 4 * C
+    rn, x, W = _inputs(T, C, off, 5 * T + C + off)
+    p = _params(C)
+    li, H, hq, hp, proj, inv = K.premap_fwd(x, W, *p)
+    proj1, inv1 = K.k1_fwd(x.view(T, nC), W)
+    hp1, hq1, H1 = K.k2_fwd(proj1, *p)
+    want = (K.k3_fwd(x, hp1), H1, hq1, hp1, proj1, inv1)
+    for name, u, v in zip(("layer_input", "H", "h_post", "h_pre", "proj", "inv_rms"), (li, H, hq, hp, proj, inv), want):
+        assert torch.equal(u, v), name
 
 
 @pytest.mark.parametrize("off", [0, 1, 3])
