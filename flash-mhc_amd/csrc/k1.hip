@@ -968,6 +968,14 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
 // Workgroups from dw_blocks on sum K2's parameter gradients instead, one
 // workgroup per parameter (the pre-map backward; one launch fewer than K2's
 // own reduce).
+// SPLIT: the four waves of a workgroup take the same elements and a quarter of
+// the runs each, added in wave order.  For up to kReduceSplitSlices slices,
+// whose elements alone leave CUs without a workgroup while every thread walks
+// hundreds of runs one load latency after the other: pre-map backward at
+// T = 65536, C = 64 87.4 -> 62.5 us, 100 91 -> 78, 256 131 -> 127.5; T = 8192,
+// C = 512 51 -> 48.7.  With more slices it loses 1% (C = 1024, 2560).
+constexpr int kReduceSplitSlices = 16;
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ partial,
                                                     uint16_t* __restrict__ dW, int64_t nparts,
                                                     const BwdSlices sl, int nC, unsigned dw_blocks,
@@ -977,13 +985,17 @@ __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ pa
     return;
   }
   const int64_t per_part = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave);
-  const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
-  if (i0 >= per_part) return;
+  constexpr int kVecs = SPLIT ? kWave : 256;  // 16-byte vectors per workgroup
+  const int wave = SPLIT ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6) : 0;
+  const int lane = static_cast<int>(threadIdx.x) & (kVecs - 1);
+  // Below per_part, which is a multiple of 8192.
+  const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * kVecs + lane) * 4;
   const f32x4* src = reinterpret_cast<const f32x4*>(partial + i0);
   const int64_t stride = per_part / 4;  // in 16-byte vectors
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  int64_t p = 0;
-  for (; p + 4 <= nparts; p += 4) {
+  int64_t p = SPLIT ? nparts * wave / 4 : 0;
+  const int64_t end = SPLIT ? nparts * (wave + 1) / 4 : nparts;
+  for (; p + 4 <= end; p += 4) {
     const f32x4 v0 = src[(p + 0) * stride], v1 = src[(p + 1) * stride];
     const f32x4 v2 = src[(p + 2) * stride], v3 = src[(p + 3) * stride];
     acc += v0;
@@ -991,7 +1003,15 @@ __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ pa
     acc += v2;
     acc += v3;
   }
-  for (; p < nparts; ++p) acc += src[p * stride];
+  for (; p < end; ++p) acc += src[p * stride];
+  if constexpr (SPLIT) {
+    __shared__ f32x4 quarter[4][kWave];
+    quarter[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) acc += quarter[w][lane];
+  }
   const int lane0 = static_cast<int>(i0 % kWave);  // multiple of 4
   const int rr = static_cast<int>((i0 / kWave) % 4);
   const int h = static_cast<int>((i0 / (4 * kWave)) % 2);
@@ -1402,6 +1422,22 @@ int64_t k1_bwd_runs(int64_t T, int64_t nslices) {
   return r < nblocks ? r : nblocks;
 }
 
+// grad_W from its partial sums; k2_params workgroups more sum K2's parameter
+// gradients.
+int launch_dw_reduce(const float* partial, uint16_t* grad_W, int64_t nruns, const BwdSlices& sl, int nC,
+                     const K2ParamSums& sums, int k2_params, hipStream_t s) {
+  static_assert(kK2SumThreads == 256, "K2's parameter sums share the reduce's workgroups");
+  const int64_t vecs = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave) / 4;
+  if (sl.n <= kReduceSplitSlices) {
+    const unsigned nb = blocks_for(vecs, kWave);
+    k1_dw_reduce<true><<<dim3(nb + k2_params), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
+  } else {
+    const unsigned nb = blocks_for(vecs, 256);
+    k1_dw_reduce<false><<<dim3(nb + k2_params), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
+  }
+  return launch_status();
+}
+
 // Bytes of grad_W's partial sums.
 int64_t k1_bwd_dw_bytes(int64_t T, const BwdSlices& sl) {
   return k1_bwd_runs(T, sl.n) * sl.n * (8 * 2 * 4 * kWave) * static_cast<int64_t>(sizeof(float));
@@ -1438,10 +1474,7 @@ extern "C" int fmhc_k1_bwd(const uint16_t* x_flat, const uint16_t* W, const uint
     launch_k1_bwd_mfma<true>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, partial, T, nc, sl, nruns);
     const int st = launch_status();
     if (st != FMHC_OK) return st;
-    const int64_t per_part = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave);
-    const unsigned nb = blocks_for(per_part / 4, 256);
-    k1_dw_reduce<<<dim3(nb), 256, 0, s>>>(partial, grad_W, nruns, sl, nc, nb, K2ParamSums{});
-    return launch_status();
+    return launch_dw_reduce(partial, grad_W, nruns, sl, nc, K2ParamSums{}, 0, s);
   }
   const int st = fmhc_k1_bwd_dx(x_flat, W, grad_out, proj_out, inv_rms, grad_x, T, nC, D_out, stream);
   if (st != FMHC_OK) return st;
@@ -1479,20 +1512,9 @@ int k1_fwd_partials(const uint16_t* x_flat, const uint16_t* W, void* ws, int64_t
 
 int64_t k1_bwd_dw_runs(int64_t T, int64_t nC) { return k1_bwd_runs(T, (nC + 127) / 128); }
 
-namespace {
-int dw_finish(const float* partial, uint16_t* grad_W, int64_t nruns, const BwdSlices& sl, int nC,
-              const K2ParamSums& sums, hipStream_t s) {
-  const int64_t per_part = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave);
-  const unsigned nb = blocks_for(per_part / 4, 256);
-  static_assert(kK2SumThreads == 256, "K2's parameter sums share the reduce's workgroups");
-  k1_dw_reduce<<<dim3(nb + kNPar), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
-  return launch_status();
-}
-}  // namespace
-
 int k1_dw_finish(const float* partial, uint16_t* grad_W, int64_t nruns, int nC, const K2ParamSums& sums,
                  hipStream_t s) {
-  return dw_finish(partial, grad_W, nruns, bwd_slices(nC, nC), nC, sums, s);
+  return launch_dw_reduce(partial, grad_W, nruns, bwd_slices(nC, nC), nC, sums, kNPar, s);
 }
 
 // K1 backward of the pre-map region (premap.hip): grad_W as fmhc_k1_bwd and
@@ -1530,7 +1552,7 @@ int k1_bwd_premap(const uint16_t* x_flat, const uint16_t* W, const uint16_t* gra
                                      go3, h_pre, static_cast<int>(C));
     const int st = launch_status();
     if (st != FMHC_OK) return st;
-    return dw_finish(partial, grad_W, nruns, sl, nc, k2_sums, s);
+    return launch_dw_reduce(partial, grad_W, nruns, sl, nc, k2_sums, kNPar, s);
   }
   k1_bwd_scalar<true><<<dim3(blocks_for(T, 4)), 256, 0, s>>>(x_flat, W, grad_proj, proj, inv_rms, grad_x,
                                                              grad_x_in, T, nc);
