@@ -90,6 +90,21 @@ __device__ __forceinline__ void st8_stream(void* p, u32x2 v) {
 #endif
 }
 
+// Loads carry the hint in launches that read more than fits the memory-side
+// cache (256 MB) along with what the launch before it wrote and read.  Below
+// that, x and its gradients are read again by the next kernel of a step, and
+// lines loaded under the hint are not kept for it: ordinary loads win where an
+// earlier launch touched the operands, and lose 2-5% where none did, from HBM.
+// Stores keep the hint at every size (without it T = 1024, C = 1024 K4 backward
+// 8.0 -> 8.9 us, K4 forward 4.3 -> 5.1).  With the hint against
+// without, three sets of operands in turn, us: T = 1003, C = 2560 K1 backward
+// 24.1 / 19.1, K3 forward 6.2 / 5.9, K4 forward 9.5 / 8.9; T = 4096, C = 1024
+// K1 backward 25.9 / 20.4; T = 8192, C = 1024 K1 forward 18.5 / 13.8, K3 backward 26.2 / 23.9, K4 forward 25.4 / 23.5; past
+// the line, T = 16384, C = 1024 K1 forward 25.1 / 26.9, K3 backward 49.2 /
+// 51.7, K4 forward 47.9 / 51.7.
+constexpr int64_t kCachedReadBytes = int64_t{80} << 20;
+inline bool stream_reads(int64_t bytes) { return bytes > kCachedReadBytes; }
+
 // bf16 bit pattern -> fp32 (exact).
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
@@ -174,7 +189,9 @@ __device__ __forceinline__ void row_tail(int C, int first, F&& f) {
 // h1 x1[c] + h2 x2[c] + h3 x3[c]), the products added in stream order with
 // fused multiply-adds.  Shared by the K3 kernel and the pre-map's kernels,
 // which must agree bit for bit.
-template <int VEC, bool NT>
+// NT: x with the nontemporal hint; WHOLE: the output with it (rows of whole,
+// aligned groups), and rows have no tail.
+template <int VEC, bool WHOLE, bool NT = WHOLE>
 __device__ __forceinline__ void k3_mix(const uint16_t* __restrict__ x0, const float h[4], uint16_t* __restrict__ orow,
                                        int g, int C) {
   const uint16_t* x1 = x0 + C;
@@ -192,17 +209,17 @@ __device__ __forceinline__ void k3_mix(const uint16_t* __restrict__ x0, const fl
     acc = __builtin_fmaf(h[2], c[e], acc);
     o[e] = __builtin_fmaf(h[3], d[e], acc);
   }
-  Lanes<VEC, NT>::store(orow, g, o);
+  Lanes<VEC, WHOLE>::store(orow, g, o);
 }
 
 // A whole token: groups first, first + step, ... below C / 8, then the tail.
-template <bool NT>
+template <bool WHOLE, bool NT = WHOLE>
 __device__ __forceinline__ void k3_token(const uint16_t* __restrict__ x0, const float h[4],
                                          uint16_t* __restrict__ orow, int first, int step, int C) {
   const int ng = C / 8;
 #pragma unroll 2
-  for (int g = first; g < ng; g += step) k3_mix<8, NT>(x0, h, orow, g, C);
-  row_tail<NT>(C, first, [&](int c) { k3_mix<1, NT>(x0, h, orow, c, C); });
+  for (int g = first; g < ng; g += step) k3_mix<8, WHOLE, NT>(x0, h, orow, g, C);
+  row_tail<WHOLE>(C, first, [&](int c) { k3_mix<1, WHOLE, NT>(x0, h, orow, c, C); });
 }
 
 // Residency caps.  K3's and K4's kernels use a few dozen VGPRs, so eight
@@ -410,16 +427,19 @@ constexpr int block_of() {
 inline int64_t tokens_per_block(int lpt) { return kBlock % lpt == 0 ? kBlock / lpt : 1; }
 
 // How K3 and K4 walk a row, as compile-time constants: LPT lanes per token,
-// LOOP: several groups per lane, NT: whole, aligned groups, accessed with the
-// nontemporal hint.
-template <int kLpt, bool kLoop, bool kNt>
+// LOOP: several groups per lane, WHOLE: whole, aligned groups, stored with the
+// nontemporal hint, NT: also loaded with it.
+template <int kLpt, bool kLoop, bool kWhole, bool kNt>
 struct RowWalk {
   static constexpr int LPT = kLpt;
   static constexpr bool LOOP = kLoop;
+  static constexpr bool WHOLE = kWhole;
   static constexpr bool NT = kNt;
+  static_assert(WHOLE || !NT, "unaligned groups are loaded without the hint");
 };
 
-// f(RowWalk) for rows of C columns whose 16-byte groups are aligned or not.
+// f(RowWalk) for rows of C columns whose 16-byte groups are aligned or not, in
+// a launch that reads `reads` bytes (stream_reads).
 // Unaligned groups (C % 8 != 0, or a base address off 16 bytes) leave out the
 // nontemporal hint: neighbouring lanes' groups share lines, and the hint
 // makes each access fetch or write its part on its own (K3 forward / backward,
@@ -427,28 +447,30 @@ struct RowWalk {
 // 17.5 / 32.0 / 32.5 / 53.4 against 11.8 / 24.0 / 24.7 / 45.1; T = 20011,
 // C = 300 14.3 / 24.0 / 23.8 / 42.5 against 12.1 / 19.3 / 19.9 / 38.3).
 template <typename F>
-void with_row_walk(int C, bool aligned, F&& f) {
-  auto pick = [&](auto nt) {
-    constexpr bool NT = decltype(nt)::value;
+void with_row_walk(int C, bool aligned, int64_t reads, F&& f) {
+  auto pick = [&](auto whole, auto nt) {
+    constexpr bool WHOLE = decltype(whole)::value, NT = decltype(nt)::value;
     const int lpt = lanes_per_token(C);
-    if (C / 8 > lpt) return f(RowWalk<kLoopLpt, true, NT>{});
+    if (C / 8 > lpt) return f(RowWalk<kLoopLpt, true, WHOLE, NT>{});
     switch (lpt) {
-      case 448: return f(RowWalk<448, false, NT>{});
-      case 384: return f(RowWalk<384, false, NT>{});
-      case 320: return f(RowWalk<320, false, NT>{});
-      case 256: return f(RowWalk<256, false, NT>{});
-      case 192: return f(RowWalk<192, false, NT>{});
-      case 128: return f(RowWalk<128, false, NT>{});
-      case 64: return f(RowWalk<64, false, NT>{});
-      case 32: return f(RowWalk<32, false, NT>{});
-      case 16: return f(RowWalk<16, false, NT>{});
-      default: return f(RowWalk<8, false, NT>{});
+      case 448: return f(RowWalk<448, false, WHOLE, NT>{});
+      case 384: return f(RowWalk<384, false, WHOLE, NT>{});
+      case 320: return f(RowWalk<320, false, WHOLE, NT>{});
+      case 256: return f(RowWalk<256, false, WHOLE, NT>{});
+      case 192: return f(RowWalk<192, false, WHOLE, NT>{});
+      case 128: return f(RowWalk<128, false, WHOLE, NT>{});
+      case 64: return f(RowWalk<64, false, WHOLE, NT>{});
+      case 32: return f(RowWalk<32, false, WHOLE, NT>{});
+      case 16: return f(RowWalk<16, false, WHOLE, NT>{});
+      default: return f(RowWalk<8, false, WHOLE, NT>{});
     }
   };
-  if (aligned && C % 8 == 0)
-    pick(std::true_type{});
+  if (!aligned || C % 8 != 0)
+    pick(std::false_type{}, std::false_type{});
+  else if (stream_reads(reads))
+    pick(std::true_type{}, std::true_type{});
   else
-    pick(std::false_type{});
+    pick(std::true_type{}, std::false_type{});
 }
 
 // Token of a lane.  LPT <= 64: 64 / LPT tokens per wave; wider: LPT / 64 waves

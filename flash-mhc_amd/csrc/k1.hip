@@ -201,6 +201,7 @@ __device__ __forceinline__ void k3_narrow_tokens(const uint16_t* __restrict__ x,
 // streams into the layer input while L2 and the memory-side cache may still
 // hold the rows it just read (its x loads are ordinary loads, which allocate
 // there).  Same values as K1 -> K2 -> K3 launched separately.
+// NT: x's loads carry the nontemporal hint (plain kernel, stream_reads).
 // WHOLE: rows of whole 128-byte lines (the plain kernel), of whole aligned
 // 16-byte groups and more than kNarrowC columns (TILE), or of whole groups
 // (SPLITK); otherwise x is loaded without the nontemporal hint, the last group
@@ -212,7 +213,7 @@ __device__ __forceinline__ void k3_narrow_tokens(const uint16_t* __restrict__ x,
 // C = 77 18.2 -> 3.8, and with K2 and K3 on each tile (pre-map forward)
 // 2246 -> 125 and 24.6 -> 6.5 us, T = 20011, C = 300 42 -> 32, T = 65536,
 // C = 100 43 -> 28; x off 16 bytes at T = 8192, C = 1024 781 -> 52.
-template <int R, int SPLIT, bool SPLITK, bool TILE, bool WHOLE>
+template <int R, int SPLIT, bool SPLITK, bool TILE, bool WHOLE, bool NT>
 __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __restrict__ x,
                                                              const uint16_t* __restrict__ W,
                                                              uint16_t* __restrict__ out,
@@ -274,9 +275,9 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
   // concurrent reads of all workgroups over the DRAM channels instead of every
   // workgroup hitting the same column of its 8 KiB-strided rows), and keeps
   // three chunks in flight: the next two chunks' fragments are loaded while
-  // the MFMAs of the current one run.  x is read once per launch, so its loads carry the
-  // nontemporal hint (8-10% faster than ordinary loads).  With SPLITK (few
-  // tokens) they do not: the pre-map's few-token kernel reads the same x
+  // the MFMAs of the current one run.  x is read once per launch; NT: its loads carry
+  // the nontemporal hint (launches past kCachedReadBytes, 8-10% faster there than
+  // ordinary loads).  With SPLITK (few tokens) they do not: the pre-map's few-token kernel reads the same x
   // again right after, from the caches.  With SPLITK the workgroup's chunks
   // are cbeg .. cbeg + nfull - 1 (no rotation: the workgroups of one token
   // block already cover different columns), and only the last split takes the
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const uint16_t* px = xw + xoff[s * R + r] + k;
-        if constexpr (WHOLE && !SPLITK && (!TILE || kTileNt))
+        if constexpr (NT)
           f.xv[s][r] = ld16_stream(px);
         else
           f.xv[s][r] = ld16(px);
@@ -659,7 +660,7 @@ struct BwdFrag {
 // operand takes the kernel to one wave per SIMD; it is still bound by HBM
 // (measured: +80 us at T=65536, C=1024 for the 512 MiB it reads, against
 // 260 us for the separate accumulation pass it replaces).
-template <bool DW, bool FULLK, bool EPI, bool GI, int NBUF>
+template <bool DW, bool FULLK, bool EPI, bool GI, bool NT, int NBUF>
 __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ x,
                                                    const uint16_t* __restrict__ W,
                                                    const uint16_t* __restrict__ go,
@@ -784,7 +785,7 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
       const int r0 = 4 * grp + q;
       const uint32_t r = static_cast<uint32_t>(r0 < last ? r0 : last);
       if (last != 15) f.inv[q] = *reinterpret_cast<const float*>(ib + 4u * r);
-      f.xv[q] = ld16_stream(xb + (r * row_bytes + kbytes));
+      f.xv[q] = Lanes<8, NT>::raw(reinterpret_cast<const uint16_t*>(xb + (r * row_bytes + kbytes)), 0);
       if constexpr (EPI) {
         const char* g3b = reinterpret_cast<const char*>(go3 + tbase * C);
         f.hp[q] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(h_pre + tbase * 4) + 16u * r +
@@ -794,7 +795,8 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
         f.g3[q] = ld16(g3b + (r * 2u * static_cast<uint32_t>(C) + c3bytes));
       }
       if constexpr (GI)
-        f.gi[q] = ld16_stream(reinterpret_cast<const char*>(gi + tbase * nC) + (r * row_bytes + kbytes));
+        f.gi[q] = Lanes<8, NT>::raw(
+            reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(gi + tbase * nC) + (r * row_bytes + kbytes)), 0);
     }
   };
   auto compute = [&](const BwdFrag<EPI, GI>& f, int tb) {
@@ -1255,14 +1257,14 @@ constexpr int fwd_waves() {
 
 // The one-pass forward with R blocks per workgroup (k1_fwd_blocks); TILE: the
 // pre-map forward on the same tiles.
-template <bool TILE, bool WHOLE>
+template <bool TILE, bool WHOLE, bool NT>
 void launch_k1_fwd_onepass(int R, const uint16_t* x, const uint16_t* W, uint16_t* out, float* inv_rms,
                            int64_t T, int nc, const PremapTile& pt, hipStream_t s) {
   const dim3 grid(blocks_for(T, 16 * R));
   auto launch = [&](auto r) {
     constexpr int kR = decltype(r)::value;
     constexpr int kS = fwd_waves<kR>();
-    k1_fwd_mfma<kR, kS, false, TILE, WHOLE><<<grid, kWave * kS, 0, s>>>(x, W, out, inv_rms, nullptr, T, nc, 0, pt);
+    k1_fwd_mfma<kR, kS, false, TILE, WHOLE, NT><<<grid, kWave * kS, 0, s>>>(x, W, out, inv_rms, nullptr, T, nc, 0, pt);
   };
   switch (R) {
     case 1: launch(std::integral_constant<int, 1>{}); break;
@@ -1277,10 +1279,10 @@ int launch_k1_fwd_split(const K1FwdSplit& p, const uint16_t* x, const uint16_t* 
                         hipStream_t s) {
   const dim3 grid(blocks_for(T, 16 * kSplitR), p.S);
   if (nc % 8 == 0)
-    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, true><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr, part,
+    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, true, false><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr, part,
                                                                                        T, nc, p.cps);
   else
-    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, false><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr,
+    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, false, false><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr,
                                                                                         part, T, nc, p.cps);
   return launch_status();
 }
@@ -1298,10 +1300,12 @@ int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* 
       const int st = launch_k1_fwd_split(p, x_flat, W, part, T, nc, s);
       if (st != FMHC_OK) return st;
       k1_fwd_finish<<<dim3(blocks_for(T, 4)), 256, 0, s>>>(part, out, inv_rms, T, nc, p.S);
+    } else if (nC % 64 == 0 && aligned16(x_flat) && stream_reads(2 * T * nC)) {
+      launch_k1_fwd_onepass<false, true, true>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     } else if (nC % 64 == 0 && aligned16(x_flat)) {
-      launch_k1_fwd_onepass<false, true>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
+      launch_k1_fwd_onepass<false, true, false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     } else {
-      launch_k1_fwd_onepass<false, false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
+      launch_k1_fwd_onepass<false, false, false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     }
   } else {
     const dim3 grid(blocks_for(T, 4));
@@ -1344,16 +1348,30 @@ void launch_k1_bwd_mfma(hipStream_t s, const uint16_t* x, const uint16_t* W, con
   // slower (T = 65536 and 262144).  With grad_W it changed nothing
   // (202.7-203.1 against 201.8-203.3 us at T = 65536, C = 1024).
   const bool cap = !DW && !EPI && FMHC_LDS_CAP && nC <= 4 * 2560;
+  auto launch = [&](auto fullk, auto nt) {
+    constexpr bool FULLK = decltype(fullk)::value, NT = decltype(nt)::value;
+    static const unsigned lds =
+        lds_reserve(reinterpret_cast<const void*>(&k1_bwd_mfma<DW, FULLK, EPI, GI, NT, nbuf>), kLdsCapOne);
+    k1_bwd_mfma<DW, FULLK, EPI, GI, NT, nbuf><<<grid, 256, cap ? lds : 0u, s>>>(
+        x, W, go, proj, inv_rms, gx, partial, go3, h_pre, gi, T, nC, sl, nruns, C);
+  };
+  // x, the incoming gradient and the layer input's gradient (stream_reads).
+  // With grad_W alone, rows off 128-byte lines also take the ordinary loads at
+  // any size: lines that two runs' rows share are then fetched once (T =
+  // 32768, C = 1023 155 -> 143 us, T = 50000, C = 2049 483 -> 444); dx alone
+  // there is equal, and the pre-map's kernel loses 2% (T = 30011, C = 1001).
+  const bool lines = nC % 64 == 0 && aligned16(x);
+  const bool nt = stream_reads(T * nC * (GI ? 4 : 2) + (EPI ? T * C * 2 : 0)) && (lines || !DW || EPI);
   if (sl.len % 128 == 0) {
-    static const unsigned lds =
-        lds_reserve(reinterpret_cast<const void*>(&k1_bwd_mfma<DW, true, EPI, GI, nbuf>), kLdsCapOne);
-    k1_bwd_mfma<DW, true, EPI, GI, nbuf><<<grid, 256, cap ? lds : 0u, s>>>(x, W, go, proj, inv_rms, gx, partial,
-                                                                          go3, h_pre, gi, T, nC, sl, nruns, C);
+    if (nt)
+      launch(std::true_type{}, std::true_type{});
+    else
+      launch(std::true_type{}, std::false_type{});
   } else {
-    static const unsigned lds =
-        lds_reserve(reinterpret_cast<const void*>(&k1_bwd_mfma<DW, false, EPI, GI, nbuf>), kLdsCapOne);
-    k1_bwd_mfma<DW, false, EPI, GI, nbuf><<<grid, 256, cap ? lds : 0u, s>>>(x, W, go, proj, inv_rms, gx, partial,
-                                                                           go3, h_pre, gi, T, nC, sl, nruns, C);
+    if (nt)
+      launch(std::false_type{}, std::true_type{});
+    else
+      launch(std::false_type{}, std::false_type{});
   }
 }
 
@@ -1494,9 +1512,9 @@ bool k1_premap_tile(const uint16_t* x, const uint16_t* W, uint16_t* proj, float*
   PremapTile p = pt;
   p.groups16 = C % 8 == 0 && aligned16(x) && (!pt.layer_input || aligned16(pt.layer_input));
   if (p.groups16 && C > kNarrowC)
-    launch_k1_fwd_onepass<true, true>(k1_fwd_blocks(T), x, W, proj, inv_rms, T, static_cast<int>(nC), p, s);
+    launch_k1_fwd_onepass<true, true, kTileNt>(k1_fwd_blocks(T), x, W, proj, inv_rms, T, static_cast<int>(nC), p, s);
   else
-    launch_k1_fwd_onepass<true, false>(k1_fwd_blocks(T), x, W, proj, inv_rms, T, static_cast<int>(nC), p, s);
+    launch_k1_fwd_onepass<true, false, false>(k1_fwd_blocks(T), x, W, proj, inv_rms, T, static_cast<int>(nC), p, s);
   *status = launch_status();
   return true;
 }

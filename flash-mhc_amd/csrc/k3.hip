@@ -30,7 +30,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_fwd_kernel(const uin
                                                         uint16_t* __restrict__ out,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
   if (tok >= T) return;
@@ -39,10 +39,10 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_fwd_kernel(const uin
   const float h[4] = {hp[0], hp[1], hp[2], hp[3]};
   const uint16_t* x0 = x + tok * 4 * C;
   if constexpr (!LOOP) {
-    if (sub < C / 8) k3_mix<8, NT>(x0, h, out + tok * C, sub, C);
-    row_tail<NT>(C, sub, [&](int c) { k3_mix<1, NT>(x0, h, out + tok * C, c, C); });
+    if (sub < C / 8) k3_mix<8, WHOLE, NT>(x0, h, out + tok * C, sub, C);
+    row_tail<WHOLE>(C, sub, [&](int c) { k3_mix<1, WHOLE, NT>(x0, h, out + tok * C, c, C); });
   } else {
-    k3_token<NT>(x0, h, out + tok * C, sub, LPT, C);
+    k3_token<WHOLE, NT>(x0, h, out + tok * C, sub, LPT, C);
   }
 }
 
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_bwd_kernel(const uin
                                                         float* __restrict__ grad_h_pre,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
   static_assert(!CANON || LPT >= 16, "slice order: whole 16-lane rows");
   constexpr int WPT = LPT > kWave ? LPT / kWave : 1;  // waves per token
   const int lane = threadIdx.x & (kWave - 1);
@@ -104,16 +104,16 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_bwd_kernel(const uin
     if constexpr (GX) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[e] = h0 * q[e];
-      Lanes<VEC, NT>::store(gx0, g, o);
+      Lanes<VEC, WHOLE>::store(gx0, g, o);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[e] = h1 * q[e];
-      Lanes<VEC, NT>::store(gx1, g, o);
+      Lanes<VEC, WHOLE>::store(gx1, g, o);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[e] = h2 * q[e];
-      Lanes<VEC, NT>::store(gx2, g, o);
+      Lanes<VEC, WHOLE>::store(gx2, g, o);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[e] = h3 * q[e];
-      Lanes<VEC, NT>::store(gx3, g, o);
+      Lanes<VEC, WHOLE>::store(gx3, g, o);
     }
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_bwd_kernel(const uin
 #pragma unroll 2
       for (int g = sub; g < ng; g += LPT) round(Vec<8>{}, g, s);
     }
-    row_tail<NT>(C, sub, [&](int c) { round(Vec<1>{}, c, s); });
+    row_tail<WHOLE>(C, sub, [&](int c) { round(Vec<1>{}, c, s); });
   }
   }
   if constexpr (!CANON) {
@@ -208,13 +208,13 @@ int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t 
   // workgroups per CU (T = 65536 104.5 us, against 106.3 with 128 lanes; with
   // few tokens 128 lanes: T = 4096 9.8 -> 8.8 us).
   if (C == 2 * 8 * kWave && T >= 16384 && aligned16(x) && aligned16(out)) {
-    using Walk = RowWalk<kWave, true, true>;
+    using Walk = RowWalk<kWave, true, true, true>;
     static const unsigned lds = lds_reserve(reinterpret_cast<const void*>(&k3_fwd_kernel<Walk>), kLdsCapSix);
     k3_fwd_kernel<Walk><<<dim3(blocks_for(T, tokens_per_block(kWave))), block_of<kWave>(), FMHC_LDS_CAP ? lds : 0u,
                           s>>>(x, h_pre, out, T, C);
     return launch_status();
   }
-  with_row_walk(C, aligned16(x) && aligned16(out), [&](auto w) {
+  with_row_walk(C, aligned16(x) && aligned16(out), T * C * 8, [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
     const dim3 grid(blocks_for(T, tokens_per_block(L)));
@@ -223,8 +223,8 @@ int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t 
     unsigned lds = 0;
     if (Walk::LOOP)
       lds = kLdsCapSix;
-    else if (Walk::NT && 4 * (C / 8) >= 3 * L)
-      lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::NT);
+    else if (Walk::WHOLE && 4 * (C / 8) >= 3 * L)
+      lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
     k3_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(x, h_pre, out, T, C);
   });
   return launch_status();
@@ -234,7 +234,7 @@ template <bool GX>
 int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uint16_t* grad_x,
                   float* grad_h_pre, int64_t T, int C, hipStream_t s) {
   const bool canon = k3_canon(C, lanes_per_token(C));
-  with_row_walk(C, aligned16(x) && aligned16(go) && aligned16(grad_x), [&](auto w) {
+  with_row_walk(C, aligned16(x) && aligned16(go) && aligned16(grad_x), T * C * 10, [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
     const dim3 grid(blocks_for(T, tokens_per_block(L)));
@@ -243,7 +243,7 @@ int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uin
       // Residency cap (fmhc_common.h): with grad_x and one group per lane.
       static const unsigned own = own_lds(reinterpret_cast<const void*>(&k3_bwd_kernel<Walk, GX, CANON>));
       unsigned lds = 0;
-      if (GX && FMHC_LDS_CAP && !Walk::LOOP) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::NT);
+      if (GX && FMHC_LDS_CAP && !Walk::LOOP) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
       k3_bwd_kernel<Walk, GX, CANON><<<grid, block_of<L>(), lds, s>>>(x, h_pre, go, grad_x, grad_h_pre, T, C);
     };
     if constexpr (L >= 16) {

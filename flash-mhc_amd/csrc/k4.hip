@@ -30,7 +30,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_fwd_kernel(const uin
                                                         uint16_t* __restrict__ out,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
   if (tok >= T) return;
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_fwd_kernel(const uin
         for (int j = 0; j < 4; ++j) acc = __builtin_fmaf(h[i][j], xv[j][e], acc);
         o[e] = acc;
       }
-      Lanes<VEC, NT>::store(orow[i], g, o);
+      Lanes<VEC, WHOLE>::store(orow[i], g, o);
     }
   };
   if constexpr (!LOOP) {
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_fwd_kernel(const uin
 #pragma unroll 2
     for (int g = sub; g < ng; g += LPT) mix(Vec<8>{}, g);
   }
-  row_tail<NT>(C, sub, [&](int c) { mix(Vec<1>{}, c); });
+  row_tail<WHOLE>(C, sub, [&](int c) { mix(Vec<1>{}, c); });
 }
 
 template <typename WALK, bool EARLY>
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
                                                         float* __restrict__ grad_hp,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
   constexpr int WPT = LPT > kWave ? LPT / kWave : 1;  // waves per token
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
         acc = __builtin_fmaf(p[2], q[2][e], acc);
         o[e] = __builtin_fmaf(p[3], q[3][e], acc);
       }
-      Lanes<VEC, NT>::store(glrow, g, o);
+      Lanes<VEC, WHOLE>::store(glrow, g, o);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
         acc = __builtin_fmaf(h[2][j], q[2][e], acc);
         o[e] = __builtin_fmaf(h[3][j], q[3][e], acc);
       }
-      Lanes<VEC, NT>::store(gxr[j], g, o);
+      Lanes<VEC, WHOLE>::store(gxr[j], g, o);
     }
   };
   if constexpr (!LOOP) {
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
 #pragma unroll 2
     for (int g = sub; g < ng; g += LPT) round(Vec<8>{}, g);
   }
-  row_tail<NT>(C, sub, [&](int c) { round(Vec<1>{}, c); });
+  row_tail<WHOLE>(C, sub, [&](int c) { round(Vec<1>{}, c); });
   }
 
   constexpr int GS = LPT < kWave ? LPT : kWave;
@@ -257,11 +257,11 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
 
 int launch_k4_fwd(const uint16_t* x, const uint16_t* lo, const float* H, const float* hp,
                   uint16_t* out, int64_t T, int C, hipStream_t s) {
-  with_row_walk(C, aligned16(x) && aligned16(lo) && aligned16(out), [&](auto w) {
+  with_row_walk(C, aligned16(x) && aligned16(lo) && aligned16(out), T * C * 10, [&](auto w) {
     constexpr int L = decltype(w)::LPT;
     // Tokens narrower than a wave are faster in the loop's schedule (T = 65536,
     // C = 176 42.7 -> 36.5 us, 256 50.5 -> 48.6); wider ones equal or slower.
-    using Walk = RowWalk<L, decltype(w)::LOOP || L < kWave, decltype(w)::NT>;
+    using Walk = RowWalk<L, decltype(w)::LOOP || L < kWave, decltype(w)::WHOLE, decltype(w)::NT>;
     const dim3 grid(blocks_for(T, tokens_per_block(L)));
     // Residency cap (fmhc_common.h).
     static const unsigned own = own_lds(reinterpret_cast<const void*>(&k4_fwd_kernel<Walk>));
@@ -269,7 +269,7 @@ int launch_k4_fwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
     if (decltype(w)::LOOP)
       lds = grid.x >= kCapMinBlocks ? kLdsCapFive : 0u;
     else
-      lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::NT);
+      lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
     k4_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(x, lo, H, hp, out, T, C);
   });
   return launch_status();
@@ -281,7 +281,12 @@ int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
                   const uint16_t* go, uint16_t* gx, uint16_t* glo, float* gH, float* ghp,
                   int64_t T, int C, hipStream_t s) {
   const bool aligned = aligned16(x) && aligned16(lo) && aligned16(go) && aligned16(gx) && aligned16(glo);
-  with_row_walk(C, aligned, [&](auto w) {
+  // Twice the bytes it reads: grad_out is new and x was last read before the
+  // layer, so ordinary loads win only where all of a step's tensors stay
+  // cached (training step, us, hint against none: T = 2048, C = 1024 113.3 /
+  // 111.8, T = 3000 145.5 / 149.5, T = 4096 160.9 / 163.3, T = 1003, C = 2560
+  // 174 / 178).
+  with_row_walk(C, aligned, 2 * (T * C * 18), [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
     const dim3 grid(blocks_for(T, tokens_per_block(L)));
@@ -292,7 +297,7 @@ int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
       // (T = 30000, C = 3000 440 us with and without).
       static const unsigned own = own_lds(reinterpret_cast<const void*>(&k4_bwd_kernel<W, E>));
       unsigned lds = 0;
-      if (FMHC_LDS_CAP && C / 8 <= L && L <= 256) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::NT);
+      if (FMHC_LDS_CAP && C / 8 <= L && L <= 256) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
       k4_bwd_kernel<W, E><<<grid, block_of<L>(), lds, s>>>(x, lo, H, hp, go, gx, glo, gH, ghp, T, C);
     };
     // EARLY: all of a lane's loads go out before its first store, so a wave
@@ -306,10 +311,10 @@ int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
     // keep the coefficients in vector registers and the plain order.
     if constexpr (L < kWave)
       launch(w, std::false_type{});
-    else if (!Walk::NT || T * L <= kK4EarlyLanes)
+    else if (!Walk::WHOLE || T * L <= kK4EarlyLanes)
       launch(w, std::true_type{});
     else
-      launch(RowWalk<L, true, Walk::NT>{}, std::false_type{});
+      launch(RowWalk<L, true, Walk::WHOLE, Walk::NT>{}, std::false_type{});
   });
   return launch_status();
 }

@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         xv[it][j] = u32x4{0u, 0u, 0u, 0u};
-        if (g < ng) xv[it][j] = Lanes<8, WHOLE>::raw(x0 + j * C, g);
+        if (g < ng) xv[it][j] = Lanes<8, false>::raw(x0 + j * C, g);  // the split kernel has just read it
       }
     }
   }
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
   __syncthreads();
   const float h[4] = {hsh[0], hsh[1], hsh[2], hsh[3]};
   if (!pre) {
-    k3_token<WHOLE>(x0, h, layer_input + t * C, lane, kFinishThreads, C);
+    k3_token<WHOLE, false>(x0, h, layer_input + t * C, lane, kFinishThreads, C);
     return;
   }
 #pragma unroll
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
       Lanes<8, WHOLE>::store(layer_input + t * C, g, o);
     }
   }
-  row_tail<WHOLE>(C, lane, [&](int c) { k3_mix<1, WHOLE>(x0, h, layer_input + t * C, c, C); });
+  row_tail<WHOLE>(C, lane, [&](int c) { k3_mix<1, WHOLE, false>(x0, h, layer_input + t * C, c, C); });
 }
 
 // Backward, few tokens (T <= kK2BwdSmallT) for rows of 17 to 255 groups of 8
@@ -236,11 +236,12 @@ __global__ __launch_bounds__(kK2BwdTok * LPT) void k3_reduce_k2_bwd(
   auto round = [&](auto vec, int g, float (&acc)[4]) __attribute__((always_inline)) {
     constexpr int VEC = decltype(vec)::value;
     float gq[VEC], a[VEC], b[VEC], c[VEC], d[VEC];
-    Lanes<VEC, true>::load(grow, g, gq);
-    Lanes<VEC, true>::load(x0, g, a);
-    Lanes<VEC, true>::load(x1, g, b);
-    Lanes<VEC, true>::load(x2, g, c);
-    Lanes<VEC, true>::load(x3, g, d);
+    // Ordinary loads: K1's backward reads both again right after.
+    Lanes<VEC, false>::load(grow, g, gq);
+    Lanes<VEC, false>::load(x0, g, a);
+    Lanes<VEC, false>::load(x1, g, b);
+    Lanes<VEC, false>::load(x2, g, c);
+    Lanes<VEC, false>::load(x3, g, d);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       acc[0] = __builtin_fmaf(a[e], gq[e], acc[0]);
