@@ -1158,24 +1158,30 @@ constexpr int kFwdSplit = 4;  // waves per workgroup (split of the nC axis)
 // equal at T = 65536 and 2% slower at T = 262144, C = 4096.
 constexpr int kFwdR = 4;
 constexpr int64_t kFwdCUs = 256;
-// Split forward for few tokens: one 16-token block per workgroup and up to
-// kSplitMax column ranges per block, aiming at kSplitTarget workgroups, each
-// range at least one 64-wide chunk per wave of the workgroup (narrower ranges
-// left waves idle: C = 1024, T = 1 ... 257 took 0.5-0.9 us longer); taken
-// when the plan has at least kSplitMinS ranges (T <= 2720 from C = 128 on),
-// twice that for rows of up to 64 chunks (C <= 1024: T <= 1024), whose
-// one-pass waves walk at most 8 chunks each.  At C = 1024 the pre-map forward
-// then takes 14.9 / 16.7 / 17.0 us at T = 1536 / 2048 / 2720 instead of
-// 18.8 / 18.6 / 24.8 (the K1 op 11.6 / 11.8 / 12.0 against 10.7 / 10.9 /
-// 13.7); at C = 4096 (32 chunks per wave) the split stays the faster form
-// (T = 1536: pre-map 39.0 against 48.6 us), and at C = 2048 it is up to
-// T = 2048 (K1 op 16.2 against 19.4 us at T = 1536, though 35.2 against
-// 28.4 us for the pre-map at 2720).  Above these counts the one-pass
-// kernel is faster (T = 3000 ... 6000: 20-40%).
-constexpr int kSplitR = 1;
-constexpr int64_t kSplitTarget = 512;
+// Split forward for few tokens: up to kSplitMax column ranges per token block,
+// as many as keep the launch within one workgroup per CU (kFwdCUs), each range
+// at least one 64-wide chunk per wave of the workgroup (narrower ranges left
+// waves idle: C = 1024, T = 1 ... 257 took 0.5-0.9 us longer).  Twice as many
+// ranges (up to 2.2 workgroups per CU, a last round of which kept a few CUs
+// busy alone) cost, pre-map forward: T = 1003, C = 2560 20.7 against 17.0 us,
+// T = 400, C = 4096 15.9 / 14.7, T = 512, C = 1024 10.3 / 9.7, T = 1003,
+// C = 1320 15.1 / 12.9.  Blocks of 32 tokens, which read W half as often, from
+// kSplitWideBlocks blocks of 16 on for rows of more than 64 chunks: T = 1003,
+// C = 2560 17.0 -> 16.3 us, C = 4096 21.4 -> 19.6; T = 2048, C = 2048 25.6 ->
+// 23.1, C = 4096 39.3 -> 33.4; below, T = 700, C = 2560 14.9 against 15.2.
+// The split is taken up to 73 blocks of 16 for rows of up to 64 chunks
+// (C <= 1024), 100 up to 88 chunks, kSplitMaxBlocks beyond: above, the pre-map
+// forward is faster as one kernel (the tile; tile against split, C = 1024
+// T = 1024 15.4 / 11.6 us, 1280 15.4 / 15.3, 1536 15.4 / 16.8; C = 1400
+// T = 1300 16.9 / 18.2, where K1 alone takes 11.9 / 10.8, T = 1700 17.2 / 19;
+// C = 2048 T = 2048 26.5 / 23.2, 2700 28.4 / 29.4; C = 4096 T = 2700 53.6 /
+// 44.3, 3400 58.6 / 60.0).  Pre-map forward with all three rules, before and
+// after: T = 1003, C = 2560 20.7 -> 16.3 us, C = 4096 26.0 -> 19.8; T = 2000,
+// C = 1320 22.0 -> 16.6; T = 2700, C = 4096 54.5 -> 43.9; T = 64 and fewer
+// tokens unchanged.
 constexpr int64_t kSplitMax = 64;
-constexpr int64_t kSplitMinS = 4;
+constexpr int64_t kSplitMaxBlocks = 170;
+constexpr int64_t kSplitWideBlocks = 57;
 // Runs of k1_bwd_mfma: up to kBwdNTB blocks of 16 tokens per run for dx
 // alone, kBwdDwNTB with grad_W (fewer runs, fewer grad_W partials); with few
 // tokens, runs as short as kBwdDwMinNTB blocks with grad_W (its partials then
@@ -1212,29 +1218,49 @@ BwdSlices bwd_premap_slices(int64_t C) { return bwd_slices(4 * C, C % 8 == 0 ? 4
 // element offsets.
 bool k1_fwd_mfma_path(int64_t nC) { return nC >= 8 && nC <= (int64_t{1} << 24); }
 
-// Column split of the forward for T tokens (S = 1: the one-pass kernel).
+// S column ranges of nall chunks, at least one chunk per wave each, none empty
+// (cps chunks in each but the last); S = 1: no split.
+struct ColumnRanges {
+  int64_t S, cps;
+};
+ColumnRanges column_ranges(int64_t S, int64_t nall) {
+  S = S < kSplitMax ? S : kSplitMax;
+  S = S < nall / kFwdSplit ? S : nall / kFwdSplit;
+  if (S < 2) return {1, nall};
+  const int64_t cps = (nall + S - 1) / S;
+  return {(nall + cps - 1) / cps, cps};
+}
+
+// Column split of the forward for T tokens (S = 1: the one-pass kernel), with
+// R blocks of 16 tokens per workgroup.
 struct K1FwdSplit {
-  int S = 1, cps = 0;
-  int64_t bytes = 0;  // partial sums: T x 33 x S4 fp32
+  int S = 1, R = 1, cps = 0;
 };
 
 K1FwdSplit k1_fwd_split(int64_t T, int64_t nC) {
   K1FwdSplit p;
   const int64_t nall = nC >> 6;
-  if (T <= 0 || !k1_fwd_mfma_path(nC) || nall < 2) return p;
-  const int64_t nblk = (T + 16 * kSplitR - 1) / (16 * kSplitR);
-  int64_t S = (kSplitTarget + nblk - 1) / nblk;
-  if (S < (nall <= 64 ? 2 * kSplitMinS : kSplitMinS)) return p;
-  S = S < kSplitMax ? S : kSplitMax;
-  S = S < nall / kFwdSplit ? S : nall / kFwdSplit;
-  if (S < 2) return p;
-  const int64_t cps = (nall + S - 1) / S;
-  S = (nall + cps - 1) / cps;  // every split non-empty
-  if (S < 2) return p;
-  p.S = static_cast<int>(S);
-  p.cps = static_cast<int>(cps);
-  p.bytes = T * (kDout + 1) * ((S + 3) & ~int64_t{3}) * static_cast<int64_t>(sizeof(float));
+  if (T <= 0 || !k1_fwd_mfma_path(nC)) return p;
+  const int64_t n16 = (T + 15) / 16;
+  if (n16 > (nall <= 64 ? 73 : nall <= 88 ? 100 : kSplitMaxBlocks)) return p;
+  p.R = n16 >= kSplitWideBlocks && nall > 64 ? 2 : 1;
+  const ColumnRanges c = column_ranges(kFwdCUs / ((n16 + p.R - 1) / p.R), nall);
+  p.S = static_cast<int>(c.S);
+  p.cps = static_cast<int>(c.cps);
   return p;
+}
+
+// Workspace for the partial sums, T x 33 x S4 fp32 (S4: S rounded up to 4):
+// that of twice as many column ranges, up to kSplitMaxBlocks blocks of 16
+// tokens (73 for rows of up to 64 chunks).  The plan needs no more (fewer
+// ranges, or none); callers' workspaces keep the size they have had.
+int64_t k1_fwd_split_bytes(int64_t T, int64_t nC) {
+  const int64_t nall = nC >> 6;
+  if (T <= 0 || !k1_fwd_mfma_path(nC)) return 0;
+  const int64_t n16 = (T + 15) / 16;
+  if (n16 > (nall <= 64 ? 73 : kSplitMaxBlocks)) return 0;
+  const int64_t S = column_ranges((2 * kFwdCUs + n16 - 1) / n16, nall).S;
+  return S < 2 ? 0 : T * (kDout + 1) * ((S + 3) & ~int64_t{3}) * static_cast<int64_t>(sizeof(float));
 }
 
 // Blocks of 16 tokens per workgroup of the one-pass forward for T tokens.
@@ -1277,17 +1303,18 @@ void launch_k1_fwd_onepass(int R, const uint16_t* x, const uint16_t* W, uint16_t
 // The column-split forward's first kernel.
 int launch_k1_fwd_split(const K1FwdSplit& p, const uint16_t* x, const uint16_t* W, float* part, int64_t T, int nc,
                         hipStream_t s) {
-  const dim3 grid(blocks_for(T, 16 * kSplitR), p.S);
-  if (nc % 8 == 0)
-    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, true, false><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr, part,
-                                                                                       T, nc, p.cps);
-  else
-    k1_fwd_mfma<kSplitR, kFwdSplit, true, false, false, false><<<grid, kWave * kFwdSplit, 0, s>>>(x, W, nullptr, nullptr,
-                                                                                        part, T, nc, p.cps);
+  auto launch = [&](auto r, auto whole) {
+    constexpr int R = decltype(r)::value;
+    constexpr bool WHOLE = decltype(whole)::value;
+    k1_fwd_mfma<R, kFwdSplit, true, false, WHOLE, false><<<dim3(blocks_for(T, 16 * R), p.S), kWave * kFwdSplit, 0, s>>>(
+        x, W, nullptr, nullptr, part, T, nc, p.cps);
+  };
+  auto rows = [&](auto r) { nc % 8 == 0 ? launch(r, std::true_type{}) : launch(r, std::false_type{}); };
+  p.R == 2 ? rows(std::integral_constant<int, 2>{}) : rows(std::integral_constant<int, 1>{});
   return launch_status();
 }
 
-// K1 forward; with a workspace of k1_fwd_split(T, nC).bytes (allow_split) few
+// K1 forward; with a workspace of k1_fwd_split_bytes(T, nC) (allow_split) few
 // tokens take the column-split kernel.
 int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* inv_rms, void* ws,
                int64_t ws_bytes, bool allow_split, int64_t T, int64_t nC, hipStream_t s) {
@@ -1295,7 +1322,7 @@ int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* 
   if (k1_fwd_mfma_path(nC)) {
     const K1FwdSplit p = allow_split ? k1_fwd_split(T, nC) : K1FwdSplit{};
     if (p.S > 1) {
-      if (!ws || ws_bytes < p.bytes || !aligned16(ws)) return FMHC_ERR_INVALID_ARGUMENT;
+      if (!ws || ws_bytes < k1_fwd_split_bytes(T, nC) || !aligned16(ws)) return FMHC_ERR_INVALID_ARGUMENT;
       float* part = static_cast<float*>(ws);
       const int st = launch_k1_fwd_split(p, x_flat, W, part, T, nc, s);
       if (st != FMHC_OK) return st;
@@ -1388,7 +1415,7 @@ extern "C" int fmhc_k1_fwd(const uint16_t* x_flat, const uint16_t* W, uint16_t* 
 }
 
 extern "C" int64_t fmhc_k1_fwd_workspace_bytes(int64_t T, int64_t nC) {
-  return fmhc::k1_fwd_split(T, nC).bytes;
+  return fmhc::k1_fwd_split_bytes(T, nC);
 }
 
 extern "C" int fmhc_k1_fwd_ws(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* inv_rms,
@@ -1523,7 +1550,7 @@ int k1_fwd_partials(const uint16_t* x_flat, const uint16_t* W, void* ws, int64_t
                     int64_t nC, hipStream_t s) {
   const K1FwdSplit p = k1_fwd_split(T, nC);
   if (p.S < 2) return 0;
-  if (!ws || ws_bytes < p.bytes || !aligned16(ws)) return -FMHC_ERR_INVALID_ARGUMENT;
+  if (!ws || ws_bytes < k1_fwd_split_bytes(T, nC) || !aligned16(ws)) return -FMHC_ERR_INVALID_ARGUMENT;
   const int st = launch_k1_fwd_split(p, x_flat, W, static_cast<float*>(ws), T, static_cast<int>(nC), s);
   return st == FMHC_OK ? p.S : -st;
 }

@@ -14,8 +14,8 @@
 // Forward.  Rows of C = 512 or 1024 per stream with at least 16384 tokens
 // and a layer input: the single-read kernel (premap_resident.hip), which
 // keeps W on each CU and reads every row of x once.  Other shapes from the
-// token count where K1 runs one pass (no column split; T > 1024 up to
-// C = 1024, T > 2720 above): one tile kernel (k1_premap_tile, k1.hip).  Each
+// token count where K1 runs one pass (no column split: T > 1168 up to
+// C = 1024, T > 1600 up to 1423, T > 2720 above): one tile kernel (k1_premap_tile, k1.hip).  Each
 // workgroup runs K1 on its tile (16, 32, 48 or 64 tokens, the fewest that
 // keep the launch to one round on the CUs) with ordinary loads of x, then K2
 // on the tile's tokens (four lanes per token) and K3 on the tile.  K3's
@@ -375,7 +375,7 @@ int premap_fwd_run(const uint16_t* x, const uint16_t* W, const void* alpha_pre, 
 }
 
 // Scratch of fmhc_premap_fwd_noalloc: the column-split forward's partial sums
-// (T x 33 x S4 fp32 for T <= 2720 tokens; at most 2,145,792 bytes over every
+// (T x 33 x S4 fp32; k1_fwd_split_bytes is at most 2,145,792 bytes over every
 // (T, C), at T = 2032, C = 1040).  Each device holds its own copy for the life
 // of the process.  In host code `scratch` names a host-side stand-in, so its
 // device address is looked up once per device (scratch_on_device) and only

@@ -54,9 +54,9 @@ extern "C" {
  *           src/flash_mhc/kernels.py:250-303 (_fused_rmsnorm_project_fwd_kernel). */
 int fmhc_k1_fwd(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* inv_rms,
                 int64_t T, int64_t nC, int64_t D_out, void* stream);
-/* fmhc_k1_fwd with a workspace: for few tokens (T <= 1024 up to nC = 4096,
- * T <= 2720 above) the nC axis is split
- * over up to 64 workgroups per 16-token block, whose fp32 partial sums (in
+/* fmhc_k1_fwd with a workspace: for few tokens (T <= 1168 up to nC = 4159,
+ * 1600 up to nC = 5695, 2720 above) the nC axis is split over up to 64
+ * workgroups per 16- or 32-token block, whose fp32 partial sums (in
  * `workspace`) a second kernel adds in a fixed order.  `workspace`: at least
  * fmhc_k1_fwd_workspace_bytes(T, nC) bytes, 16-byte aligned (may be NULL when
  * that is 0).  Results equal fmhc_k1_fwd's up to fp32 summation order.  No

@@ -53,7 +53,9 @@ def _params(C):
 # chunk of 1 to 63 columns: C = 2 and 3 (one group, rows of 8 and 12 columns),
 # 15 ... 17 around one 64-column chunk.
 FWD = [*SHAPES, (5, 2), (40, 3), (4096, 16), (2721, 129), (5000, 131), (9000, 33), (12300, 25), (20011, 300),
-       (2720, 4099), (3, 4103)]
+       (2720, 4099), (3, 4103),
+       # The split's blocks of 16 (up to 912 tokens) and of 32, and its last token counts.
+       (912, 1100), (913, 1101), (929, 1100), (1168, 1024), (1169, 1024), (1600, 1423), (1601, 1420), (2719, 1424)]
 
 
 @pytest.mark.parametrize("off", [0, 1, 3])
