@@ -1179,7 +1179,7 @@ constexpr int64_t kFwdCUs = 256;
 // after: T = 1003, C = 2560 20.7 -> 16.3 us, C = 4096 26.0 -> 19.8; T = 2000,
 // C = 1320 22.0 -> 16.6; T = 2700, C = 4096 54.5 -> 43.9; T = 64 and fewer
 // tokens unchanged.
-constexpr int64_t kSplitMax = 64;
+constexpr int64_t kSplitMax = kK1MaxSplits;
 constexpr int64_t kSplitMaxBlocks = 170;
 constexpr int64_t kSplitWideBlocks = 57;
 // Runs of k1_bwd_mfma: up to kBwdNTB blocks of 16 tokens per run for dx

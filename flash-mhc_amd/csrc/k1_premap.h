@@ -10,6 +10,7 @@
 namespace fmhc {
 
 constexpr float kRmsEps = 1e-6f;  // K1's RMSNorm epsilon (kernels.py:296 of the reference)
+constexpr int kK1MaxSplits = 64;   // column ranges of K1's split forward, at most
 
 // The first kernel of K1's column-split forward alone: when T tokens take that
 // path (few tokens, MFMA-eligible pointers) it writes the fp32 partial sums to

@@ -426,25 +426,37 @@ __device__ __forceinline__ void k2_token4(const float* p, const K2Smem& sm, int 
 // denominator and each H_res entry are added sequentially over m), so the
 // results are bit-identical to the one-thread chain's.
 // Returns lane q's sigmoid value: h_pre[t, q] for q < 4.
+// LOW: the group is lanes 0-31 of its wave, the only active ones; the values
+// then pass between lanes as scalars and on the VALU's cross-lane moves
+// instead of LDS permutes (the same values and sums).
+template <bool LOW = false>
 __device__ __forceinline__ float k2_token32(const K2Smem& sm, float p, int q, int64_t t, float* __restrict__ h_pre,
                                             float* __restrict__ h_post, float* __restrict__ H) {
 #pragma clang fp contract(off)
+  auto from = [](float v, int src) __attribute__((always_inline)) {  // src: a constant
+    return LOW ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src)) : __shfl(v, src, 32);
+  };
   const float alpha = q < kN ? sm.sc[0] : (q < 2 * kN ? sm.sc[1] : sm.sc[2]);
   const float z = rb(rb(alpha * p) + sm.sc[3 + q]);
   const float y = q < 2 * kN ? rb(sigmoid_f32(z)) : 0.f;  // h_pre (q < 4), sigmoid of the post logit
   const float hq = rb(2.f * y);                             // h_post for 4 <= q < 8
   float mx = q >= 2 * kN ? z : -INFINITY;
+  if constexpr (LOW) {
 #pragma unroll
-  for (int o = 16; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 32));
+    for (int m = kN * 2; m < kDk; ++m) mx = fmaxf(mx, from(z, m));
+  } else {
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 32));
+  }
   const float e = q >= 2 * kN ? expf(z - mx) : 0.f;
   float sum = 0.f;
 #pragma unroll
-  for (int m = 0; m < kNF; ++m) sum = sum + __shfl(e, 2 * kN + m, 32);
+  for (int m = 0; m < kNF; ++m) sum = sum + from(e, 2 * kN + m);
   const float a = rb(e / sum);
   const float* pf = reinterpret_cast<const float*>(sm.perm);
   float acc = 0.f;
 #pragma unroll
-  for (int m = 0; m < kNF; ++m) acc = acc + __shfl(a, 2 * kN + m, 32) * pf[m * kN * kN + (q & 15)];
+  for (int m = 0; m < kNF; ++m) acc = acc + from(a, 2 * kN + m) * pf[m * kN * kN + (q & 15)];
   const float hp_j = __shfl(y, q & 3, 32);
   const float hq_i = __shfl(hq, kN + ((q & 15) >> 2), 32);
   if (q < kN * kN) H[t * kN * kN + q] = rb(rb(acc) - rb(hq_i * hp_j));

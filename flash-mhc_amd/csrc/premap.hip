@@ -72,25 +72,18 @@ bool param_dtype_ok(int d) { return d == FMHC_PARAM_F32 || d == FMHC_PARAM_BF16;
 
 constexpr int kFinishThreads = 256;  // 8 tokens of 32 lanes
 
-// Few tokens: K1's second stage and K2 in one kernel, 32 lanes per token.
-// Lane q adds the S partials of projection q and those of the sum of squares
-// in split order (as k1_fwd_finish does), stores proj[t, q] =
-// bf16(sum * inv_rms) and inv_rms, then runs K2 on that bf16 value
-// (k2_token32): the same values as K1's finish kernel followed by K2.
-// K1's second stage for token t in 32 lanes: lane q adds the S partials of
-// projection q and of the sum of squares in split order, stores proj[t, q]
-// and (lane 0) inv_rms[t], and returns the stored bf16 projection as fp32.
-__device__ __forceinline__ float finish_token32(const float* __restrict__ part, int S, int nC, int q, int64_t t,
-                                                uint16_t* __restrict__ proj, float* __restrict__ inv_rms) {
-  // The loads of both sums run ahead together.
-  const int s4 = (S + 3) & ~3;
-  const f32x4* pv = reinterpret_cast<const f32x4*>(part + (t * (kDk + 1) + q) * s4);
-  const f32x4* ps = reinterpret_cast<const f32x4*>(part + (t * (kDk + 1) + kDk) * s4);
-  float v = 0.f, ss = 0.f;
+// Adds the S partials of a projection and of the sum of squares in split
+// order; at(i) gives the i-th four of each.
+struct SplitPair {
+  f32x4 v, ss;
+};
+template <typename F>
+__device__ __forceinline__ void add_splits(int S, F&& at, float& v, float& ss) {
 #pragma unroll 8
-  for (int i = 0; i < s4 / 4; ++i) {
-    const f32x4 a = pv[i], b = ps[i];
-    v += a[0];  // 4 i < S always
+  for (int i = 0; 4 * i < S; ++i) {
+    const SplitPair w = at(i);
+    const f32x4 a = w.v, b = w.ss;
+    v += a[0];
     ss += b[0];
     if (4 * i + 1 < S) {
       v += a[1];
@@ -105,6 +98,12 @@ __device__ __forceinline__ float finish_token32(const float* __restrict__ part, 
       ss += b[3];
     }
   }
+}
+
+// K1's outputs of token t from those sums: lane q stores proj[t, q] and (lane
+// 0) inv_rms[t], and returns the stored bf16 projection as fp32.
+__device__ __forceinline__ float store_projection(float v, float ss, int nC, int q, int64_t t,
+                                                  uint16_t* __restrict__ proj, float* __restrict__ inv_rms) {
   const float inv = rsqrtf(ss / static_cast<float>(nC) + kRmsEps);
   const uint16_t pj = f32_to_bf16(v * inv);
   proj[t * kDk + q] = pj;
@@ -112,6 +111,25 @@ __device__ __forceinline__ float finish_token32(const float* __restrict__ part, 
   return bf16_to_f32(pj);
 }
 
+// K1's second stage for token t in 32 lanes: lane q adds the S partials of
+// projection q and of the sum of squares in split order, stores proj[t, q]
+// and (lane 0) inv_rms[t], and returns the stored bf16 projection as fp32.
+__device__ __forceinline__ float finish_token32(const float* __restrict__ part, int S, int nC, int q, int64_t t,
+                                                uint16_t* __restrict__ proj, float* __restrict__ inv_rms) {
+  // The loads of both sums run ahead together.
+  const int s4 = (S + 3) & ~3;
+  const f32x4* pv = reinterpret_cast<const f32x4*>(part + (t * (kDk + 1) + q) * s4);
+  const f32x4* ps = reinterpret_cast<const f32x4*>(part + (t * (kDk + 1) + kDk) * s4);
+  float v = 0.f, ss = 0.f;
+  add_splits(S, [&](int i) { return SplitPair{pv[i], ps[i]}; }, v, ss);
+  return store_projection(v, ss, nC, q, t, proj, inv_rms);
+}
+
+// Few tokens: K1's second stage and K2 in one kernel, 32 lanes per token.
+// Lane q adds the S partials of projection q and those of the sum of squares
+// in split order (as k1_fwd_finish does), stores proj[t, q] =
+// bf16(sum * inv_rms) and inv_rms, then runs K2 on that bf16 value
+// (k2_token32): the same values as K1's finish kernel followed by K2.
 __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2(
     const float* __restrict__ part, int S, int nC, const K2Params P, uint16_t* __restrict__ proj,
     float* __restrict__ inv_rms, float* __restrict__ h_pre, float* __restrict__ h_post, float* __restrict__ H,
@@ -130,19 +148,40 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2(
 // lanes finish K1 and run K2 and leave h_pre in LDS; after the barrier all
 // 256 lanes mix the token's streams into layer_input with those values
 // (k3_token's arithmetic, so the results are those of the separate K3 kernel
-// reading the stored h_pre).  Saves K3's launch for few tokens.  Up to
-// C = 4096 (two 16-byte groups per lane) every lane loads its x vectors
-// before K1's partial sums and K2's chain run, so their latency overlaps.
+// reading the stored h_pre).  Saves K3's launch for few tokens.  A chain of
+// latencies bounds it, so everything it reads is asked for at once: the x
+// vectors (up to C = 4096, two 16-byte groups per lane), K2's parameters and
+// the token's partial sums, spread over all lanes and handed to the first 32
+// through LDS.  One after the other (the parameters, then up to two batches of
+// partial sums in the first 32 lanes, then K2 on LDS permutes) the pre-map
+// forward took, us: T = 1, C = 4096 8.9, now 8.6; T = 64 9.8 / 9.5; T = 1003,
+// C = 2560 16.2 / 15.3; T = 1024, C = 1024 11.7 / 11.0; T = 1536, C = 2048
+// 20.5 / 18.7.
 template <bool WHOLE>
 __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
     const float* __restrict__ part, int S, int nC, const K2Params P, uint16_t* __restrict__ proj,
     float* __restrict__ inv_rms, float* __restrict__ h_pre, float* __restrict__ h_post, float* __restrict__ H,
     const ZeroWords z, const uint16_t* __restrict__ x, uint16_t* __restrict__ layer_input, int C) {
+  constexpr int kVecs = (kDk + 1) * (kK1MaxSplits / 4);  // 16-byte vectors of partial sums, at most
+  constexpr int kVecsPerLane = (kVecs + kFinishThreads - 1) / kFinishThreads;
   __shared__ K2Smem sm;
   __shared__ float hsh[kN];  // the token's h_pre, handed from the K2 lanes to all
+  // Vector i at i + i / 16, which spreads rows of 16 vectors over the banks.
+  __shared__ f32x4 psum[kVecs + kVecs / 16];
   constexpr int kPre = 2;    // 16-byte groups per lane and stream loaded ahead
   const int64_t t = blockIdx.x;
   const int lane = static_cast<int>(threadIdx.x);
+  const int row4 = (S + 3) >> 2;  // vectors per value
+  const int n4 = (kDk + 1) * row4;
+  const f32x4* pv = reinterpret_cast<const f32x4*>(part) + t * n4;
+  f32x4 pr[kVecsPerLane];
+#pragma unroll
+  for (int r = 0; r < kVecsPerLane; ++r) {
+    const int i = lane + r * kFinishThreads;
+    if (i < n4) pr[r] = pv[i];
+  }
+  K2ParamRegs<kFinishThreads> regs;
+  regs.load(P);
   const uint16_t* x0 = x + t * 4 * C;
   const int ng = C / 8;
   const bool pre = ng <= kPre * kFinishThreads;
@@ -159,11 +198,22 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
     }
   }
   zero_words(z);
-  stage_params<kFinishThreads>(P, sm);
+#pragma unroll
+  for (int r = 0; r < kVecsPerLane; ++r) {
+    const int i = lane + r * kFinishThreads;
+    if (i < n4) psum[i + (i >> 4)] = pr[r];
+  }
+  regs.store(sm);
+  __syncthreads();
   if (threadIdx.x < 32) {
     const int q = lane;
-    const float p = finish_token32(part, S, nC, q, t, proj, inv_rms);
-    const float y = k2_token32(sm, p, q, t, h_pre, h_post, H);
+    float v = 0.f, ss = 0.f;
+    add_splits(S, [&](int i) {
+      const int a = q * row4 + i, b = kDk * row4 + i;
+      return SplitPair{psum[a + (a >> 4)], psum[b + (b >> 4)]};
+    }, v, ss);
+    const float p = store_projection(v, ss, nC, q, t, proj, inv_rms);
+    const float y = k2_token32<true>(sm, p, q, t, h_pre, h_post, H);
     if (q < kN) hsh[q] = y;
   }
   __syncthreads();
