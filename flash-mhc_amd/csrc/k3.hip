@@ -235,10 +235,10 @@ int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uin
                   float* grad_h_pre, int64_t T, int C, hipStream_t s) {
   const bool canon = k3_canon(C, lanes_per_token(C));
   with_row_walk(C, aligned16(x) && aligned16(go) && aligned16(grad_x), T * C * 10, [&](auto w) {
-    using Walk = decltype(w);
-    constexpr int L = Walk::LPT;
+    constexpr int L = decltype(w)::LPT;
     const dim3 grid(blocks_for(T, tokens_per_block(L)));
-    auto launch = [&](auto canon_c) {
+    auto launch = [&](auto walk, auto canon_c) {
+      using Walk = decltype(walk);
       constexpr bool CANON = decltype(canon_c)::value;
       // Residency cap (fmhc_common.h): with grad_x and one group per lane.
       static const unsigned own = own_lds(reinterpret_cast<const void*>(&k3_bwd_kernel<Walk, GX, CANON>));
@@ -247,9 +247,15 @@ int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uin
       k3_bwd_kernel<Walk, GX, CANON><<<grid, block_of<L>(), lds, s>>>(x, h_pre, go, grad_x, grad_h_pre, T, C);
     };
     if constexpr (L >= 16) {
-      if (canon) return launch(std::true_type{});
+      if (canon) return launch(w, std::true_type{});
     }
-    launch(std::false_type{});
+    // With grad_x, tokens narrower than a wave are equal or faster in the
+    // loop's schedule (T = 65536, C = 100 25.7 -> 23.2 us, C = 250 51.2 -> 49.7,
+    // T = 100000, C = 60 24.7 -> 23.3).
+    if constexpr (GX && L < kWave)
+      launch(RowWalk<L, true, decltype(w)::WHOLE, decltype(w)::NT>{}, std::false_type{});
+    else
+      launch(w, std::false_type{});
   });
   return launch_status();
 }
