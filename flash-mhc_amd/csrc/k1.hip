@@ -970,14 +970,18 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
 // Workgroups from dw_blocks on sum K2's parameter gradients instead, one
 // workgroup per parameter (the pre-map backward; one launch fewer than K2's
 // own reduce).
-// SPLIT: the four waves of a workgroup take the same elements and a quarter of
-// the runs each, added in wave order.  For up to kReduceSplitSlices slices,
-// whose elements alone leave CUs without a workgroup while every thread walks
-// hundreds of runs one load latency after the other: pre-map backward at
-// T = 65536, C = 64 87.4 -> 62.5 us, 100 91 -> 78, 256 131 -> 127.5; T = 8192,
-// C = 512 51 -> 48.7.  With more slices it loses 1% (C = 1024, 2560).
-constexpr int kReduceSplitSlices = 16;
-template <bool SPLIT>
+// GROUPS: that many groups of threads take the same elements and a share of
+// the runs each, added in group order.  With few slices the elements alone
+// leave CUs without a workgroup while every thread walks hundreds of runs, up
+// to 1024, one load latency after the other.  Four groups up to
+// kReduceSplit4Slices slices: pre-map backward at T = 65536, C = 64 87.4 ->
+// 62.5 us, 100 91 -> 78, 256 131 -> 127.5; T = 8192, C = 512 51 -> 48.7; with
+// more slices 1% slower (C = 1024, 2560).  Sixteen up to kReduceSplit16Slices:
+// T = 65536, C = 24 59.7 -> 43.8, 64 59.3 -> 54.5; K1 backward C = 24 35.0 ->
+// 22.2, 100 32.1 -> 30.9, T = 8192, C = 256 17.7 -> 17.0; equal above.
+constexpr int kReduceSplit16Slices = 8;
+constexpr int kReduceSplit4Slices = 16;
+template <int GROUPS>
 __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ partial,
                                                     uint16_t* __restrict__ dW, int64_t nparts,
                                                     const BwdSlices sl, int nC, unsigned dw_blocks,
@@ -987,16 +991,16 @@ __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ pa
     return;
   }
   const int64_t per_part = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave);
-  constexpr int kVecs = SPLIT ? kWave : 256;  // 16-byte vectors per workgroup
-  const int wave = SPLIT ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6) : 0;
-  const int lane = static_cast<int>(threadIdx.x) & (kVecs - 1);
+  constexpr int kVecs = 256 / GROUPS;  // 16-byte vectors per workgroup
+  const int group = static_cast<int>(threadIdx.x) / kVecs;
+  const int lane = static_cast<int>(threadIdx.x) % kVecs;
   // Below per_part, which is a multiple of 8192.
   const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * kVecs + lane) * 4;
   const f32x4* src = reinterpret_cast<const f32x4*>(partial + i0);
   const int64_t stride = per_part / 4;  // in 16-byte vectors
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  int64_t p = SPLIT ? nparts * wave / 4 : 0;
-  const int64_t end = SPLIT ? nparts * (wave + 1) / 4 : nparts;
+  int64_t p = nparts * group / GROUPS;
+  const int64_t end = nparts * (group + 1) / GROUPS;
   for (; p + 4 <= end; p += 4) {
     const f32x4 v0 = src[(p + 0) * stride], v1 = src[(p + 1) * stride];
     const f32x4 v2 = src[(p + 2) * stride], v3 = src[(p + 3) * stride];
@@ -1006,13 +1010,13 @@ __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ pa
     acc += v3;
   }
   for (; p < end; ++p) acc += src[p * stride];
-  if constexpr (SPLIT) {
-    __shared__ f32x4 quarter[4][kWave];
-    quarter[wave][lane] = acc;
+  if constexpr (GROUPS > 1) {
+    __shared__ f32x4 sums[GROUPS][kVecs];
+    sums[group][lane] = acc;
     __syncthreads();
-    if (wave != 0) return;
+    if (group != 0) return;
 #pragma unroll
-    for (int w = 1; w < 4; ++w) acc += quarter[w][lane];
+    for (int g = 1; g < GROUPS; ++g) acc += sums[g][lane];
   }
   const int lane0 = static_cast<int>(i0 % kWave);  // multiple of 4
   const int rr = static_cast<int>((i0 / kWave) % 4);
@@ -1473,13 +1477,17 @@ int launch_dw_reduce(const float* partial, uint16_t* grad_W, int64_t nruns, cons
                      const K2ParamSums& sums, int k2_params, hipStream_t s) {
   static_assert(kK2SumThreads == 256, "K2's parameter sums share the reduce's workgroups");
   const int64_t vecs = static_cast<int64_t>(sl.n) * (8 * 2 * 4 * kWave) / 4;
-  if (sl.n <= kReduceSplitSlices) {
-    const unsigned nb = blocks_for(vecs, kWave);
-    k1_dw_reduce<true><<<dim3(nb + k2_params), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
-  } else {
-    const unsigned nb = blocks_for(vecs, 256);
-    k1_dw_reduce<false><<<dim3(nb + k2_params), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
-  }
+  auto launch = [&](auto groups) {
+    constexpr int G = decltype(groups)::value;
+    const unsigned nb = blocks_for(vecs, 256 / G);
+    k1_dw_reduce<G><<<dim3(nb + k2_params), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
+  };
+  if (sl.n <= kReduceSplit16Slices)
+    launch(std::integral_constant<int, 16>{});
+  else if (sl.n <= kReduceSplit4Slices)
+    launch(std::integral_constant<int, 4>{});
+  else
+    launch(std::integral_constant<int, 1>{});
   return launch_status();
 }
 

@@ -161,7 +161,17 @@ __device__ __forceinline__ void k2_param_sum(const K2ParamSums& r, int k) {
   __shared__ float wsum[kK2SumThreads / kWave];
   const int t = static_cast<int>(threadIdx.x);
   float v = 0.f;
-  for (int64_t b = t; b < r.nblocks; b += kK2SumThreads) v += r.partial[b * kNPar + k];
+  // Eight loads ahead of their sums: one after the other their latencies were
+  // the launch's longest chain.
+  int64_t b = t;
+  for (; b + 7 * kK2SumThreads < r.nblocks; b += 8 * kK2SumThreads) {
+    float w[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) w[u] = r.partial[(b + u * kK2SumThreads) * kNPar + k];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v += w[u];
+  }
+  for (; b < r.nblocks; b += kK2SumThreads) v += r.partial[b * kNPar + k];
   v = wave_sum(v);
   if ((t & (kWave - 1)) == 0) wsum[t / kWave] = v;
   __syncthreads();

@@ -151,3 +151,18 @@ def test_k3_k4(T, C, off):
     check_bf16("k4 grad_lo", glo, *ref["grad_lo"], 4)
     check_fp32("k4 grad_H", gH, *ref["grad_H"], C)
     check_fp32("k4 grad_hp", ghp, *ref["grad_hp"], C)
+
+
+# grad_W's reduce: 16 shares of the runs up to 8 slices of 128 columns (C = 256),
+# four up to 16, one above; one run to several hundred, fewer runs than shares.
+@pytest.mark.parametrize("T,C", [(1, 64), (40, 24), (9000, 24), (16001, 33), (3000, 256), (3000, 264), (2000, 512),
+                                 (2000, 520)])
+def test_grad_W_reduce(T, C):
+    nC = 4 * C
+    rn, x, W = _inputs(T, C, 0, 17 * T + C)
+    x = x.view(T, nC)
+    proj, inv = K.k1_fwd(x, W)
+    go = rn(T, 32)
+    _, gW = K.k1_bwd(go, x, W, proj, inv)
+    R, S = O.k1_grad_W(go.cpu(), x.cpu(), inv.cpu())
+    check_bf16("grad_W", gW, R, S, T)
