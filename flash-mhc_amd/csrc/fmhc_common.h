@@ -96,12 +96,12 @@ __device__ __forceinline__ void st8_stream(void* p, u32x2 v) {
 // lines loaded under the hint are not kept for it: ordinary loads win where an
 // earlier launch touched the operands, and lose 2-5% where none did, from HBM.
 // Stores keep the hint at every size (without it T = 1024, C = 1024 K4 backward
-// 8.0 -> 8.9 us, K4 forward 4.3 -> 5.1).  With the hint against
-// without, three sets of operands in turn, us: T = 1003, C = 2560 K1 backward
-// 24.1 / 19.1, K3 forward 6.2 / 5.9, K4 forward 9.5 / 8.9; T = 4096, C = 1024
-// K1 backward 25.9 / 20.4; T = 8192, C = 1024 K1 forward 18.5 / 13.8, K3 backward 26.2 / 23.9, K4 forward 25.4 / 23.5; past
-// the line, T = 16384, C = 1024 K1 forward 25.1 / 26.9, K3 backward 49.2 /
-// 51.7, K4 forward 47.9 / 51.7.
+// 8.0 -> 8.9 us, K4 forward 4.3 -> 5.1).  With the hint against without, three
+// sets of operands in turn, us: T = 1003, C = 2560 K1 backward 24.1 / 19.1, K3
+// forward 6.2 / 5.9, K4 forward 9.5 / 8.9; T = 4096, C = 1024 K1 backward 25.9 /
+// 20.4; T = 8192, C = 1024 K1 forward 18.5 / 13.8, K3 backward 26.2 / 23.9, K4
+// forward 25.4 / 23.5; past the line, T = 16384, C = 1024 K1 forward 25.1 /
+// 26.9, K3 backward 49.2 / 51.7, K4 forward 47.9 / 51.7.
 constexpr int64_t kCachedReadBytes = int64_t{80} << 20;
 inline bool stream_reads(int64_t bytes) { return bytes > kCachedReadBytes; }
 

@@ -162,7 +162,7 @@ def test_grad_W_reduce(T, C):
     rn, x, W = _inputs(T, C, 0, 17 * T + C)
     x = x.view(T, nC)
     proj, inv = K.k1_fwd(x, W)
-    go = rn(T, 32)
+    go = _at(rn(T, 32), 0)
     _, gW = K.k1_bwd(go, x, W, proj, inv)
     R, S = O.k1_grad_W(go.cpu(), x.cpu(), inv.cpu())
     check_bf16("grad_W", gW, R, S, T)
