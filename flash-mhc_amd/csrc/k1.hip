@@ -1324,9 +1324,13 @@ int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* 
                int64_t ws_bytes, bool allow_split, int64_t T, int64_t nC, hipStream_t s) {
   const int nc = static_cast<int>(nC);
   if (k1_fwd_mfma_path(nC)) {
-    const K1FwdSplit p = allow_split ? k1_fwd_split(T, nC) : K1FwdSplit{};
+    // Without room for the partial sums, rows off 8 columns or operands off 16
+    // bytes take one pass.
+    const bool room = ws && ws_bytes >= k1_fwd_split_bytes(T, nC) && aligned16(ws);
+    const bool whole = nC % 8 == 0 && aligned16(x_flat) && aligned16(W);
+    const K1FwdSplit p = allow_split && (room || whole) ? k1_fwd_split(T, nC) : K1FwdSplit{};
     if (p.S > 1) {
-      if (!ws || ws_bytes < k1_fwd_split_bytes(T, nC) || !aligned16(ws)) return FMHC_ERR_INVALID_ARGUMENT;
+      if (!room) return FMHC_ERR_INVALID_ARGUMENT;
       float* part = static_cast<float*>(ws);
       const int st = launch_k1_fwd_split(p, x_flat, W, part, T, nc, s);
       if (st != FMHC_OK) return st;
@@ -1518,9 +1522,16 @@ extern "C" int fmhc_k1_bwd(const uint16_t* x_flat, const uint16_t* W, const uint
     return launch_status();
   }
   if (!x_flat || !W || !grad_out || !proj_out || !inv_rms || !grad_x) return FMHC_ERR_INVALID_ARGUMENT;
-  if (k1_bwd_mfma_path(nC, nC)) {
-    const int64_t need = fmhc_k1_bwd_workspace_bytes(T, nC);
-    if (!workspace || workspace_bytes < need || !aligned16(workspace)) return FMHC_ERR_INVALID_ARGUMENT;
+  // Without room for the partial sums, rows off 8 columns or operands off 16
+  // bytes take dx alone and the element-wise grad_W.
+  bool whole = nC % 8 == 0;
+  for (const void* p : {static_cast<const void*>(x_flat), static_cast<const void*>(W), static_cast<const void*>(grad_out),
+                        static_cast<const void*>(proj_out), static_cast<const void*>(inv_rms),
+                        static_cast<const void*>(grad_x)})
+    whole = whole && aligned16(p);
+  const bool room = workspace && workspace_bytes >= fmhc_k1_bwd_workspace_bytes(T, nC) && aligned16(workspace);
+  if (k1_bwd_mfma_path(nC, nC) && (room || whole)) {
+    if (!room) return FMHC_ERR_INVALID_ARGUMENT;
     const BwdSlices sl = bwd_slices(nC, nC);
     const int64_t nruns = k1_bwd_runs(T, sl.n);
     float* partial = static_cast<float*>(workspace);
@@ -1557,8 +1568,9 @@ bool k1_premap_tile(const uint16_t* x, const uint16_t* W, uint16_t* proj, float*
 int k1_fwd_partials(const uint16_t* x_flat, const uint16_t* W, void* ws, int64_t ws_bytes, int64_t T,
                     int64_t nC, hipStream_t s) {
   const K1FwdSplit p = k1_fwd_split(T, nC);
-  if (p.S < 2) return 0;
-  if (!ws || ws_bytes < k1_fwd_split_bytes(T, nC) || !aligned16(ws)) return -FMHC_ERR_INVALID_ARGUMENT;
+  const bool room = ws && ws_bytes >= k1_fwd_split_bytes(T, nC) && aligned16(ws);
+  if (p.S < 2 || (!room && (nC % 8 != 0 || !aligned16(x_flat) || !aligned16(W)))) return 0;
+  if (!room) return -FMHC_ERR_INVALID_ARGUMENT;
   const int st = launch_k1_fwd_split(p, x_flat, W, static_cast<float*>(ws), T, static_cast<int>(nC), s);
   return st == FMHC_OK ? p.S : -st;
 }
@@ -1591,7 +1603,7 @@ int k1_bwd_premap(const uint16_t* x_flat, const uint16_t* W, const uint16_t* gra
     launch_k2_param_reduce(k2_sums, s);
     return launch_status();
   }
-  if (k1_bwd_premap_fused(C)) {
+  if (k1_bwd_premap_fused(C) && (workspace || C % 8 == 0)) {
     if (!workspace || workspace_bytes < k1_bwd_premap_ws_bytes(T, C) || !aligned16(workspace))
       return FMHC_ERR_INVALID_ARGUMENT;
     const BwdSlices sl = bwd_premap_slices(C);

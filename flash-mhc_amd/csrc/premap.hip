@@ -522,7 +522,11 @@ extern "C" int fmhc_premap_bwd(const uint16_t* x, const uint16_t* W, const void*
     if (a < b + bytes && b < a + bytes) return FMHC_ERR_INVALID_ARGUMENT;
   }
   const PremapWs w = premap_ws(T, C);
-  if (T > 0 && (!workspace || workspace_bytes < w.total || !aligned16(workspace))) return FMHC_ERR_INVALID_ARGUMENT;
+  // A workspace without grad_W's partial sums does where C % 8 != 0: those
+  // rows then take K3's backward and K1's element-wise kernels.
+  const bool partials = workspace_bytes >= w.total;
+  if (T > 0 && (!workspace || (!partials && (C % 8 == 0 || workspace_bytes < w.k1)) || !aligned16(workspace)))
+    return FMHC_ERR_INVALID_ARGUMENT;
   char* ws = static_cast<char*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (FMHC_PREMAP_SPLIT && premap_split_ok(x, W, proj, inv_rms, grad_x, grad_layer_input, grad_x_in, T, C)) {
@@ -536,7 +540,7 @@ extern "C" int fmhc_premap_bwd(const uint16_t* x, const uint16_t* W, const void*
   float* gh = T > 0 ? reinterpret_cast<float*>(ws + w.gh) : nullptr;
   uint16_t* gp = T > 0 ? reinterpret_cast<uint16_t*>(ws + w.gp) : nullptr;
   int st = FMHC_OK;
-  const bool fused = T > 0 && k1_bwd_premap_fused(C);
+  const bool fused = T > 0 && partials && k1_bwd_premap_fused(C);
   K2Params P;
   if (!k2_params(alpha_pre, alpha_post, alpha_res, bias, perm, param_dtype, P)) return FMHC_ERR_INVALID_ARGUMENT;
   // K2's backward, whose parameter partials K1's grad_W reduce also sums.
@@ -572,6 +576,6 @@ extern "C" int fmhc_premap_bwd(const uint16_t* x, const uint16_t* W, const void*
   }
   if (st == FMHC_OK)
     st = k1_bwd_premap(x, W, gp, proj, inv_rms, grad_layer_input, h_pre, grad_x_in, grad_x, grad_W,
-                       T > 0 ? ws + w.k1 : nullptr, T > 0 ? w.total - w.k1 : 0, T, C, sums, s);
+                       fused ? ws + w.k1 : nullptr, fused ? w.total - w.k1 : 0, T, C, sums, s);
   return st;
 }

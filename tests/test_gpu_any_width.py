@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from flash_mhc import build_permutation_matrices
+from flash_mhc import _abi
 from flash_mhc import kernels as K
 from oracle import mhc_oracle as O
 from parity import check_bf16, check_fp32, check_rel
@@ -166,3 +167,32 @@ def test_grad_W_reduce(T, C):
     _, gW = K.k1_bwd(go, x, W, proj, inv)
     R, S = O.k1_grad_W(go.cpu(), x.cpu(), inv.cpu())
     check_bf16("grad_W", gW, R, S, T)
+
+
+# Workspaces of the sizes that rows off 8 columns have had (none, and no room
+# for grad_W's partial sums): the calls still run, on other kernels.
+@pytest.mark.parametrize("T,C", [(300, 129), (1037, 131)])
+def test_without_partials(T, C, monkeypatch):
+    nC = 4 * C
+    rn, x, W = _inputs(T, C, 0, 19 * T + C)
+    p = _params(C)
+    go, g_li, g_in = _at(rn(T, 32), 0), _at(rn(T, C), 0), _at(rn(T, 4, C), 0)
+
+    def run():
+        proj, inv = K.k1_fwd(x.view(T, nC), W)
+        li, H, hq, hp, pj, iv = K.premap_fwd(x, W, *p)
+        return (proj, inv, li, H, hq, hp, *K.k1_bwd(go, x.view(T, nC), W, proj, inv),
+                *K.premap_bwd(x, W, *p, hp, pj, iv, g_li, hq, H, g_in))
+
+    want = run()
+    lib = _abi.load()
+    up = lambda n: (n + 255) // 256 * 256
+    small = up(16 * T) + up(64 * T) + up(int(lib.fmhc_k2_bwd_workspace_bytes(T)))
+    assert small < int(lib.fmhc_premap_bwd_workspace_bytes(T, C))
+    for name in ("fmhc_k1_fwd_workspace_bytes", "fmhc_premap_fwd_workspace_bytes", "fmhc_k1_bwd_workspace_bytes"):
+        monkeypatch.setattr(lib, name, lambda *a: 0)
+    monkeypatch.setattr(lib, "fmhc_premap_bwd_workspace_bytes", lambda *a: small)
+    for a, b in zip(run(), want):
+        a, b = a.double(), b.double()
+        # One more bf16 rounding here or there (K1's projection feeds the rest): 2^-8 of each value, 2^-6 of the whole.
+        assert float((a - b).norm()) <= 2.0 ** -6 * float(b.norm())
