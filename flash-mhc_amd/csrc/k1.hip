@@ -1327,7 +1327,7 @@ int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* 
     // Without room for the partial sums, rows off 8 columns or operands off 16
     // bytes take one pass.
     const bool room = ws && ws_bytes >= k1_fwd_split_bytes(T, nC) && aligned16(ws);
-    const bool whole = nC % 8 == 0 && aligned16(x_flat) && aligned16(W);
+    const bool whole = nC % 8 == 0 && aligned16(x_flat) && aligned16(W) && aligned16(out);
     const K1FwdSplit p = allow_split && (room || whole) ? k1_fwd_split(T, nC) : K1FwdSplit{};
     if (p.S > 1) {
       if (!room) return FMHC_ERR_INVALID_ARGUMENT;

@@ -196,3 +196,26 @@ def test_without_partials(T, C, monkeypatch):
         a, b = a.double(), b.double()
         # One more bf16 rounding here or there (K1's projection feeds the rest): 2^-8 of each value, 2^-6 of the whole.
         assert float((a - b).norm()) <= 2.0 ** -6 * float(b.norm())
+
+
+# K1's few-token forward with no workspace: one pass where any of x, W and out
+# is off 16 bytes, as ever; refused, as ever, where all three are aligned.
+@pytest.mark.parametrize("x_off,w_off,out_off", [(1, 0, 0), (0, 1, 0), (0, 0, 1), (0, 0, 0)])
+def test_k1_fwd_without_workspace(x_off, w_off, out_off):
+    T, nC = 64, 1024
+    g = torch.Generator().manual_seed(41)
+    x = _at(torch.randn(T, nC, generator=g).to(BF16), x_off)
+    W = _at((torch.randn(32, nC, generator=g) * 0.02).to(BF16), w_off)
+    out = _at(torch.zeros(T, 32, dtype=BF16), out_off)
+    inv = torch.zeros(T, device=DEV)
+    lib = _abi.load()
+    assert lib.fmhc_k1_fwd_workspace_bytes(T, nC) > 0
+    st = lib.fmhc_k1_fwd_ws(x.data_ptr(), W.data_ptr(), out.data_ptr(), inv.data_ptr(), None, 0, T, nC, 32,
+                            _abi.stream_of(x))
+    if not (x_off or w_off or out_off):
+        assert st == 1
+        return
+    assert st == 0
+    R, S, invR = O.k1_fwd(x.cpu(), W.cpu())
+    check_bf16("proj", out, R, S, nC)
+    check_rel("inv_rms", inv, invR, rtol=4 * nC ** 0.5 * 2.0**-24 + 4 * 2.0**-24)
