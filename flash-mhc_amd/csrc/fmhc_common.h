@@ -426,6 +426,17 @@ constexpr int block_of() {
 // Tokens per workgroup with lpt lanes per token.
 inline int64_t tokens_per_block(int lpt) { return kBlock % lpt == 0 ? kBlock / lpt : 1; }
 
+// f(first token, tokens) over pieces of T tokens whose launches, of `block`
+// threads for per_block tokens, stay below 2^32 threads, the most a HIP launch
+// takes: one piece but for the largest operands (T = 2^25 from C = 520 on, 174
+// GB for K3 forward).  Pieces of whole eights of tokens, so that their rows are
+// aligned as the operands are.
+template <typename F>
+void for_launches(int64_t T, int block, int64_t per_block, F&& f) {
+  const int64_t most = (((int64_t{1} << 32) - 1) / block * per_block) & ~int64_t{7};
+  for (int64_t t = 0; t < T; t += most) f(t, T - t < most ? T - t : most);
+}
+
 // How K3 and K4 walk a row, as compile-time constants: LPT lanes per token,
 // LOOP: several groups per lane, WHOLE: whole, aligned groups, stored with the
 // nontemporal hint, NT: also loaded with it.

@@ -210,22 +210,27 @@ int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t 
   if (C == 2 * 8 * kWave && T >= 16384 && aligned16(x) && aligned16(out)) {
     using Walk = RowWalk<kWave, true, true, true>;
     static const unsigned lds = lds_reserve(reinterpret_cast<const void*>(&k3_fwd_kernel<Walk>), kLdsCapSix);
-    k3_fwd_kernel<Walk><<<dim3(blocks_for(T, tokens_per_block(kWave))), block_of<kWave>(), FMHC_LDS_CAP ? lds : 0u,
-                          s>>>(x, h_pre, out, T, C);
+    for_launches(T, block_of<kWave>(), tokens_per_block(kWave), [&](int64_t t, int64_t n) {
+      k3_fwd_kernel<Walk><<<dim3(blocks_for(n, tokens_per_block(kWave))), block_of<kWave>(), FMHC_LDS_CAP ? lds : 0u,
+                            s>>>(x + t * 4 * C, h_pre + t * 4, out + t * C, n, C);
+    });
     return launch_status();
   }
   with_row_walk(C, aligned16(x) && aligned16(out), T * C * 8, [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
-    const dim3 grid(blocks_for(T, tokens_per_block(L)));
     // Residency cap (fmhc_common.h).
     static const unsigned own = own_lds(reinterpret_cast<const void*>(&k3_fwd_kernel<Walk>));
-    unsigned lds = 0;
-    if (Walk::LOOP)
-      lds = kLdsCapSix;
-    else if (Walk::WHOLE && 4 * (C / 8) >= 3 * L)
-      lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
-    k3_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(x, h_pre, out, T, C);
+    for_launches(T, block_of<L>(), tokens_per_block(L), [&](int64_t t, int64_t n) {
+      const dim3 grid(blocks_for(n, tokens_per_block(L)));
+      unsigned lds = 0;
+      if (Walk::LOOP)
+        lds = kLdsCapSix;
+      else if (Walk::WHOLE && 4 * (C / 8) >= 3 * L)
+        lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+      k3_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(x + t * 4 * C, h_pre + t * 4,
+                                                                              out + t * C, n, C);
+    });
   });
   return launch_status();
 }
@@ -236,15 +241,18 @@ int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uin
   const bool canon = k3_canon(C, lanes_per_token(C));
   with_row_walk(C, aligned16(x) && aligned16(go) && aligned16(grad_x), T * C * 10, [&](auto w) {
     constexpr int L = decltype(w)::LPT;
-    const dim3 grid(blocks_for(T, tokens_per_block(L)));
     auto launch = [&](auto walk, auto canon_c) {
       using Walk = decltype(walk);
       constexpr bool CANON = decltype(canon_c)::value;
       // Residency cap (fmhc_common.h): with grad_x and one group per lane.
       static const unsigned own = own_lds(reinterpret_cast<const void*>(&k3_bwd_kernel<Walk, GX, CANON>));
-      unsigned lds = 0;
-      if (GX && FMHC_LDS_CAP && !Walk::LOOP) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
-      k3_bwd_kernel<Walk, GX, CANON><<<grid, block_of<L>(), lds, s>>>(x, h_pre, go, grad_x, grad_h_pre, T, C);
+      for_launches(T, block_of<L>(), tokens_per_block(L), [&](int64_t t, int64_t n) {
+        const dim3 grid(blocks_for(n, tokens_per_block(L)));
+        unsigned lds = 0;
+        if (GX && FMHC_LDS_CAP && !Walk::LOOP) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+        k3_bwd_kernel<Walk, GX, CANON><<<grid, block_of<L>(), lds, s>>>(
+            x + t * 4 * C, h_pre + t * 4, go + t * C, GX ? grad_x + t * 4 * C : nullptr, grad_h_pre + t * 4, n, C);
+      });
     };
     if constexpr (L >= 16) {
       if (canon) return launch(w, std::true_type{});

@@ -262,15 +262,18 @@ int launch_k4_fwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
     // Tokens narrower than a wave are faster in the loop's schedule (T = 65536,
     // C = 176 42.7 -> 36.5 us, 256 50.5 -> 48.6); wider ones equal or slower.
     using Walk = RowWalk<L, decltype(w)::LOOP || L < kWave, decltype(w)::WHOLE, decltype(w)::NT>;
-    const dim3 grid(blocks_for(T, tokens_per_block(L)));
     // Residency cap (fmhc_common.h).
     static const unsigned own = own_lds(reinterpret_cast<const void*>(&k4_fwd_kernel<Walk>));
-    unsigned lds = 0;
-    if (decltype(w)::LOOP)
-      lds = grid.x >= kCapMinBlocks ? kLdsCapFive : 0u;
-    else
-      lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
-    k4_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(x, lo, H, hp, out, T, C);
+    for_launches(T, block_of<L>(), tokens_per_block(L), [&](int64_t t, int64_t n) {
+      const dim3 grid(blocks_for(n, tokens_per_block(L)));
+      unsigned lds = 0;
+      if (decltype(w)::LOOP)
+        lds = grid.x >= kCapMinBlocks ? kLdsCapFive : 0u;
+      else
+        lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+      k4_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(
+          x + t * 4 * C, lo + t * C, H + t * 16, hp + t * 4, out + t * 4 * C, n, C);
+    });
   });
   return launch_status();
 }
@@ -289,16 +292,20 @@ int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
   with_row_walk(C, aligned, 2 * (T * C * 18), [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
-    const dim3 grid(blocks_for(T, tokens_per_block(L)));
     auto launch = [&](auto walk, auto early) {
       using W = decltype(walk);
       constexpr bool E = decltype(early)::value;
       // Residency cap (fmhc_common.h) with one group per lane, up to 256 lanes
       // (T = 30000, C = 3000 440 us with and without).
       static const unsigned own = own_lds(reinterpret_cast<const void*>(&k4_bwd_kernel<W, E>));
-      unsigned lds = 0;
-      if (FMHC_LDS_CAP && C / 8 <= L && L <= 256) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
-      k4_bwd_kernel<W, E><<<grid, block_of<L>(), lds, s>>>(x, lo, H, hp, go, gx, glo, gH, ghp, T, C);
+      for_launches(T, block_of<L>(), tokens_per_block(L), [&](int64_t t, int64_t n) {
+        const dim3 grid(blocks_for(n, tokens_per_block(L)));
+        unsigned lds = 0;
+        if (FMHC_LDS_CAP && C / 8 <= L && L <= 256) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+        k4_bwd_kernel<W, E><<<grid, block_of<L>(), lds, s>>>(
+            x + t * 4 * C, lo + t * C, H + t * 16, hp + t * 4, go + t * 4 * C, gx + t * 4 * C, glo + t * C,
+            gH + t * 16, ghp + t * 4, n, C);
+      });
     };
     // EARLY: all of a lane's loads go out before its first store, so a wave
     // waits for one round trip instead of five, but holds more registers and
