@@ -1343,10 +1343,21 @@ int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* 
       launch_k1_fwd_onepass<false, false, false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     }
   } else {
-    const dim3 grid(blocks_for(T, 4));
-    k1_fwd_scalar<<<grid, 256, 0, s>>>(x_flat, W, out, inv_rms, T, nc);
+    for_launches(T, 256, 4, [&](int64_t t, int64_t n) {
+      k1_fwd_scalar<<<dim3(blocks_for(n, 4)), 256, 0, s>>>(x_flat + t * nC, W, out + t * kDout, inv_rms + t, n, nc);
+    });
   }
   return launch_status();
+}
+
+template <bool ACC>
+void launch_k1_bwd_scalar(hipStream_t s, const uint16_t* x, const uint16_t* W, const uint16_t* go, const uint16_t* proj,
+                          const float* inv_rms, uint16_t* gx, const uint16_t* gi, int64_t T, int nC) {
+  for_launches(T, 256, 4, [&](int64_t t, int64_t n) {
+    k1_bwd_scalar<ACC><<<dim3(blocks_for(n, 4)), 256, 0, s>>>(x + t * nC, W, go + t * kDout, proj + t * kDout,
+                                                              inv_rms + t, gx + t * nC, gi ? gi + t * nC : nullptr, n,
+                                                              nC);
+  });
 }
 
 // Number of runs of k1_bwd_mfma for T tokens (nblocks blocks of 16) and
@@ -1452,8 +1463,7 @@ extern "C" int fmhc_k1_bwd_dx(const uint16_t* x_flat, const uint16_t* W, const u
     const int64_t nruns = k1_bwd_nruns(T, sl.n, kBwdNTB, 1);
     launch_k1_bwd_mfma<false>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, nullptr, T, nc, sl, nruns);
   } else {
-    const dim3 grid(blocks_for(T, 4));
-    k1_bwd_scalar<false><<<grid, 256, 0, s>>>(x_flat, W, grad_out, proj_out, inv_rms, grad_x, nullptr, T, nc);
+    launch_k1_bwd_scalar<false>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, nullptr, T, nc);
   }
   return launch_status();
 }
@@ -1619,8 +1629,7 @@ int k1_bwd_premap(const uint16_t* x_flat, const uint16_t* W, const uint16_t* gra
     if (st != FMHC_OK) return st;
     return launch_dw_reduce(partial, grad_W, nruns, sl, nc, k2_sums, kNPar, s);
   }
-  k1_bwd_scalar<true><<<dim3(blocks_for(T, 4)), 256, 0, s>>>(x_flat, W, grad_proj, proj, inv_rms, grad_x,
-                                                             grad_x_in, T, nc);
+  launch_k1_bwd_scalar<true>(s, x_flat, W, grad_proj, proj, inv_rms, grad_x, grad_x_in, T, nc);
   const int st = launch_status();
   if (st != FMHC_OK) return st;
   k1_dw_scalar<<<dim3(blocks_for(static_cast<int64_t>(kDout) * nC, 256)), 256, 0, s>>>(

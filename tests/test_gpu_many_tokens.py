@@ -1,6 +1,7 @@
-"""K3 and K4 for more tokens than one launch can hold: a HIP launch stays below
-2^32 threads, eight lanes per token at C = 1 reach that at T = 2^29, and the
-entry points then launch pieces of the tokens.  Every output element must be
+"""K3, K4 and element-wise K1 for more tokens than one launch can hold: a HIP
+launch stays below 2^32 threads, which K3's and K4's eight lanes per token at
+C = 1 reach at T = 2^29 and element-wise K1's 64 (rows of fewer than eight
+columns) at T = 2^26, and the entry points then launch pieces of the tokens.  Every output element must be
 written, and tokens at the ends and around the seam must have the bits of a
 call on those tokens alone."""
 
@@ -29,11 +30,11 @@ def _nan(*shape, dtype=BF16):
     return torch.full(shape, float("nan"), device=DEV, dtype=dtype)
 
 
-def _check(outs, alone):
+def _check(outs, alone, windows=WINDOWS):
     for o in outs:
         for piece in o.view(-1).split(1 << 28):
             assert not bool(torch.isnan(piece).any())
-    for w in WINDOWS:
+    for w in windows:
         for o, want in zip(outs, alone(w)):
             assert torch.equal(o[w], want), w
 
@@ -61,3 +62,16 @@ def test_pieces(kernel):
             _check(outs, lambda w: K.k4_bwd(go[w], x[w], lo[w], H[w], h[w]))
     del x, h
     torch.cuda.empty_cache()
+
+
+def test_element_wise_k1():
+    tokens, nC = (1 << 26) + 40, 7
+    seam = ((1 << 32) - 1) // 256 * 4 & ~7
+    assert 0 < tokens - seam < 128
+    windows = [slice(0, 90), slice(seam - 64, seam + 32), slice(tokens - 90, tokens)]
+    x, W, go = _rand(tokens, nC), _rand(32, nC), _rand(tokens, 32)
+    outs = K.k1_fwd(x, W, out=_nan(tokens, 32), inv_rms=_nan(tokens, dtype=torch.float32))
+    _check(outs, lambda w: K.k1_fwd(x[w], W), windows)
+    proj, inv = outs
+    gx = K.k1_bwd_dx(go, x, W, proj, inv, grad_x=_nan(tokens, nC))
+    _check([gx], lambda w: [K.k1_bwd_dx(go[w], x[w], W, proj[w], inv[w])], windows)
