@@ -1458,7 +1458,10 @@ extern "C" int fmhc_k1_bwd_dx(const uint16_t* x_flat, const uint16_t* W, const u
     return FMHC_ERR_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int nc = static_cast<int>(nC);
-  if (k1_bwd_mfma_path(nC, nC)) {
+  // In place (grad_x is x_flat) rows off 8 columns run element-wise: the
+  // matrix-core kernel's last lane re-reads up to 7 columns that the wave of
+  // the slice before it writes, and writes them again.
+  if (k1_bwd_mfma_path(nC, nC) && (nC % 8 == 0 || grad_x != x_flat)) {
     const BwdSlices sl = bwd_slices(nC, nC);
     const int64_t nruns = k1_bwd_nruns(T, sl.n, kBwdNTB, 1);
     launch_k1_bwd_mfma<false>(s, x_flat, W, grad_out, proj_out, inv_rms, grad_x, nullptr, T, nc, sl, nruns);

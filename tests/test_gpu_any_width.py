@@ -219,3 +219,18 @@ def test_k1_fwd_without_workspace(x_off, w_off, out_off):
     R, S, invR = O.k1_fwd(x.cpu(), W.cpu())
     check_bf16("proj", out, R, S, nC)
     check_rel("inv_rms", inv, invR, rtol=4 * nC ** 0.5 * 2.0**-24 + 4 * 2.0**-24)
+
+
+# grad_x written over x: 1, 4 and 7 columns past a 128-column slice, whose last
+# lane shares columns with the slice before; whole groups beside them.
+@pytest.mark.parametrize("T,nC", [(3000, 129), (3000, 132), (700, 1031), (700, 1024), (300, 136), (40, 9)])
+def test_k1_bwd_dx_in_place(T, nC):
+    g = torch.Generator().manual_seed(T + nC)
+    x = torch.randn(T, nC, generator=g).to(BF16).to(DEV)
+    W = (torch.randn(32, nC, generator=g) * 0.02).to(BF16).to(DEV)
+    go = torch.randn(T, 32, generator=g).to(BF16).to(DEV)
+    proj, inv = K.k1_fwd(x, W)
+    R, S = O.k1_bwd_dx(go.cpu(), x.cpu(), W.cpu(), proj.cpu(), inv.cpu())
+    got = K.k1_bwd_dx(go, x, W, proj, inv, grad_x=x)
+    assert got.data_ptr() == x.data_ptr()
+    check_bf16("grad_x", got, R, S, 64)
