@@ -90,20 +90,16 @@ __device__ __forceinline__ void st8_stream(void* p, u32x2 v) {
 #endif
 }
 
-// Loads carry the hint in launches that read more than fits the memory-side
-// cache (256 MB) along with what the launch before it wrote and read.  Below
-// that, x and its gradients are read again by the next kernel of a step, and
-// lines loaded under the hint are not kept for it: ordinary loads win where an
-// earlier launch touched the operands, and lose 2-5% where none did, from HBM.
-// Stores keep the hint at every size (without it T = 1024, C = 1024 K4 backward
-// 8.0 -> 8.9 us, K4 forward 4.3 -> 5.1).  With the hint against without, three
-// sets of operands in turn, us: T = 1003, C = 2560 K1 backward 24.1 / 19.1, K3
-// forward 6.2 / 5.9, K4 forward 9.5 / 8.9; T = 4096, C = 1024 K1 backward 25.9 /
-// 20.4; T = 8192, C = 1024 K1 forward 18.5 / 13.8, K3 backward 26.2 / 23.9, K4
-// forward 25.4 / 23.5; past the line, T = 16384, C = 1024 K1 forward 25.1 /
-// 26.9, K3 backward 49.2 / 51.7, K4 forward 47.9 / 51.7.
-constexpr int64_t kCachedReadBytes = int64_t{80} << 20;
-inline bool stream_reads(int64_t bytes) { return bytes > kCachedReadBytes; }
+// Loads carry the hint at every size.  Without it launches that read up to 80
+// MiB were faster where the same few tensors came round again and stayed in the
+// memory-side cache (hint / none, us: forward of T = 1003, C = 2560 51.9 / 50.3,
+// training step of T = 4096, C = 1024 163 / 160 replayed on one state), and
+// slower on new tensors and inside a stack of blocks: T = 8192, C = 1024 K1
+// forward 18.4 / 18.9, K3 forward 15.9 / 16.5, K3 backward 25.9 / 26.8, K4
+// forward 25.6 / 26.6, K1 forward then backward 54.5 / 58.8; forward of T = 8192
+// 77 / 80; per block of a six-block training step T = 8192 262 / 267, T = 1003,
+// C = 2560 164.5 / 168.6.  Kernels that read again what the launch before them
+// or their own first pass has read take ordinary loads (premap.hip, k1.hip).
 
 // bf16 bit pattern -> fp32 (exact).
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
@@ -438,19 +434,16 @@ void for_launches(int64_t T, int block, int64_t per_block, F&& f) {
 }
 
 // How K3 and K4 walk a row, as compile-time constants: LPT lanes per token,
-// LOOP: several groups per lane, WHOLE: whole, aligned groups, stored with the
-// nontemporal hint, NT: also loaded with it.
-template <int kLpt, bool kLoop, bool kWhole, bool kNt>
+// LOOP: several groups per lane, WHOLE: whole, aligned groups, loaded and
+// stored with the nontemporal hint.
+template <int kLpt, bool kLoop, bool kWhole>
 struct RowWalk {
   static constexpr int LPT = kLpt;
   static constexpr bool LOOP = kLoop;
   static constexpr bool WHOLE = kWhole;
-  static constexpr bool NT = kNt;
-  static_assert(WHOLE || !NT, "unaligned groups are loaded without the hint");
 };
 
-// f(RowWalk) for rows of C columns whose 16-byte groups are aligned or not, in
-// a launch that reads `reads` bytes (stream_reads).
+// f(RowWalk) for rows of C columns whose 16-byte groups are aligned or not.
 // Unaligned groups (C % 8 != 0, or a base address off 16 bytes) leave out the
 // nontemporal hint: neighbouring lanes' groups share lines, and the hint
 // makes each access fetch or write its part on its own (K3 forward / backward,
@@ -458,30 +451,28 @@ struct RowWalk {
 // 17.5 / 32.0 / 32.5 / 53.4 against 11.8 / 24.0 / 24.7 / 45.1; T = 20011,
 // C = 300 14.3 / 24.0 / 23.8 / 42.5 against 12.1 / 19.3 / 19.9 / 38.3).
 template <typename F>
-void with_row_walk(int C, bool aligned, int64_t reads, F&& f) {
-  auto pick = [&](auto whole, auto nt) {
-    constexpr bool WHOLE = decltype(whole)::value, NT = decltype(nt)::value;
+void with_row_walk(int C, bool aligned, F&& f) {
+  auto pick = [&](auto whole) {
+    constexpr bool WHOLE = decltype(whole)::value;
     const int lpt = lanes_per_token(C);
-    if (C / 8 > lpt) return f(RowWalk<kLoopLpt, true, WHOLE, NT>{});
+    if (C / 8 > lpt) return f(RowWalk<kLoopLpt, true, WHOLE>{});
     switch (lpt) {
-      case 448: return f(RowWalk<448, false, WHOLE, NT>{});
-      case 384: return f(RowWalk<384, false, WHOLE, NT>{});
-      case 320: return f(RowWalk<320, false, WHOLE, NT>{});
-      case 256: return f(RowWalk<256, false, WHOLE, NT>{});
-      case 192: return f(RowWalk<192, false, WHOLE, NT>{});
-      case 128: return f(RowWalk<128, false, WHOLE, NT>{});
-      case 64: return f(RowWalk<64, false, WHOLE, NT>{});
-      case 32: return f(RowWalk<32, false, WHOLE, NT>{});
-      case 16: return f(RowWalk<16, false, WHOLE, NT>{});
-      default: return f(RowWalk<8, false, WHOLE, NT>{});
+      case 448: return f(RowWalk<448, false, WHOLE>{});
+      case 384: return f(RowWalk<384, false, WHOLE>{});
+      case 320: return f(RowWalk<320, false, WHOLE>{});
+      case 256: return f(RowWalk<256, false, WHOLE>{});
+      case 192: return f(RowWalk<192, false, WHOLE>{});
+      case 128: return f(RowWalk<128, false, WHOLE>{});
+      case 64: return f(RowWalk<64, false, WHOLE>{});
+      case 32: return f(RowWalk<32, false, WHOLE>{});
+      case 16: return f(RowWalk<16, false, WHOLE>{});
+      default: return f(RowWalk<8, false, WHOLE>{});
     }
   };
   if (!aligned || C % 8 != 0)
-    pick(std::false_type{}, std::false_type{});
-  else if (stream_reads(reads))
-    pick(std::true_type{}, std::true_type{});
+    pick(std::false_type{});
   else
-    pick(std::true_type{}, std::false_type{});
+    pick(std::true_type{});
 }
 
 // Token of a lane.  LPT <= 64: 64 / LPT tokens per wave; wider: LPT / 64 waves

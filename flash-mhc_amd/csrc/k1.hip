@@ -201,7 +201,7 @@ __device__ __forceinline__ void k3_narrow_tokens(const uint16_t* __restrict__ x,
 // streams into the layer input while L2 and the memory-side cache may still
 // hold the rows it just read (its x loads are ordinary loads, which allocate
 // there).  Same values as K1 -> K2 -> K3 launched separately.
-// NT: x's loads carry the nontemporal hint (plain kernel, stream_reads).
+// NT: x's loads carry the nontemporal hint (plain kernel, rows of whole lines).
 // WHOLE: rows of whole 128-byte lines (the plain kernel), of whole aligned
 // 16-byte groups and more than kNarrowC columns (TILE), or of whole groups
 // (SPLITK); otherwise x is loaded without the nontemporal hint, the last group
@@ -275,9 +275,9 @@ __global__ __launch_bounds__(kWave * SPLIT) void k1_fwd_mfma(const uint16_t* __r
   // concurrent reads of all workgroups over the DRAM channels instead of every
   // workgroup hitting the same column of its 8 KiB-strided rows), and keeps
   // three chunks in flight: the next two chunks' fragments are loaded while
-  // the MFMAs of the current one run.  x is read once per launch; NT: its loads carry
-  // the nontemporal hint (launches past kCachedReadBytes, 8-10% faster there than
-  // ordinary loads).  With SPLITK (few tokens) they do not: the pre-map's few-token kernel reads the same x
+  // the MFMAs of the current one run.  x is read once per launch, so with NT its loads
+  // carry the nontemporal hint (8-10% faster than ordinary loads at T = 65536,
+  // C = 1024).  With SPLITK (few tokens) they do not: the pre-map's few-token kernel reads the same x
   // again right after, from the caches.  With SPLITK the workgroup's chunks
   // are cbeg .. cbeg + nfull - 1 (no rotation: the workgroups of one token
   // block already cover different columns), and only the last split takes the
@@ -1335,10 +1335,8 @@ int k1_fwd_run(const uint16_t* x_flat, const uint16_t* W, uint16_t* out, float* 
       const int st = launch_k1_fwd_split(p, x_flat, W, part, T, nc, s);
       if (st != FMHC_OK) return st;
       k1_fwd_finish<<<dim3(blocks_for(T, 4)), 256, 0, s>>>(part, out, inv_rms, T, nc, p.S);
-    } else if (nC % 64 == 0 && aligned16(x_flat) && stream_reads(2 * T * nC)) {
-      launch_k1_fwd_onepass<false, true, true>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     } else if (nC % 64 == 0 && aligned16(x_flat)) {
-      launch_k1_fwd_onepass<false, true, false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
+      launch_k1_fwd_onepass<false, true, true>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     } else {
       launch_k1_fwd_onepass<false, false, false>(k1_fwd_blocks(T), x_flat, W, out, inv_rms, T, nc, PremapTile{}, s);
     }
@@ -1401,24 +1399,20 @@ void launch_k1_bwd_mfma(hipStream_t s, const uint16_t* x, const uint16_t* W, con
     k1_bwd_mfma<DW, FULLK, EPI, GI, NT, nbuf><<<grid, 256, cap ? lds : 0u, s>>>(
         x, W, go, proj, inv_rms, gx, partial, go3, h_pre, gi, T, nC, sl, nruns, C);
   };
-  // x, the incoming gradient and the layer input's gradient (stream_reads).
-  // With grad_W alone, rows off 128-byte lines also take the ordinary loads at
-  // any size: lines that two runs' rows share are then fetched once (T =
-  // 32768, C = 1023 155 -> 143 us, T = 50000, C = 2049 483 -> 444); dx alone
-  // there is equal, and the pre-map's kernel loses 2% (T = 30011, C = 1001).
-  const bool lines = nC % 64 == 0 && aligned16(x);
-  const bool nt = stream_reads(T * nC * (GI ? 4 : 2) + (EPI ? T * C * 2 : 0)) && (lines || !DW || EPI);
-  if (sl.len % 128 == 0) {
-    if (nt)
-      launch(std::true_type{}, std::true_type{});
-    else
-      launch(std::true_type{}, std::false_type{});
-  } else {
-    if (nt)
-      launch(std::false_type{}, std::true_type{});
-    else
-      launch(std::false_type{}, std::false_type{});
+  auto rows = [&](auto nt) {
+    sl.len % 128 == 0 ? launch(std::true_type{}, nt) : launch(std::false_type{}, nt);
+  };
+  // x and the incoming gradient carry the nontemporal hint, except with grad_W
+  // at rows off 128-byte lines: lines that two runs' rows share are then fetched
+  // once (hint / none, us: T = 32768, C = 1023 155 / 143, T = 50000, C = 2049 483 /
+  // 444; pre-map backward T = 20011, C = 300 70.0 / 67.6, T = 65536, C = 100 77.8 /
+  // 75.5, C = 1000 480 / 473, T = 3000, C = 999 47.3 / 45.9; the hint is better at
+  // T = 30011, C = 1001 267.7 / 272.7 and T = 4000, C = 100 27.7 / 29.1).  dx alone
+  // is equal.
+  if constexpr (DW) {
+    if (nC % 64 != 0 || !aligned16(x)) return rows(std::false_type{});
   }
+  rows(std::true_type{});
 }
 
 }  // namespace

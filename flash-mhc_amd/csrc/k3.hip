@@ -30,7 +30,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_fwd_kernel(const uin
                                                         uint16_t* __restrict__ out,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
   if (tok >= T) return;
@@ -39,10 +39,10 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_fwd_kernel(const uin
   const float h[4] = {hp[0], hp[1], hp[2], hp[3]};
   const uint16_t* x0 = x + tok * 4 * C;
   if constexpr (!LOOP) {
-    if (sub < C / 8) k3_mix<8, WHOLE, NT>(x0, h, out + tok * C, sub, C);
-    row_tail<WHOLE>(C, sub, [&](int c) { k3_mix<1, WHOLE, NT>(x0, h, out + tok * C, c, C); });
+    if (sub < C / 8) k3_mix<8, WHOLE>(x0, h, out + tok * C, sub, C);
+    row_tail<WHOLE>(C, sub, [&](int c) { k3_mix<1, WHOLE>(x0, h, out + tok * C, c, C); });
   } else {
-    k3_token<WHOLE, NT>(x0, h, out + tok * C, sub, LPT, C);
+    k3_token<WHOLE>(x0, h, out + tok * C, sub, LPT, C);
   }
 }
 
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_bwd_kernel(const uin
                                                         float* __restrict__ grad_h_pre,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE;
   static_assert(!CANON || LPT >= 16, "slice order: whole 16-lane rows");
   constexpr int WPT = LPT > kWave ? LPT / kWave : 1;  // waves per token
   const int lane = threadIdx.x & (kWave - 1);
@@ -96,11 +96,11 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_bwd_kernel(const uin
   auto round = [&](auto vec, int g, float (&acc)[4]) __attribute__((always_inline)) {
     constexpr int VEC = decltype(vec)::value;
     float q[VEC], a[VEC], b[VEC], c[VEC], d[VEC], o[VEC];
-    Lanes<VEC, NT>::load(grow, g, q);
-    Lanes<VEC, NT>::load(x0, g, a);
-    Lanes<VEC, NT>::load(x1, g, b);
-    Lanes<VEC, NT>::load(x2, g, c);
-    Lanes<VEC, NT>::load(x3, g, d);
+    Lanes<VEC, WHOLE>::load(grow, g, q);
+    Lanes<VEC, WHOLE>::load(x0, g, a);
+    Lanes<VEC, WHOLE>::load(x1, g, b);
+    Lanes<VEC, WHOLE>::load(x2, g, c);
+    Lanes<VEC, WHOLE>::load(x3, g, d);
     if constexpr (GX) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[e] = h0 * q[e];
@@ -208,7 +208,7 @@ int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t 
   // workgroups per CU (T = 65536 104.5 us, against 106.3 with 128 lanes; with
   // few tokens 128 lanes: T = 4096 9.8 -> 8.8 us).
   if (C == 2 * 8 * kWave && T >= 16384 && aligned16(x) && aligned16(out)) {
-    using Walk = RowWalk<kWave, true, true, true>;
+    using Walk = RowWalk<kWave, true, true>;
     static const unsigned lds = lds_reserve(reinterpret_cast<const void*>(&k3_fwd_kernel<Walk>), kLdsCapSix);
     for_launches(T, block_of<kWave>(), tokens_per_block(kWave), [&](int64_t t, int64_t n) {
       k3_fwd_kernel<Walk><<<dim3(blocks_for(n, tokens_per_block(kWave))), block_of<kWave>(), FMHC_LDS_CAP ? lds : 0u,
@@ -216,7 +216,7 @@ int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t 
     });
     return launch_status();
   }
-  with_row_walk(C, aligned16(x) && aligned16(out), T * C * 8, [&](auto w) {
+  with_row_walk(C, aligned16(x) && aligned16(out), [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
     // Residency cap (fmhc_common.h).
@@ -239,7 +239,7 @@ template <bool GX>
 int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uint16_t* grad_x,
                   float* grad_h_pre, int64_t T, int C, hipStream_t s) {
   const bool canon = k3_canon(C, lanes_per_token(C));
-  with_row_walk(C, aligned16(x) && aligned16(go) && aligned16(grad_x), T * C * 10, [&](auto w) {
+  with_row_walk(C, aligned16(x) && aligned16(go) && aligned16(grad_x), [&](auto w) {
     constexpr int L = decltype(w)::LPT;
     auto launch = [&](auto walk, auto canon_c) {
       using Walk = decltype(walk);
@@ -261,7 +261,7 @@ int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uin
     // loop's schedule (T = 65536, C = 100 25.7 -> 23.2 us, C = 250 51.2 -> 49.7,
     // T = 100000, C = 60 24.7 -> 23.3).
     if constexpr (GX && L < kWave)
-      launch(RowWalk<L, true, decltype(w)::WHOLE, decltype(w)::NT>{}, std::false_type{});
+      launch(RowWalk<L, true, decltype(w)::WHOLE>{}, std::false_type{});
     else
       launch(w, std::false_type{});
   });

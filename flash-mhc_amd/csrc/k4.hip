@@ -30,7 +30,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_fwd_kernel(const uin
                                                         uint16_t* __restrict__ out,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
   if (tok >= T) return;
@@ -62,9 +62,9 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_fwd_kernel(const uin
   auto mix = [&](auto vec, int g) __attribute__((always_inline)) {
     constexpr int VEC = decltype(vec)::value;
     float l[VEC], xv[4][VEC];
-    Lanes<VEC, NT>::load(lrow, g, l);
+    Lanes<VEC, WHOLE>::load(lrow, g, l);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) Lanes<VEC, NT>::load(xr[j], g, xv[j]);
+    for (int j = 0; j < 4; ++j) Lanes<VEC, WHOLE>::load(xr[j], g, xv[j]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float o[VEC];
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
                                                         float* __restrict__ grad_hp,
                                                         int64_t T, int C) {
   constexpr int LPT = WALK::LPT;
-  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE, NT = WALK::NT;
+  constexpr bool LOOP = WALK::LOOP, WHOLE = WALK::WHOLE;
   constexpr int WPT = LPT > kWave ? LPT / kWave : 1;  // waves per token
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t tok = token_of_lane<LPT>(lane);
@@ -149,15 +149,15 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
     constexpr int VEC = decltype(vec)::value;
     float q[4][VEC], l[VEC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) Lanes<VEC, NT>::load(gr[i], g, q[i]);
-    Lanes<VEC, NT>::load(lrow, g, l);
+    for (int i = 0; i < 4; ++i) Lanes<VEC, WHOLE>::load(gr[i], g, q[i]);
+    Lanes<VEC, WHOLE>::load(lrow, g, l);
 
     // EARLY: the iteration's x rows load with grad_out and lo, before its
     // first store (the compiler keeps a load behind an earlier store).
     float xs[EARLY ? 4 : 1][VEC];
     if constexpr (EARLY) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) Lanes<VEC, NT>::load(xr[j], g, xs[j]);
+      for (int j = 0; j < 4; ++j) Lanes<VEC, WHOLE>::load(xr[j], g, xs[j]);
     }
     // grad_lo and the grad_h_post partial sums.
     {
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
       if constexpr (EARLY)
         xv = xs[j];
       else
-        Lanes<VEC, NT>::load(xr[j], g, xl);
+        Lanes<VEC, WHOLE>::load(xr[j], g, xl);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -257,11 +257,11 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k4_bwd_kernel(const uin
 
 int launch_k4_fwd(const uint16_t* x, const uint16_t* lo, const float* H, const float* hp,
                   uint16_t* out, int64_t T, int C, hipStream_t s) {
-  with_row_walk(C, aligned16(x) && aligned16(lo) && aligned16(out), T * C * 10, [&](auto w) {
+  with_row_walk(C, aligned16(x) && aligned16(lo) && aligned16(out), [&](auto w) {
     constexpr int L = decltype(w)::LPT;
     // Tokens narrower than a wave are faster in the loop's schedule (T = 65536,
     // C = 176 42.7 -> 36.5 us, 256 50.5 -> 48.6); wider ones equal or slower.
-    using Walk = RowWalk<L, decltype(w)::LOOP || L < kWave, decltype(w)::WHOLE, decltype(w)::NT>;
+    using Walk = RowWalk<L, decltype(w)::LOOP || L < kWave, decltype(w)::WHOLE>;
     // Residency cap (fmhc_common.h).
     static const unsigned own = own_lds(reinterpret_cast<const void*>(&k4_fwd_kernel<Walk>));
     for_launches(T, block_of<L>(), tokens_per_block(L), [&](int64_t t, int64_t n) {
@@ -284,12 +284,7 @@ int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
                   const uint16_t* go, uint16_t* gx, uint16_t* glo, float* gH, float* ghp,
                   int64_t T, int C, hipStream_t s) {
   const bool aligned = aligned16(x) && aligned16(lo) && aligned16(go) && aligned16(gx) && aligned16(glo);
-  // Twice the bytes it reads: grad_out is new and x was last read before the
-  // layer, so ordinary loads win only where all of a step's tensors stay
-  // cached (training step, us, hint against none: T = 2048, C = 1024 113.3 /
-  // 111.8, T = 3000 145.5 / 149.5, T = 4096 160.9 / 163.3, T = 1003, C = 2560
-  // 174 / 178).
-  with_row_walk(C, aligned, 2 * (T * C * 18), [&](auto w) {
+  with_row_walk(C, aligned, [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
     auto launch = [&](auto walk, auto early) {
@@ -321,7 +316,7 @@ int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
     else if (!Walk::WHOLE || T * L <= kK4EarlyLanes)
       launch(w, std::true_type{});
     else
-      launch(RowWalk<L, true, Walk::WHOLE, Walk::NT>{}, std::false_type{});
+      launch(RowWalk<L, true, Walk::WHOLE>{}, std::false_type{});
   });
   return launch_status();
 }

@@ -1,7 +1,8 @@
-"""Both load policies of K1, K3 and K4: launches that read more than
-kCachedReadBytes (fmhc_common.h; K4 backward half as much) carry the
-nontemporal hint, smaller ones do not.  The hint changes no arithmetic, so a launch one token block past the line
-must give, for the tokens the two share, the bits of a launch on the line.
+"""A token's outputs do not depend on how many tokens a launch has: K1, K3 and
+K4 and the pre-map backward at two token counts, one block of 16 tokens and a
+ragged one apart, at sizes where a launch reads about as much as stays in the
+memory-side cache (80 MiB of the 256).  For the tokens the two share, the larger
+launch must give the bits of the smaller one.
 """
 
 from __future__ import annotations
