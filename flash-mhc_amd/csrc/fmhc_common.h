@@ -255,10 +255,14 @@ inline unsigned lds_reserve(const void* kernel, unsigned dyn) {
 }
 
 constexpr int kCapLanes = 680;
-// Unaligned groups keep more waves in flight (T = 30011, C = 1001, no cap / 1150
-// / 680 lanes: K3 backward 105 / 96 / 97, K4 forward 103 / 96 / 95, K4 backward
-// 157 / 154 / 153; T = 50000, C = 700 off 16 bytes 122 / 127 / 137, 120 / 126 /
-// 134, 197 / 206 / 223); K3 forward 52 / 55 / 58 there and takes none.
+// Unaligned groups keep more waves in flight.  No cap against this one, us, K3
+// backward, K4 forward: T = 30011, C = 1001 102 / 94, 104 / 97; T = 50000, C = 700
+// off 16 bytes 122 / 119, 120 / 118; T = 40000, C = 777 105 / 100, 104 / 99, 900
+// off 16 bytes 126 / 119, 123 / 118; T = 20011, C = 1535 107 / 100, 105 / 99; T =
+// 16000, C = 2049 111 / 106, 109 / 106; T = 65536, C = 513 115 / 108, 117 / 108;
+// C = 521, 601 (half the lanes idle) equal.  K4 backward is within 1.5%
+// either way (C = 513 184 / 178).  680 lanes lost at C = 700 (137, 134).  K3
+// forward takes none (C = 1001 52 against 55).
 constexpr int kCapLanesUnaligned = 1150;
 constexpr unsigned kCapMinBlocks = 16u * 256u;
 
@@ -269,14 +273,14 @@ inline unsigned own_lds(const void* kernel) {
   return hipFuncGetAttributes(&a, kernel) == hipSuccess ? static_cast<unsigned>(a.sharedSizeBytes) : kLdsPerCu;
 }
 
-// The LDS reserve that leaves about kCapLanes (kCapLanesUnaligned) lanes with
-// work resident on a CU, for `blocks` workgroups of a kernel with `own` bytes
-// of LDS and `block` threads, lpt lanes per token and `groups` groups per row.
-// 1280 bytes stay free per workgroup, the granularity of an allocation.
-inline unsigned cap_lds(unsigned own, unsigned blocks, int block, int lpt, int groups, bool aligned) {
+// The LDS reserve that leaves about `lanes` lanes with work resident on a CU, for
+// `blocks` workgroups of a kernel with `own` bytes of LDS and `block` threads,
+// lpt lanes per token and `groups` groups per row.  1280 bytes stay free per
+// workgroup, the granularity of an allocation.
+inline unsigned cap_lds(unsigned own, unsigned blocks, int block, int lpt, int groups, int lanes) {
   if (blocks < kCapMinBlocks || lpt < kWave) return 0u;
   const int busy = block * groups / lpt;  // lanes with work in a workgroup
-  const int n = busy > 0 ? ((aligned ? kCapLanes : kCapLanesUnaligned) + busy / 2) / busy : 0;
+  const int n = busy > 0 ? (lanes + busy / 2) / busy : 0;
   if (n < 1 || n >= 8) return 0u;
   const unsigned each = kLdsPerCu / static_cast<unsigned>(n);
   return each > own + 1280u ? each - own - 1280u : 0u;
@@ -441,6 +445,7 @@ struct RowWalk {
   static constexpr int LPT = kLpt;
   static constexpr bool LOOP = kLoop;
   static constexpr bool WHOLE = kWhole;
+  static constexpr int CAP = WHOLE ? kCapLanes : kCapLanesUnaligned;  // lanes of cap_lds
 };
 
 // f(RowWalk) for rows of C columns whose 16-byte groups are aligned or not.

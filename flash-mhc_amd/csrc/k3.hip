@@ -202,6 +202,17 @@ __global__ __launch_bounds__(block_of<WALK::LPT>()) void k3_bwd_kernel(const uin
   }
 }
 
+// K3 forward's residency from 16 to 40 workgroups per CU, where fewer resident
+// ones leave a longer last round: T = 16384, C = 512 14.5 us, with kCapLanes
+// 15.8, with no cap 14.8; T = 24000 20.7 / 22.2 / 21.4; T = 16384, C = 448 13.0 /
+// 14.5 / 13.0; T = 12000, C = 1024 20.9 / 21.9 / 21.3; T = 4096, C = 2048 14.6 /
+// 15.7 / 14.9, C = 2560 17.9 / 19.5 / 18.0.  From 40 per CU on kCapLanes is equal
+// or better (T = 65536, C = 512 54.5 against 55.3).  K3 backward and K4 keep
+// kCapLanes there (T = 10000, C = 3000 K4 forward 89.8 against 92.6, C = 1400 K3
+// backward 42.7 / 44.7, T = 12000, C = 1000 K4 backward 58.9 / 60.7).
+constexpr unsigned kK3FewBlocks = 40u * 256u;
+constexpr int kK3FewLanes = 1280;
+
 int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t T, int C,
                   hipStream_t s) {
   // 128 whole groups and many tokens: one wave walks two groups per lane, six
@@ -227,7 +238,7 @@ int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t 
       if (Walk::LOOP)
         lds = kLdsCapSix;
       else if (Walk::WHOLE && 4 * (C / 8) >= 3 * L)
-        lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+        lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, grid.x < kK3FewBlocks ? kK3FewLanes : kCapLanes);
       k3_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(x + t * 4 * C, h_pre + t * 4,
                                                                               out + t * C, n, C);
     });
@@ -249,7 +260,7 @@ int launch_k3_bwd(const uint16_t* x, const float* h_pre, const uint16_t* go, uin
       for_launches(T, block_of<L>(), tokens_per_block(L), [&](int64_t t, int64_t n) {
         const dim3 grid(blocks_for(n, tokens_per_block(L)));
         unsigned lds = 0;
-        if (GX && FMHC_LDS_CAP && !Walk::LOOP) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+        if (GX && FMHC_LDS_CAP && !Walk::LOOP) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::CAP);
         k3_bwd_kernel<Walk, GX, CANON><<<grid, block_of<L>(), lds, s>>>(
             x + t * 4 * C, h_pre + t * 4, go + t * C, GX ? grad_x + t * 4 * C : nullptr, grad_h_pre + t * 4, n, C);
       });

@@ -270,7 +270,7 @@ int launch_k4_fwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
       if (decltype(w)::LOOP)
         lds = grid.x >= kCapMinBlocks ? kLdsCapFive : 0u;
       else
-        lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+        lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::CAP);
       k4_fwd_kernel<Walk><<<grid, block_of<L>(), FMHC_LDS_CAP ? lds : 0u, s>>>(
           x + t * 4 * C, lo + t * C, H + t * 16, hp + t * 4, out + t * 4 * C, n, C);
     });
@@ -296,7 +296,7 @@ int launch_k4_bwd(const uint16_t* x, const uint16_t* lo, const float* H, const f
       for_launches(T, block_of<L>(), tokens_per_block(L), [&](int64_t t, int64_t n) {
         const dim3 grid(blocks_for(n, tokens_per_block(L)));
         unsigned lds = 0;
-        if (FMHC_LDS_CAP && C / 8 <= L && L <= 256) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::WHOLE);
+        if (FMHC_LDS_CAP && C / 8 <= L && L <= 256) lds = cap_lds(own, grid.x, block_of<L>(), L, C / 8, Walk::CAP);
         k4_bwd_kernel<W, E><<<grid, block_of<L>(), lds, s>>>(
             x + t * 4 * C, lo + t * C, H + t * 16, hp + t * 4, go + t * 4 * C, gx + t * 4 * C, glo + t * C,
             gH + t * 16, ghp + t * 4, n, C);
