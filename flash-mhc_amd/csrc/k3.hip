@@ -215,18 +215,6 @@ constexpr int kK3FewLanes = 1280;
 
 int launch_k3_fwd(const uint16_t* x, const float* h_pre, uint16_t* out, int64_t T, int C,
                   hipStream_t s) {
-  // 128 whole groups and many tokens: one wave walks two groups per lane, six
-  // workgroups per CU (T = 65536 104.5 us, against 106.3 with 128 lanes; with
-  // few tokens 128 lanes: T = 4096 9.8 -> 8.8 us).
-  if (C == 2 * 8 * kWave && T >= 16384 && aligned16(x) && aligned16(out)) {
-    using Walk = RowWalk<kWave, true, true>;
-    static const unsigned lds = lds_reserve(reinterpret_cast<const void*>(&k3_fwd_kernel<Walk>), kLdsCapSix);
-    for_launches(T, block_of<kWave>(), tokens_per_block(kWave), [&](int64_t t, int64_t n) {
-      k3_fwd_kernel<Walk><<<dim3(blocks_for(n, tokens_per_block(kWave))), block_of<kWave>(), FMHC_LDS_CAP ? lds : 0u,
-                            s>>>(x + t * 4 * C, h_pre + t * 4, out + t * C, n, C);
-    });
-    return launch_status();
-  }
   with_row_walk(C, aligned16(x) && aligned16(out), [&](auto w) {
     using Walk = decltype(w);
     constexpr int L = Walk::LPT;
