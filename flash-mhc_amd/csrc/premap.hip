@@ -71,6 +71,14 @@ int64_t round_up(int64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 bool param_dtype_ok(int d) { return d == FMHC_PARAM_F32 || d == FMHC_PARAM_BF16; }
 
 constexpr int kFinishThreads = 256;  // 8 tokens of 32 lanes
+// k1_finish_k2_k3's AHEAD for rows off 8 columns or 16 bytes: up to a full round
+// of four workgroups per CU, and two groups per lane.  Pre-map forward ahead /
+// not / the element-wise K3 these rows had, us: T = 1168, C = 250 10.0 / 8.0 /
+// 8.3, T = 1168, C = 1100 15.1 / 12.6 / 14.2, T = 2700, C = 3002 37.0 / 33.3 /
+// 43.1; T = 64, C = 1100 7.3 / 7.1 / 7.8, T = 700, C = 2050 12.1 / 11.8; T = 64,
+// C = 2100 7.9 / 8.4 / 8.5, T = 400, C = 2500 11.7 / 13.2, T = 1000, C = 2100
+// 14.0 / 15.3.
+constexpr int64_t kAheadT = 4 * 256;
 
 // Adds the S partials of a projection and of the sum of squares in split
 // order; at(i) gives the i-th four of each.
@@ -157,7 +165,9 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2(
 // forward took, us: T = 1, C = 4096 8.9, now 8.6; T = 64 9.8 / 9.5; T = 1003,
 // C = 2560 16.2 / 15.3; T = 1024, C = 1024 11.7 / 11.0; T = 1536, C = 2048
 // 20.5 / 18.7.
-template <bool WHOLE>
+// AHEAD: the x vectors are loaded ahead.  Their registers leave four workgroups
+// on a CU (109 VGPRs; eight without them).
+template <bool WHOLE, bool AHEAD>
 __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
     const float* __restrict__ part, int S, int nC, const K2Params P, uint16_t* __restrict__ proj,
     float* __restrict__ inv_rms, float* __restrict__ h_pre, float* __restrict__ h_post, float* __restrict__ H,
@@ -184,7 +194,7 @@ __global__ __launch_bounds__(kFinishThreads) void k1_finish_k2_k3(
   regs.load(P);
   const uint16_t* x0 = x + t * 4 * C;
   const int ng = C / 8;
-  const bool pre = ng <= kPre * kFinishThreads;
+  const bool pre = AHEAD && ng <= kPre * kFinishThreads;
   u32x4 xv[kPre][4];
   if (pre) {
 #pragma unroll
@@ -404,12 +414,16 @@ int premap_fwd_run(const uint16_t* x, const uint16_t* W, const void* alpha_pre, 
   if (S >= 2 && layer_input) {
     const dim3 grid(static_cast<unsigned>(T));
     const int c = static_cast<int>(C);
+    auto launch = [&](auto whole, auto ahead) {
+      k1_finish_k2_k3<decltype(whole)::value, decltype(ahead)::value><<<grid, kFinishThreads, 0, s>>>(
+          part, S, nc, P, proj, inv_rms, h_pre, h_post, H_merged, z, x, layer_input, c);
+    };
     if (C % 8 == 0 && aligned16(x) && aligned16(layer_input))
-      k1_finish_k2_k3<true><<<grid, kFinishThreads, 0, s>>>(part, S, nc, P, proj, inv_rms, h_pre, h_post, H_merged,
-                                                            z, x, layer_input, c);
+      launch(std::true_type{}, std::true_type{});
+    else if (T <= kAheadT && C / 8 > kFinishThreads)
+      launch(std::false_type{}, std::true_type{});
     else
-      k1_finish_k2_k3<false><<<grid, kFinishThreads, 0, s>>>(part, S, nc, P, proj, inv_rms, h_pre, h_post, H_merged,
-                                                             z, x, layer_input, c);
+      launch(std::false_type{}, std::false_type{});
     return fmhc::launch_status();
   }
   if (S >= 2) {

@@ -56,7 +56,9 @@ def _params(C):
 FWD = [*SHAPES, (5, 2), (40, 3), (4096, 16), (2721, 129), (5000, 131), (9000, 33), (12300, 25), (20011, 300),
        (2720, 4099), (3, 4103),
        # The split's blocks of 16 (up to 912 tokens) and of 32, and its last token counts.
-       (912, 1100), (913, 1101), (929, 1100), (1168, 1024), (1169, 1024), (1600, 1423), (1601, 1420), (2719, 1424)]
+       (912, 1100), (913, 1101), (929, 1100), (1168, 1024), (1169, 1024), (1600, 1423), (1601, 1420), (2719, 1424),
+       # The split's finish: x ahead of the sums from 257 groups of 8 columns on, up to 1024 tokens.
+       (30, 2054), (30, 2060), (1024, 2060), (1025, 2060)]
 
 
 @pytest.mark.parametrize("off", [0, 1, 3])
