@@ -14,7 +14,7 @@ from flash_mhc import build_permutation_matrices
 from flash_mhc import _abi
 from flash_mhc import kernels as K
 from oracle import mhc_oracle as O
-from parity import check_bf16, check_fp32, check_rel
+from parity import bf16_ulp, check_bf16, check_fp32, check_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -55,8 +55,8 @@ def _params(C):
 # 15 ... 17 around one 64-column chunk.
 FWD = [*SHAPES, (5, 2), (40, 3), (4096, 16), (2721, 129), (5000, 131), (9000, 33), (12300, 25), (20011, 300),
        (2720, 4099), (3, 4103),
-       # The split's blocks of 16 (up to 912 tokens) and of 32, and its last token counts.
-       (912, 1100), (913, 1101), (929, 1100), (1168, 1024), (1169, 1024), (1600, 1423), (1601, 1420), (2719, 1424),
+       # The split's blocks of 16 (up to 896 tokens) and of 32, and its last token counts.
+       (896, 1100), (897, 1101), (912, 1100), (913, 1101), (929, 1100), (1168, 1024), (1169, 1024), (1600, 1423), (1601, 1420), (2719, 1424),
        # The split's finish: x ahead of the sums from 257 groups of 8 columns on, up to 1024 tokens.
        (30, 2054), (30, 2060), (1024, 2060), (1025, 2060)]
 
@@ -67,11 +67,9 @@ def test_k1_fwd(T, C, off):
     nC = 4 * C
     rn, x, W = _inputs(T, C, off, 7 * T + C + off)
     proj, inv = K.k1_fwd(x.view(T, nC), W, out=_at(torch.zeros(T, 32, dtype=BF16), off))
-    i = torch.cat([torch.arange(min(T, 80)), torch.arange(max(0, T - 80), T)]).unique()
-    xs = x.view(T, nC)[i.to(DEV)].cpu()
-    R, S, invR = O.k1_fwd(xs, W.cpu())
-    check_bf16("proj", proj[i.to(DEV)], R, S, nC)
-    check_rel("inv_rms", inv[i.to(DEV)], invR, rtol=4 * nC ** 0.5 * 2.0**-24 + 4 * 2.0**-24)
+    R, S, invR = O.k1_fwd(x.view(T, nC).cpu(), W.cpu())
+    check_bf16("proj", proj, R, S, nC)
+    check_rel("inv_rms", inv, invR, rtol=4 * nC ** 0.5 * 2.0**-24 + 4 * 2.0**-24)
 
 
 @pytest.mark.parametrize("off", [0, 1])
@@ -127,10 +125,12 @@ def test_premap_bwd(T, C, off):
 
 # K3 / K4: one 16-byte group per lane over 8, 16, 32, 64, 128, 192, ... 448
 # lanes per token and several groups per lane beyond; rows that end inside a
-# group, at a wave's edge, or one group into the next wave; enough tokens for
-# the residency caps in two of them.
+# group, at a wave's edge, or one group into the next wave.  From (16500, 519)
+# on enough workgroups (4096) for the residency caps, at one wave per token, two
+# and more; (20001, 200) has them too, at 32 lanes per token, which take no cap.
 K34 = [(1, 1), (33, 7), (9, 8), (130, 65), (65, 136), (31, 264), (77, 512), (45, 519), (5, 520), (19, 1032),
-       (7, 1535), (3, 1536), (6, 2056), (4, 3079), (2, 3592), (3, 4100), (20001, 200), (9001, 1000)]
+       (7, 1535), (3, 1536), (6, 2056), (4, 3079), (2, 3592), (3, 4100), (20001, 200), (16500, 519), (9001, 1000), (4200, 1535), (4100, 2049),
+       (4100, 2560), (4100, 3003), (4100, 3583)]
 
 
 @pytest.mark.parametrize("off", [0, 1])
@@ -194,7 +194,26 @@ def test_without_partials(T, C, monkeypatch):
     for name in ("fmhc_k1_fwd_workspace_bytes", "fmhc_premap_fwd_workspace_bytes", "fmhc_k1_bwd_workspace_bytes"):
         monkeypatch.setattr(lib, name, lambda *a: 0)
     monkeypatch.setattr(lib, "fmhc_premap_bwd_workspace_bytes", lambda *a: small)
-    for a, b in zip(run(), want):
+    got = run()
+    proj, inv, li, H, hq, hp, gx1, gW1, gx, gW, *_ = [t.cpu() for t in got]
+    c = lambda t: t.cpu()
+    xc = x.view(T, nC).cpu()
+    check_bf16("proj", proj, *O.k1_fwd(xc, c(W))[:2], nC)
+    check_bf16("layer_input", li, *O.k3_fwd(c(x), hp), 4)
+    dx, dxS = O.k1_bwd_dx(c(go), xc, c(W), proj, inv)
+    check_bf16("k1 grad_x", gx1, dx, dxS, 64)
+    check_bf16("k1 grad_W", gW1, *O.k1_grad_W(c(go), xc, inv), T)
+    # The pre-map's gradients from K2's gradient of proj, which the separate kernels give.
+    gh = K.k3_bwd(g_li, x, hp.to(DEV))[1]
+    gp = c(K.k2_bwd(proj.to(DEV), *p, gh, hq.to(DEV), H.to(DEV))[0])
+    check_bf16("grad_W", gW, *O.k1_grad_W(gp, xc, inv), T)
+    dx, dxS = (t.view(T, 4, C) for t in O.k1_bwd_dx(gp, xc, c(W), proj, inv))
+    gx3 = hp.double().unsqueeze(-1) * c(g_li).double().unsqueeze(1)
+    # Three values and two sums of them, each rounded once: half an ulp of at most M each, 2.5 in all.
+    M = c(g_in).double().abs() + gx3.abs() + dx.abs()
+    err = (gx.double() - (c(g_in).double() + gx3 + dx)).abs()
+    assert bool((err <= 2.5 * bf16_ulp(M) + 4 * 64 ** 0.5 * 2.0**-24 * dxS).all())
+    for a, b in zip(got, want):
         a, b = a.double(), b.double()
         # One more bf16 rounding here or there (K1's projection feeds the rest): 2^-8 of each value, 2^-6 of the whole.
         assert float((a - b).norm()) <= 2.0 ** -6 * float(b.norm())
@@ -236,3 +255,35 @@ def test_k1_bwd_dx_in_place(T, nC):
     got = K.k1_bwd_dx(go, x, W, proj, inv, grad_x=x)
     assert got.data_ptr() == x.data_ptr()
     check_bf16("grad_x", got, R, S, 64)
+
+
+# One infinity or NaN in x, in columns that the last, shifted group of a row
+# loads together with the group before it (nC - 8 ...), at either side of a
+# 128-column slice, and first: it reaches what the formulas say (its token's
+# projection and grad_x, its column of grad_W) and nothing else.
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("T,nC", [(40, 9), (40, 12), (33, 129), (300, 132), (2100, 1031), (20, 4404), (700, 1200)])
+def test_k1_one_odd_value(T, nC, value):
+    g = torch.Generator().manual_seed(T + nC)
+    x = torch.randn(T, nC, generator=g).to(BF16).to(DEV)
+    W = (torch.randn(32, nC, generator=g) * 0.02 + 0.5).to(BF16).to(DEV)
+    go = torch.randn(T, 32, generator=g).to(BF16).to(DEV)
+    proj, inv = K.k1_fwd(x, W)
+    gx, gW = K.k1_bwd(go, x, W, proj, inv)
+    for c in sorted({0, 127, 128, nC - 9, nC - 8, nC - 7, nC - 2, nC - 1} & set(range(nC))):
+        t = (7 * c + 3) % T
+        y = x.clone()
+        y[t, c] = value
+        proj1, inv1 = K.k1_fwd(y, W)
+        # The sum of squares is inf or NaN: 1 / rms is 0 or NaN, and the projection NaN either way.
+        assert bool(proj1[t].isnan().all()) and not float(inv1[t]) > 0
+        keep = torch.arange(T, device=DEV) != t
+        assert torch.equal(proj1[keep], proj[keep]) and torch.equal(inv1[keep], inv[keep])
+        # The backward with the finite token's proj and inv_rms: only x itself is odd.
+        gx1, gW1 = K.k1_bwd(go, y, W, proj, inv)
+        odd = torch.zeros(T, nC, dtype=torch.bool, device=DEV)
+        odd[t, c] = True
+        assert torch.equal(~gx1.isfinite(), odd) and torch.equal(gx1[~odd], gx[~odd])
+        assert torch.equal(~gW1.isfinite(), odd[t].expand(32, nC))
+        assert torch.equal(gW1[:, ~odd[t]], gW[:, ~odd[t]])
+        assert torch.equal(K.k1_bwd_dx(go, y, W, proj, inv)[~odd], gx[~odd])

@@ -2,7 +2,8 @@
 K4 and the pre-map backward at two token counts, one block of 16 tokens and a
 ragged one apart, at sizes where a launch reads about as much as stays in the
 memory-side cache (80 MiB of the 256).  For the tokens the two share, the larger
-launch must give the bits of the smaller one.
+launch must give the bits of the smaller one.  K1's grad_W, a sum over the
+tokens, is checked against the oracle at both.
 """
 
 from __future__ import annotations
@@ -12,6 +13,8 @@ import torch
 
 from flash_mhc import build_permutation_matrices
 from flash_mhc import kernels as K
+from oracle import mhc_oracle as O
+from parity import check_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -20,7 +23,8 @@ BF16 = torch.bfloat16
 LINE = 80 << 20
 
 
-@pytest.mark.parametrize("C", [256, 512, 1000])
+# 1000 and 1008: rows off and on 128-byte lines (4 C a multiple of 64), neither a power of two.
+@pytest.mark.parametrize("C", [256, 512, 1000, 1008])
 @pytest.mark.parametrize("kernel", ["k1_fwd", "k1_bwd_dx", "k1_bwd", "k3_fwd", "k3_bwd", "k4_fwd", "k4_bwd"])
 def test_same_bits_on_both_sides(kernel, C):
     read = {"k1_fwd": 8, "k1_bwd_dx": 8, "k1_bwd": 8, "k3_fwd": 8, "k3_bwd": 10, "k4_fwd": 10, "k4_bwd": 36}[kernel] * C
@@ -43,7 +47,10 @@ def test_same_bits_on_both_sides(kernel, C):
         if kernel == "k1_bwd_dx":
             return (K.k1_bwd_dx(gp[:T], xf, W, proj[:T], inv[:T]),)
         if kernel == "k1_bwd":
-            return (K.k1_bwd(gp[:T], xf, W, proj[:T], inv[:T])[0],)
+            gx, gW = K.k1_bwd(gp[:T], xf, W, proj[:T], inv[:T])  # grad_W is a sum over the tokens
+            R, S = O.k1_grad_W(gp[:T].cpu(), xf.cpu(), inv[:T].cpu())
+            check_bf16("grad_W", gW, R, S, T)
+            return (gx,)
         if kernel == "k3_fwd":
             return (K.k3_fwd(x[:T], h[:T]),)
         if kernel == "k3_bwd":

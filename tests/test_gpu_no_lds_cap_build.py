@@ -1,10 +1,10 @@
-"""The product launches K1's backward dx (up to C = 2560), K3 forward, K3
-backward (with grad_x, up to C = 2048) and K4 forward (from 16 workgroups per
-CU on) with LDS reserved that the kernels do not use, which caps how many
-workgroups share a CU.  The evidence build "no_lds_cap" launches them
-without it.  Loaded beside the product library through the same C ABI, its
-K1, K3 and K4 entry points must give the product's outputs bit for bit: the
-cap changes residency, not arithmetic."""
+"""The product launches K1's backward dx (up to C = 2560), K3 forward and K4
+forward, and K3 backward (with grad_x) and K4 backward with one 16-byte group
+per lane, from 16 workgroups per CU and 64 lanes per token on, with LDS reserved
+that the kernels do not use, which caps how many workgroups share a CU.  The
+evidence build "no_lds_cap" launches them without it.  Loaded beside the product
+library through the same C ABI, its K1, K3 and K4 entry points must give the
+product's outputs bit for bit: the cap changes residency, not arithmetic."""
 
 from __future__ import annotations
 
@@ -66,11 +66,15 @@ def _k134(lib, x, W, go1, lo, hp, hq, H, go3, go4):
     return out
 
 
-# The metric width and its neighbours at many tokens (the caps apply), a
-# ragged token count, few tokens (K4 forward below the cap's threshold),
-# C = 4096 (K1 and K3 backward uncapped) and the one-element path (C = 100).
+# The metric width and its neighbours at many tokens, a ragged token count, few
+# tokens (no caps but K1's), C = 4096 (K1 and K3 backward uncapped), narrow rows
+# (no caps); then every layout that a cap can apply to, just past 16 workgroups
+# per CU: 64, 128, 192, 256, 320, 384 and 448 lanes per token, with whole groups
+# and with rows off 8 columns, and K3 forward past 40 per CU (another cap).
 @pytest.mark.parametrize("T,C", [(65536, 1024), (20001, 512), (16384, 2048), (4096, 1024), (16384, 4096),
-                                 (3000, 2560), (777, 100)])
+                                 (3000, 2560), (777, 100), (16500, 448), (8300, 1000), (4200, 1536), (4200, 2040),
+                                 (4200, 2560), (4200, 3000), (4200, 3584), (10300, 1400), (16500, 519), (8300, 777),
+                                 (4200, 1535), (4200, 2047), (4200, 2049), (4200, 3001), (4200, 3583), (4200, 5001)])
 def test_capped_launches_equal_uncapped(nocap_lib, T, C):
     g = torch.Generator(device=DEV).manual_seed(T + C)
     x = torch.randn(T, 4, C, device=DEV, generator=g).to(BF16)
