@@ -262,7 +262,7 @@ constexpr int kCapLanes = 680;
 // 16000, C = 2049 111 / 106, 109 / 106; T = 65536, C = 513 115 / 108, 117 / 108;
 // C = 521, 601 (half the lanes idle) equal.  K4 backward is within 1.5%
 // either way (C = 513 184 / 178).  680 lanes lost at C = 700 (137, 134).  K3
-// forward takes none (C = 1001 52 against 55).
+// forward takes none (C = 1001 alone 52 against 55).
 constexpr int kCapLanesUnaligned = 1150;
 constexpr unsigned kCapMinBlocks = 16u * 256u;
 

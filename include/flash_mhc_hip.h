@@ -69,7 +69,8 @@ int64_t fmhc_k1_fwd_workspace_bytes(int64_t T, int64_t nC);
 /* K1 backward, grad of x_flat:
  *   scale[t]    = (sum_d go[t,d] * proj_out[t,d]) * inv_rms[t]^2 / nC
  *   grad_x[t,k] = bf16(inv_rms[t] * sum_d go[t,d] * W[d,k] - scale[t] * x[t,k])
- * grad_out, proj_out (T, D_out) bf16; inv_rms (T,) fp32; grad_x (T, nC) bf16.
+ * grad_out, proj_out (T, D_out) bf16; inv_rms (T,) fp32; grad_x (T, nC) bf16,
+ * which may be x_flat.
  * Replaces: src/flash_mhc/ops.py:267-344 (_fused_rmsnorm_project_bwd_dx_cuda) launching
  *           src/flash_mhc/kernels.py:306-376 (_fused_rmsnorm_project_bwd_dx_kernel). */
 int fmhc_k1_bwd_dx(const uint16_t* x_flat, const uint16_t* W, const uint16_t* grad_out,
