@@ -312,7 +312,7 @@ __global__ __launch_bounds__(kK2BwdTok * LPT) void k3_reduce_k2_bwd(
   };
   // Every slot computes (idle ones on the last token), so the slot's lanes are
   // all active for the sums below.
-  constexpr int kRounds = LPT == 64 ? 4 : 1;  // fewer than 256 groups for 64 lanes, up to 32 for 32
+  constexpr int kRounds = LPT == 64 ? 4 : 2;  // fewer than 256 groups for 64 lanes, up to 64 for 32
   const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
   float e[kRounds][4];
 #pragma unroll
@@ -322,15 +322,21 @@ __global__ __launch_bounds__(kK2BwdTok * LPT) void k3_reduce_k2_bwd(
     if (sub + k * LPT < ng) round(Vec<8>{}, sub + k * LPT, e[k]);
     if (k == 0) row_tail<false>(C, sub, [&](int c) { round(Vec<1>{}, c, e[0]); });
   }
+  if constexpr (!CANON && LPT == 32) {
+    // k3_bwd_kernel's one wave: lanes 32 apart are the first pairs of its sum.
 #pragma unroll
-  for (int k = 0; k < kRounds; ++k) {
-    if (k * LPT >= ng) break;  // uniform
-    if constexpr (CANON) {
-      slice_sums_add<LPT>(e[k], s, k, ng / 16, lane);
-    } else {
-      // k3_bwd_kernel's waves hold 64 groups each and add their sums in order.
+    for (int j = 0; j < 4; ++j) s[j] = group_sum<LPT>(e[0][j] + e[1][j]);
+  } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] += group_sum<LPT>(e[k][j]);
+    for (int k = 0; k < kRounds; ++k) {
+      if (k * LPT >= ng) break;  // uniform
+      if constexpr (CANON) {
+        slice_sums_add<LPT>(e[k], s, k, ng / 16, lane);
+      } else {
+        // k3_bwd_kernel's waves hold 64 groups each and add their sums in order.
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] += group_sum<LPT>(e[k][j]);
+      }
     }
   }
   const float s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3];
@@ -559,9 +565,11 @@ extern "C" int fmhc_premap_bwd(const uint16_t* x, const uint16_t* W, const void*
   if (!k2_params(alpha_pre, alpha_post, alpha_res, bias, perm, param_dtype, P)) return FMHC_ERR_INVALID_ARGUMENT;
   // K2's backward, whose parameter partials K1's grad_W reduce also sums.
   K2ParamSums sums;
-  // Half a wave per token for rows of 17 to 32 groups of 8, a wave up to 255.
+  // Half a wave per token for rows of 17 to 64 groups of 8, a wave up to 255: a
+  // wave at 33 to 64 took, us, T = 16, C = 448 13.3 against 12.5, T = 300 21.5 /
+  // 20.6, T = 6000, C = 300 36.5 / 32.5, C = 512 40.4 / 36.4.
   const int64_t groups = C / 8;
-  const int lanes = groups > 32 ? 64 : 32;
+  const int lanes = groups > 64 ? 64 : 32;
   if (fused && T <= kK2BwdSmallT && groups > 16 && groups < 256) {
     // Few tokens: K3's reduce-only pass and K2's backward as one kernel.
     float* partial = reinterpret_cast<float*>(ws + w.k2);

@@ -103,8 +103,13 @@ def test_k1_bwd(T, C, off):
     check_bf16("grad_W", gW, R, S, T)
 
 
+# K3's reduce and K2's backward in one kernel: half a wave per token, one and two
+# groups of 8 per lane (17 to 64), the second partly filled, then a wave.
+FUSED_BWD = [(9, 136), (41, 256), (40, 263), (300, 264), (700, 384), (33, 448), (16, 512), (20, 519), (9, 520), (9, 768)]
+
+
 @pytest.mark.parametrize("off", [0, 1])
-@pytest.mark.parametrize("T,C", SHAPES)
+@pytest.mark.parametrize("T,C", [*SHAPES, *FUSED_BWD])
 def test_premap_bwd(T, C, off):
     nC = 4 * C
     rn, x, W = _inputs(T, C, off, 13 * T + C + off)
