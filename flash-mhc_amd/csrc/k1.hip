@@ -978,9 +978,13 @@ __global__ __launch_bounds__(256) void k1_bwd_mfma(const uint16_t* __restrict__ 
 // 62.5 us, 100 91 -> 78, 256 131 -> 127.5; T = 8192, C = 512 51 -> 48.7; with
 // more slices 1% slower (C = 1024, 2560).  Sixteen up to kReduceSplit16Slices:
 // T = 65536, C = 24 59.7 -> 43.8, 64 59.3 -> 54.5; K1 backward C = 24 35.0 ->
-// 22.2, 100 32.1 -> 30.9, T = 8192, C = 256 17.7 -> 17.0; equal above.
+// 22.2, 100 32.1 -> 30.9, T = 8192, C = 256 17.7 -> 17.0; equal above.  Up to
+// kReduceSplit16Runs runs, the four that a thread loads at once, sixteen groups
+// only add a barrier (K1 backward, C = 256, one group / sixteen: T = 16 6.1 / 6.6,
+// T = 300 (four runs) 10.5 / 10.9, T = 480 (seven) 11.4 / 10.9, T = 700 11.1 / 10.3).
 constexpr int kReduceSplit16Slices = 8;
 constexpr int kReduceSplit4Slices = 16;
+constexpr int64_t kReduceSplit16Runs = 4;
 template <int GROUPS>
 __global__ __launch_bounds__(256) void k1_dw_reduce(const float* __restrict__ partial,
                                                     uint16_t* __restrict__ dW, int64_t nparts,
@@ -1493,9 +1497,9 @@ int launch_dw_reduce(const float* partial, uint16_t* grad_W, int64_t nruns, cons
     const unsigned nb = blocks_for(vecs, 256 / G);
     k1_dw_reduce<G><<<dim3(nb + k2_params), 256, 0, s>>>(partial, grad_W, nruns, sl, nC, nb, sums);
   };
-  if (sl.n <= kReduceSplit16Slices)
+  if (sl.n <= kReduceSplit16Slices && nruns > kReduceSplit16Runs)
     launch(std::integral_constant<int, 16>{});
-  else if (sl.n <= kReduceSplit4Slices)
+  else if (sl.n > kReduceSplit16Slices && sl.n <= kReduceSplit4Slices)
     launch(std::integral_constant<int, 4>{});
   else
     launch(std::integral_constant<int, 1>{});

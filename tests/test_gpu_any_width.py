@@ -161,10 +161,11 @@ def test_k3_k4(T, C, off):
     check_fp32("k4 grad_hp", ghp, *ref["grad_hp"], C)
 
 
-# grad_W's reduce: 16 shares of the runs up to 8 slices of 128 columns (C = 256),
-# four up to 16, one above; one run to several hundred, fewer runs than shares.
+# grad_W's reduce: 16 shares of five runs and more up to 8 slices of 128 columns
+# (C = 256), four up to 16, one above and for fewer runs; one run to several
+# hundred, fewer runs than shares (T = 304: four runs, 305: five).
 @pytest.mark.parametrize("T,C", [(1, 64), (40, 24), (9000, 24), (16001, 33), (3000, 256), (3000, 264), (2000, 512),
-                                 (2000, 520)])
+                                 (2000, 520), (304, 64), (305, 64), (304, 256), (305, 256), (130, 300)])
 def test_grad_W_reduce(T, C):
     nC = 4 * C
     rn, x, W = _inputs(T, C, 0, 17 * T + C)
