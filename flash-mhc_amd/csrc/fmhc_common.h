@@ -99,8 +99,9 @@ __device__ __forceinline__ void st8_stream(void* p, u32x2 v) {
 // forward 25.6 / 26.6, K1 forward then backward 54.5 / 58.8; forward of T = 8192
 // 77 / 80; per block of six in a captured training step T = 8192 261 / 268, T =
 // 4096 155 / 158, T = 16384, C = 512 285 / 302, T = 1003, C = 2560 163 / 166, in
-// an eval forward T = 8192 72.8 / 71.9, the others within 1%.  Kernels that read again what the launch before them
-// or their own first pass has read take ordinary loads (premap.hip, k1.hip).
+// an eval forward T = 8192 72.8 / 71.9, the others within 1%.  Kernels that read
+// again what the launch before them or their own first pass has read take
+// ordinary loads (premap.hip, k1.hip).
 
 // bf16 bit pattern -> fp32 (exact).
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
